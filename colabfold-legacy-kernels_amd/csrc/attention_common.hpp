@@ -232,6 +232,25 @@ __device__ __forceinline__ void stage_rows_ld(Rsrc r, int r0, int ld, char* lds,
     }
 }
 
+// stage_rows_ld from a first row r0 that may be negative: rows below 0 read zeros.
+template <int D, int ROWS, int NTHREADS>
+__device__ __forceinline__ void stage_rows_from(Rsrc r, int r0, int ld, char* lds, int tid) {
+    using T = SwzTile<D>;
+    constexpr int SLOTS = ROWS * T::PL;
+    static_assert(SLOTS % 64 == 0, "tile must be whole wave instructions");
+    const int lane = tid & 63, wave = tid >> 6;
+#pragma unroll
+    for (int i = 0; i < (SLOTS + NTHREADS - 1) / NTHREADS; ++i) {
+        const int b = wave * 64 + i * NTHREADS;
+        if (SLOTS % NTHREADS != 0 && b >= SLOTS) break;
+        const int slot = b + lane;
+        const int row = slot / T::PL;
+        const int piece = (slot % T::PL) ^ T::swz(row);
+        const int voff = piece < T::P && r0 + row >= 0 ? ((r0 + row) * ld + piece * 8) * 2
+                                                       : kPastEnd;
+        buf_dma16(r, voff, 0, lds + b * 16);
+    }
+}
 
 // The rows of one (n, h) of an attention operand: [N, H, S, D] (rows D apart), or with NSHD
 // AlphaFold's [N, S, H, D] (rows H*D apart, head h at column block h).

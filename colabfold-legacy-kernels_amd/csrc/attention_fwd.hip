@@ -4,9 +4,15 @@
 //
 // Work split: a block of 4 waves owns (query tile of 64*QT rows, head h, row n); each wave owns
 // 16*QT queries and streams the keys in tiles of 64 through double-buffered LDS: tile kt+1 is
-// fetched with direct global->LDS loads (and its bias rows into registers) while tile kt is
-// computed, so each tile costs one barrier. Which tiles contain an absent key is worked out once
-// per block from the mask row; the others skip the mask entirely.
+// fetched with direct global->LDS loads (K, V and the bias rows) while tile kt is computed, so
+// each tile costs one barrier. Which tiles contain an absent key is worked out once per block
+// from the mask row; the others skip the mask entirely.
+//
+// Any even Sk, and any odd one (by query parity, the ODD form below), loads its bias through LDS.
+// Reading bias and mask element by element, as a ragged Sk once did, left the kernel waiting on
+// sixteen 2-byte loads per lane and tile: triangle attention of 757 residues (4 heads x 32)
+// 2395 -> 550 us, 1024 sequences of 300 residues (8 heads x 8) 965 -> 292 us, 203 residues
+// 65 -> 29 us. That path remains for what the direct loads cannot take (launch_fwd_qt).
 //
 // Per 64-key tile and 16-query sub-tile a wave computes S^T = K . Q^T with the keys of each
 // 32-key chunk permuted so that lane l's accumulator holds keys 8*(l/16)+0..7 of the chunk for
@@ -62,7 +68,6 @@ struct RowFlags {
     uint64_t bits;
     float masked_logit;
 };
-template <bool VEC>
 __device__ __forceinline__ RowFlags row_flags(const uint8_t* mrow, int Sk) {
     const int lane = threadIdx.x & 63;
     const int ntiles = (Sk + 63) / 64;
@@ -73,22 +78,13 @@ __device__ __forceinline__ RowFlags row_flags(const uint8_t* mrow, int Sk) {
         for (int base = 0; base < Sk; base += 512) {
             const int k = base + 8 * lane;
             bool absent = false, present = false;
-            if constexpr (VEC) {
-                // Sk % 8 == 0 and 8-byte aligned rows: whole 8-key groups.
-                if (k < Sk) {
-                    const u32x2 m = *reinterpret_cast<const u32x2*>(mrow + k);
-                    present = (m[0] | m[1]) != 0u;
-                    absent = has_zero_byte(m);
-                }
-            } else {
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (k + j < Sk) {
-                        const bool p = mrow[k + j] != 0;
-                        present |= p;
-                        absent |= !p;
-                    }
-            }
+            for (int j = 0; j < 8; ++j)
+                if (k + j < Sk) {
+                    const bool p = mrow[k + j] != 0;
+                    present |= p;
+                    absent |= !p;
+                }
             const uint64_t ab = __ballot(absent);
             any_present |= __ballot(present) != 0ull;
 #pragma unroll
@@ -99,46 +95,29 @@ __device__ __forceinline__ RowFlags row_flags(const uint8_t* mrow, int Sk) {
     return {bits, (mrow && !any_present) ? 0.f : kMaskedLogit};
 }
 
-// Per-lane prefetch state of one key tile: the mask bytes of keys k0 + 32c + 8g + 0..7 (c = 0, 1)
-// and, unless the bias tile travels through LDS (VEC), the bias of those keys for each of the
-// lane's query rows. VEC (Sk % 8 == 0, 8-byte aligned mask rows): 8-byte mask loads whose address
-// is clamped into the row (keys past Sk are forced to -inf anyway); otherwise element loads.
-template <typename TR, int QT, bool VEC, bool BM = false>
+// Per-lane prefetch state of one key tile of the element-wise path: the mask bytes of keys
+// k0 + 32c + 8g + 0..7 (c = 0, 1) and the bias of those keys for each of the lane's query rows.
+template <typename TR, int QT>
 struct TilePrefetch {
     u32x2 mask[2];
-    u32x4 bias[VEC ? 1 : QT][2];
+    u32x4 bias[QT][2];
     __device__ __forceinline__ void load(const typename TR::elem* const* brow,
                                          const uint8_t* mrow, int k0, int g, int Sk) {
         using E = typename TR::elem;
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             const int kk = k0 + 32 * c + 8 * g;
-            if constexpr (VEC) {
-                if constexpr (BM) {
-                    // Keys k0 + 32c + 4g + 0..3 and k0 + 32c + 16 + 4g + 0..3 (the bias-MFMA
-                    // key order), 4-byte loads clamped into the row.
-                    const int k4 = k0 + 32 * c + 4 * g;
-                    mask[c] = mrow ? u32x2{*reinterpret_cast<const unsigned*>(mrow + min(k4, Sk - 4)),
-                                           *reinterpret_cast<const unsigned*>(
-                                               mrow + min(k4 + 16, Sk - 4))}
-                                   : u32x2{~0u, ~0u};
-                } else {
-                    mask[c] = mrow ? *reinterpret_cast<const u32x2*>(mrow + min(kk, Sk - 8))
-                                   : u32x2{~0u, ~0u};
-                }
-            } else {
-                uint8_t m[8];
+            uint8_t m[8];
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    m[j] = kk + j < Sk ? (mrow ? mrow[kk + j] : uint8_t(1)) : uint8_t(0);
-                __builtin_memcpy(&mask[c], m, 8);
+            for (int j = 0; j < 8; ++j)
+                m[j] = kk + j < Sk ? (mrow ? mrow[kk + j] : uint8_t(1)) : uint8_t(0);
+            __builtin_memcpy(&mask[c], m, 8);
 #pragma unroll
-                for (int qt = 0; qt < QT; ++qt) {
-                    E e[8];
+            for (int qt = 0; qt < QT; ++qt) {
+                E e[8];
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) e[j] = kk + j < Sk ? brow[qt][kk + j] : E(0.f);
-                    __builtin_memcpy(&bias[qt][c], e, 16);
-                }
+                for (int j = 0; j < 8; ++j) e[j] = kk + j < Sk ? brow[qt][kk + j] : E(0.f);
+                __builtin_memcpy(&bias[qt][c], e, 16);
             }
         }
     }
@@ -166,7 +145,13 @@ struct GateArgs {
     int C, HD;
 };
 
-template <typename TR, int D, int QT, bool VEC, bool GATE, bool BM, bool NSHD>
+// ODD (VEC and BM): Sk is odd. The direct-to-LDS loads of the bias need 4-byte aligned addresses,
+// and every other bias row starts half a dword off. A block then owns queries of one parity
+// (query q0 + 2i for its i-th row), whose bias rows are all aligned or all off by one element;
+// in the second case its key tiles start one key early (tile kt: keys 64kt - 1 ...), which
+// aligns every load, and key -1 is an absent key. So the loop is the even one, with no shifting
+// of bias pieces.
+template <typename TR, int D, int QT, bool VEC, bool GATE, bool BM, bool NSHD, bool ODD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && VEC ? 3 : 1))) void attn_fwd_kernel(
     const typename TR::elem* __restrict__ q, const typename TR::elem* __restrict__ k,
     const typename TR::elem* __restrict__ v, const typename TR::elem* __restrict__ bias,
@@ -174,6 +159,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     float* __restrict__ lse, int H, int Sq, int Sk, float scale,
     GateArgs<typename TR::elem> ga, BiasMfma bm, int grp) {
     static_assert(!BM || VEC, "the bias MFMA reads the bias tile from LDS");
+    static_assert(!ODD || BM, "odd key counts run the bias-MFMA form");
     static_assert(!(NSHD && GATE), "the gated entry takes the [N, H, S, D] layout");
     using E = typename TR::elem;
     using V8 = typename TR::vec8;
@@ -189,11 +175,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     // exponent's FMA against the running max leaves a rounding residue of about 2^-24 of the
     // logit, which must stay far below float32's exponent range.)
     constexpr bool PATCH = VEC;
-    using PF = TilePrefetch<TR, QT, VEC, BM>;
+    using PF = TilePrefetch<TR, QT>;
     constexpr int BQ = 4 * 16 * QT;
     constexpr int BK = G::BK;
     constexpr int TILE = BK * T::ROWB;  // bytes of one K or V tile
     constexpr int BTILE = VEC ? BQ * 128 : 0;  // bias tile: BQ query rows of 64 keys
+    constexpr int QS = ODD ? 2 : 1;            // query step between a block's rows
 
     // Two K/V buffers as separate LDS objects: the compiler then knows that reads of one do not
     // wait for the direct-to-LDS loads into the other.
@@ -210,11 +197,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     // groups of grp rows, then the query tile, then the row within its group -- an XCD's resident
     // blocks then read one head's bias rows (the same for every row n) and the K and V of a few
     // rows, both of which stay in its L2.
-    const int qtiles = (Sq + BQ - 1) / BQ;
+    // ODD: the even and the odd queries of a range of 2*BQ are neighbouring work items.
+    const int qtiles = QS * (((Sq + QS - 1) / QS + BQ - 1) / BQ);
     const int item = xcd_contiguous(blockIdx.x, gridDim.x);
     int q0, h, n;
     if (grp == 0) {
-        q0 = (item % qtiles) * BQ;
+        q0 = item % qtiles;
         h = (item / qtiles) % H;
         n = item / (qtiles * H);
     } else {
@@ -222,9 +210,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
         h = item / per_head;
         const int rem = item - h * per_head;
         const int gi = rem / (grp * qtiles), nb = gi * grp, gsz = min(grp, nrows - nb);
-        q0 = (rem - gi * grp * qtiles) / gsz * BQ;
+        q0 = (rem - gi * grp * qtiles) / gsz;
         n = nb + (rem - gi * grp * qtiles) % gsz;
     }
+    q0 = ODD ? (q0 >> 1) * 2 * BQ + (q0 & 1) : q0 * BQ;
     const size_t nh = (size_t)n * H + h;
     // Rows of one (n, h) in q, k, v and out: [N, H, S, D] (rows D apart), or with NSHD
     // [N, S, H, D] (rows H*D apart, head h at column block h).
@@ -235,49 +224,59 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     E* const op = out ? out + (NSHD ? ((size_t)n * Sq * H + h) * D : nh * Sq * D) : nullptr;
     const E* bp = bias + (size_t)h * Sq * Sk;
     const uint8_t* mp = kmask ? kmask + (size_t)n * Sk : nullptr;
-    const int qbase = q0 + wave * 16 * QT;
-    const int ntiles = (Sk + BK - 1) / BK;
+    const int qbase = q0 + wave * 16 * QT * QS;
+    // Keys the block's tiles start before key 0 (0 or 1; every row of the block agrees).
+    const int shift = ODD ? (h * Sq + q0) & 1 : 0;
+    const int ntiles = (Sk + shift + BK - 1) / BK;
 
     // The Sk rows of (n, h): rows past Sk read zeros.
     const uint32_t kvbytes = NSHD ? (Sk > 0 ? (uint32_t)(((size_t)(Sk - 1) * ld + D) * 2) : 0u)
                                   : (uint32_t)Sk * D * 2;
     const Rsrc rk = buffer_rsrc(kp, kvbytes);
     const Rsrc rv = buffer_rsrc(vp, kvbytes);
-    // The block's bias rows (queries q0 .. q0+BQ-1 that exist).
-    const Rsrc rb = buffer_rsrc(bp + (size_t)q0 * Sk, (uint32_t)(min(BQ, Sq - q0) * Sk * 2));
+    // The block's bias rows (queries q0 + QS*i, i < BQ, that exist), from `shift` keys before the
+    // first. Its end is rounded up to a dword (loads are range-checked by dword): for ODD the bias
+    // of all heads is an even number of elements, so that dword lies inside it.
+    const int brows = min(BQ, (Sq - q0 + QS - 1) / QS);
+    const Rsrc rb = buffer_rsrc(bp + (size_t)q0 * Sk - shift,
+                                brows > 0 ? (uint32_t)((((brows - 1) * QS * Sk + Sk + shift) * 2 + 3) & ~3)
+                                          : 0u);
     // Head h's D columns of the gate weight: row c (channel) starts HD elements after row c-1.
     const Rsrc rw = GATE ? buffer_rsrc(ga.wg + h * D, (uint32_t)((ga.C - 1) * ga.HD + D) * 2)
                          : rb;
     auto stage = [&](int k0, char* kv) {
-        if constexpr (NSHD) {
-            stage_rows_ld<D, BK, 256>(rk, k0, ld, kv, threadIdx.x);
-            stage_rows_ld<D, BK, 256>(rv, k0, ld, kv + TILE, threadIdx.x);
+        if (ODD && k0 == 0) {  // row -1 (shift = 1) reads zeros
+            stage_rows_from<D, BK, 256>(rk, -shift, ld, kv, threadIdx.x);
+            stage_rows_from<D, BK, 256>(rv, -shift, ld, kv + TILE, threadIdx.x);
+        } else if constexpr (NSHD) {
+            stage_rows_ld<D, BK, 256>(rk, k0 - shift, ld, kv, threadIdx.x);
+            stage_rows_ld<D, BK, 256>(rv, k0 - shift, ld, kv + TILE, threadIdx.x);
         } else {
-            stage_rows<D, BK, 256>(rk, k0, kv);
-            stage_rows<D, BK, 256>(rv, k0, kv + TILE);
+            stage_rows<D, BK, 256>(rk, k0 - shift, kv);
+            stage_rows<D, BK, 256>(rv, k0 - shift, kv + TILE);
         }
         if constexpr (VEC) {
-            // Bias rows q0 .. q0+BQ-1, keys k0 .. k0+63 as eight 16-byte pieces per row; piece
+            // The block's bias rows, keys k0 - shift .. + 63 as eight 16-byte pieces per row; piece
             // p of row r sits at position p ^ (r & 7), so a 16-row operand read is conflict-free.
-            // Rows past Sq read zeros; keys past Sk (last tile) read whatever follows, and are
-            // forced to -inf.
+            // Rows past Sq read zeros; keys past Sk (last tile) and key -1 read what lies there,
+            // and are patched.
 #pragma unroll
             for (int b = wave * 64; b < BQ * 8; b += 256) {
                 const int slot = b + lane;
                 const int row = slot >> 3, piece = (slot & 7) ^ (row & 7);
-                buf_dma16(rb, (row * Sk + 8 * piece) * 2, k0 * 2, kv + 2 * TILE + b * 16);
+                buf_dma16(rb, (row * QS * Sk + 8 * piece) * 2, k0 * 2, kv + 2 * TILE + b * 16);
             }
         }
     };
     // PATCH: this wave's mask bytes of its first two key tiles (t = wave, wave + 4; lane l:
-    // key 64t + l), loaded before anything else so that the presence words below wait for them
+    // key 64t + l - shift), loaded before anything else so that the presence words below wait for them
     // alone.
     uint32_t mb[2] = {0u, 0u};
     if constexpr (PATCH) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int kk = (wave + 4 * i) * BK + lane;
-            if (kk < Sk) mb[i] = mp ? mp[kk] : 1u;
+            const int kk = (wave + 4 * i) * BK + lane - shift;
+            if (kk >= 0 && kk < Sk) mb[i] = mp ? mp[kk] : 1u;
         }
     }
     if (ntiles > 0) stage(0, kv0);
@@ -286,7 +285,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     V8 qf[QT][G::KS];
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
-        const int row = qbase + qt * 16 + r16;
+        const int row = qbase + (qt * 16 + r16) * QS;
 #pragma unroll
         for (int ks = 0; ks < G::KS; ++ks) {
             const int d0 = ks * 32 + g * 8;
@@ -296,17 +295,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
         }
     }
 
-    // Bias rows of the lane's queries (clamped inside [0, Sq)), keys 32c + 8g + 0..7 per tile.
+    // Not PATCH: bias rows of the lane's queries (clamped inside [0, Sq)), keys 32c + 8g + 0..7
+    // per tile.
     const E* brow[QT];
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) brow[qt] = bp + (size_t)min(qbase + qt * 16 + r16, Sq - 1) * Sk;
     PF ca, cb;
-    if (ntiles > 0) ca.load(brow, mp, 0, g, Sk);
+    if (!PATCH && ntiles > 0) ca.load(brow, mp, 0, g, Sk);
     // The mask row's tile flags, with the Q and first-tile loads already in flight (PATCH
     // reads the same facts from the presence words instead).
-    const RowFlags rf = PATCH ? RowFlags{0ull, kMaskedLogit} : row_flags<VEC>(mp, Sk);
-    // PATCH: the row's presence bits, one 64-bit word per key tile (bit j: key 64t + j is
-    // present and below Sk; the launch keeps ntiles <= kPresWords), and per wave 1 + the last
+    const RowFlags rf = PATCH ? RowFlags{0ull, kMaskedLogit} : row_flags(mp, Sk);
+    // PATCH: the row's presence bits, one 64-bit word per key tile (bit j: key 64t + j - shift
+    // exists and is present; the launch keeps ntiles <= kPresWords), and per wave 1 + the last
     // of its tiles that holds a present key (0 if none).
     __shared__ unsigned long long pres[PATCH ? kPresWords : 1];
     __shared__ int wave_last[PATCH ? 4 : 1];
@@ -322,7 +322,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             }
         }
         for (int t = wave + 8; t < ntiles; t += 4) {
-            const int kk = t * BK + lane;
+            const int kk = t * BK + lane - shift;
             const unsigned long long b = __ballot(kk < Sk && (mp == nullptr || mp[kk] != 0));
             if (b != 0ull) last = t + 1;
             if (lane == 0) pres[t] = b;
@@ -366,9 +366,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             }
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-            const int kk = kt * BK + 32 * c + 8 * g;
-            // A key past Sk gets the fill value in every row.
-            const uint32_t fill = kk < Sk && row_empty ? 0u : neg;
+            // (A row without any present key runs tile_empty, which reads no bias.)
             const uint32_t bits = reinterpret_cast<const uint32_t*>(pres)[2 * kt + c] >> (8 * g);
             // Dword i holds keys 2i, 2i+1 (low, high half): keep the bias of present keys.
 #pragma unroll
@@ -377,7 +375,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
                                       ((bits >> (2 * i + 1)) & 1u ? 0xffff0000u : 0u);
 #pragma unroll
                 for (int qt = 0; qt < QT; ++qt)
-                    v[c][qt][i] = (v[c][qt][i] & keep) | (fill & ~keep);
+                    v[c][qt][i] = (v[c][qt][i] & keep) | (neg & ~keep);
             }
         }
 #pragma unroll
@@ -427,7 +425,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
         __syncthreads();  // tile kt visible; every wave is done with the other buffer
         bool need_mask;
         if constexpr (PATCH) {
-            const int rem = Sk - k0;  // keys of the tile below Sk
+            const int rem = Sk + shift - k0;  // keys of the tile below Sk
             const unsigned long long full = rem >= 64 ? ~0ull : (1ull << rem) - 1ull;
             need_mask = (rem < 64) || pres[kt] != full;
         } else {
@@ -435,7 +433,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
         }
         if (kt + 1 < nrun) {
             stage(k0 + BK, kvn);
-            nxt.load(brow, mp, k0 + BK, g, Sk);
+            if constexpr (!PATCH) nxt.load(brow, mp, k0 + BK, g, Sk);
         } else if constexpr (GATE) {
             // The last key tile leaves the other buffer free: the wg rows of the first
             // kGateChannels gate channels go there now, ready for the epilogue.
@@ -525,16 +523,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             asm volatile("");
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
-                // Slot j is key k0 + 32c + 8g + j, or in the bias-MFMA order
-                // k0 + 32c + 4g + j (j < 4) and k0 + 32c + 12 + 4g + j (j >= 4): it is past Sk
-                // when j (j + 12 for the upper four of that order) >= lim.
-                const int lim = Sk - (k0 + 32 * c + (BM ? 4 : 8) * g);
+                // Slot j is key k0 + 32c + 8g + j.
+                const int lim = Sk - (k0 + 32 * c + 8 * g);
                 const unsigned valid = cur.valid(c);
 #pragma unroll
                 for (int qt = 0; qt < QT; ++qt)
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
-                        x[qt][c][j] = (BM && j >= 4 ? j + 12 : j) >= lim
+                        x[qt][c][j] = j >= lim
                                           ? -INFINITY
                                           : (((valid >> j) & 1u) ? x[qt][c][j] : masked_logit);
             }
@@ -589,13 +585,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     // PATCH, a row without any present key: every logit in range is the masked logit 0, so
     // P = 1 there (and 0 past Sk) with the running max at 0 -- the values the tiles above
     // compute for such a row -- and a tile needs only its V rows: no S, no exponential.
-    auto tile_empty = [&](int kt, const char* kvc, char* kvn, PF& cur, PF& nxt) {
+    auto tile_empty = [&](int kt, const char* kvc, char* kvn) {
         const int k0 = kt * BK;
         async_wait();
         __syncthreads();  // tile kt visible; every wave is done with the other buffer
         if (kt + 1 < nrun) {
             stage(k0 + BK, kvn);
-            nxt.load(brow, mp, k0 + BK, g, Sk);
         } else if constexpr (GATE) {
             int t = threadIdx.x;
             asm volatile("" : "+v"(t));
@@ -608,16 +603,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             for (int c = 0; c < 2; ++c)
                 vf[dt][c] = BM ? swz_tr_operand_split<V8, D>(kvc + TILE, 32 * c, dt, r16, g)
                                : swz_tr_operand<V8, D>(kvc + TILE, 32 * c, dt, r16, g);
-        // Slot j of chunk c is key k0 + 32c + 8g + j, or in the bias-MFMA order
-        // k0 + 32c + 4g + j (j < 4) and k0 + 32c + 12 + 4g + j (j >= 4).
+        // Slot j of chunk c is key k0 - shift + 32c + 8g + j, or in the bias-MFMA order
+        // k0 - shift + 32c + 4g + j (j < 4) and k0 - shift + 32c + 12 + 4g + j (j >= 4). (Key -1,
+        // the first slot of lane group 0 in tile 0 when shift = 1, has P = 0.)
         V8 pf[2];
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-            const int lim = Sk - (k0 + 32 * c + (BM ? 4 : 8) * g);
+            const int lim = Sk + shift - (k0 + 32 * c + (BM ? 4 : 8) * g);
 #pragma unroll
             for (int j = 0; j < 8; ++j)
                 pf[c][j] = TR::from_f((BM && j >= 4 ? j + 12 : j) < lim ? 1.f : 0.f);
         }
+        if (ODD && k0 == 0 && g == 0 && shift) pf[0][0] = TR::from_f(0.f);
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
 #pragma unroll
@@ -632,8 +629,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) nm[qt] = 0.f;
         for (int kt = 0; kt < nrun; kt += 2) {
-            tile_empty(kt, kv0, kv1, ca, cb);
-            if (kt + 1 < nrun) tile_empty(kt + 1, kv1, kv0, cb, ca);
+            tile_empty(kt, kv0, kv1);
+            if (kt + 1 < nrun) tile_empty(kt + 1, kv1, kv0);
         }
     } else {
         for (int kt = 0; kt < nrun; kt += 2) {
@@ -676,7 +673,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             V8 xo[QT][NX];
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
-                const int row = qbase + qt * 16 + gr16;
+                const int row = qbase + (qt * 16 + gr16) * QS;
 #pragma unroll
                 for (int j = 0; j < NX; ++j) {
                     const int c = c0 + 32 * j;
@@ -718,7 +715,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     for (int qt = 0; qt < QT; ++qt) {
         const float l_tot = lsum[qt][0];
         const float inv = 1.0f / fmaxf(l_tot, 1e-30f);
-        const int row = qbase + qt * 16 + er16;
+        const int row = qbase + (qt * 16 + er16) * QS;
         if (row >= Sq) continue;
 #pragma unroll
         for (int dt = 0; dt < G::DT; ++dt) {
@@ -747,31 +744,38 @@ void launch_fwd_qt(hipStream_t st, const void* q, const void* k, const void* v, 
                    const uint8_t* kmask, void* out, float* lse, int N, int H, int Sq, int Sk,
                    float scale, GateArgs<typename TR::elem> ga) {
     using E = typename TR::elem;
-    const dim3 grid(ceil_div(Sq, 64 * QT) * H * N);
+    // The bias tile through LDS (direct loads of 4-byte aligned pieces): at most kPresWords key
+    // tiles (masked bias tiles are changed in LDS from presence words kept there). An even Sk
+    // aligns every bias row. An odd one takes the parity form of the bias-MFMA kernel, when the
+    // bias is a whole number of dwords (no load then reaches past its end). Other odd cases
+    // (scale <= 0, one head or an odd number of them with an odd Sq) and longer rows read bias and
+    // mask element by element, about four times slower (2395 against 550 us at 757 residues).
+    BiasMfma bm{};
+    const bool bmf = bias_mfma_for<TR>(scale, &bm);
+    const bool odd = Sk % 2 && bmf && (size_t)H * Sq * Sk % 2 == 0;
+    const bool vec = (Sk % 2 == 0 || odd) && Sk + (odd ? 1 : 0) <= kPresWords * 64;
+    const int BQ = 64 * QT;
+    const int qtiles = vec && odd ? 2 * ceil_div((Sq + 1) / 2, BQ) : ceil_div(Sq, BQ);
+    const dim3 grid(qtiles * H * N);
     // The head-outer work-item order when the bias of all heads passes half of an XCD's 4 MB L2,
     // in groups of rows whose query tiles make about 48 work items, half an XCD's resident
     // blocks (32 CUs x 3): at N_res = 1024 (8 MB of bias) this cut the launch's fetch from 8.2 to
     // 0.9 GB and its time by 9% (any group of 4 to 24 rows within 1%). Otherwise the head stays
     // inside the row: the MSA shapes' gate rows and [N, S, H, D] rows are shared by the heads.
     const bool head_outer = (size_t)H * Sq * Sk * 2 > (2u << 20);
-    const int grp = head_outer ? max(1, min(N, 48 / ceil_div(Sq, 64 * QT))) : 0;
-    // The bias tile through LDS: whole 8-key pieces, 8-byte aligned mask rows and at most
-    // kPresWords key tiles (masked bias tiles are changed in LDS from presence words kept there).
-    const bool vec = Sk % 8 == 0 && (reinterpret_cast<uintptr_t>(kmask) & 7u) == 0 &&
-                     Sk <= kPresWords * 64;
-    BiasMfma bm{};
-    if (vec && bias_mfma_for<TR>(scale, &bm))
-        attn_fwd_kernel<TR, D, QT, true, GATE, true, NSHD><<<grid, 256, 0, st>>>(
-            (const E*)q, (const E*)k, (const E*)v, (const E*)bias, kmask, (E*)out, lse, H, Sq, Sk,
-            scale, ga, bm, grp);
+    const int grp = head_outer ? max(1, min(N, 48 / qtiles)) : 0;
+    auto run = [&](auto kernel) {
+        kernel<<<grid, 256, 0, st>>>((const E*)q, (const E*)k, (const E*)v, (const E*)bias, kmask,
+                                     (E*)out, lse, H, Sq, Sk, scale, ga, bm, grp);
+    };
+    if (vec && odd)
+        run(attn_fwd_kernel<TR, D, QT, true, GATE, true, NSHD, true>);
+    else if (vec && bmf)
+        run(attn_fwd_kernel<TR, D, QT, true, GATE, true, NSHD, false>);
     else if (vec)
-        attn_fwd_kernel<TR, D, QT, true, GATE, false, NSHD><<<grid, 256, 0, st>>>(
-            (const E*)q, (const E*)k, (const E*)v, (const E*)bias, kmask, (E*)out, lse, H, Sq, Sk,
-            scale, ga, bm, grp);
+        run(attn_fwd_kernel<TR, D, QT, true, GATE, false, NSHD, false>);
     else
-        attn_fwd_kernel<TR, D, QT, false, GATE, false, NSHD><<<grid, 256, 0, st>>>(
-            (const E*)q, (const E*)k, (const E*)v, (const E*)bias, kmask, (E*)out, lse, H, Sq, Sk,
-            scale, ga, bm, grp);
+        run(attn_fwd_kernel<TR, D, QT, false, GATE, false, NSHD, false>);
 }
 
 template <typename TR, int D, bool GATE>

@@ -272,3 +272,45 @@ def test_attention_row_with_no_weight(cuda):
     assert_close("dK", dk, rk, tol)
     assert_close("dV", dv, rv, tol)
     assert_close("dBias", dbias, rb, tol)
+
+
+# (N, H, Sq, Sk, D): odd key counts around the edges of the 64-key tiles (blocks of one query
+# parity, half of them with tiles that start at key -1), odd and even query counts around the
+# edges of the 64- and 128-query blocks, one head (its odd biases read element by element) and
+# even key counts that are no multiple of 8.
+RAGGED_SHAPES = [(5, 2, 1, 1, 32), (5, 2, 2, 3, 8), (5, 4, 63, 63, 32), (5, 2, 64, 65, 16),
+                 (5, 2, 65, 127, 32), (5, 3, 128, 129, 32), (5, 3, 129, 129, 32),
+                 (5, 2, 255, 191, 8), (5, 2, 257, 193, 64), (5, 1, 130, 67, 32), (5, 2, 70, 66, 32),
+                 (5, 3, 131, 190, 16), (5, 4, 515, 513, 32)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=dname)
+@pytest.mark.parametrize("shape", RAGGED_SHAPES, ids=lambda c: "x".join(map(str, c)))
+def test_attention_fwd_ragged_keys(cuda, shape, dtype):
+    """Key counts that are no multiple of 8, with per-row masks: all present, none present, key 0
+    absent, only the last key present, random holes. Both layouts, against the oracle."""
+    n, h, sq, sk, d = shape
+    inp = attention_inputs(n, h, sq, sk, d, dtype, seed=sk + 7 * sq, with_dout=False)
+    gen = torch.Generator().manual_seed(sk + sq)
+    km = torch.ones((n, sk), dtype=torch.uint8)
+    km[1] = 0
+    km[2, 0] = 0
+    km[2, sk - 1] = 1
+    km[3, :sk - 1] = 0
+    km[4] = (torch.rand(sk, generator=gen) > 0.3).to(torch.uint8)
+    km[4, sk // 2] = 1
+    inp["kmask"] = km
+    g = {k: (v.to(cuda) if isinstance(v, torch.Tensor) else v) for k, v in inp.items()}
+    out, lse = ops.attention_fwd(g["q"], g["k"], g["v"], g["bias"], g["kmask"], g["scale"])
+    o_ref, lse_ref = _oracle(inp)
+    assert_close("O", out, o_ref, TOL[dname(dtype)]["o"])
+    empty = (km.numpy() == 0).all(axis=1)[:, None, None]
+    assert np.abs(np64(lse) - np.where(empty, np.log(sk), lse_ref)).max() < 5e-2
+    t = lambda x: x.transpose(1, 2).contiguous()  # noqa: E731
+    out_s, lse_s = ops.attention_nshd(t(g["q"]), t(g["k"]), t(g["v"]), g["bias"], g["kmask"],
+                                      g["scale"], want_lse=True)
+    assert torch.equal(t(out_s), out) and torch.equal(lse_s, lse)
+    # A negative scale takes the form without the bias MFMA (odd: the element-wise path).
+    neg = {**inp, "scale": -inp["scale"]}
+    out_n = ops.attention(g["q"], g["k"], g["v"], g["bias"], g["kmask"], neg["scale"])
+    assert_close("O (negative scale)", out_n, _oracle(neg)[0], TOL[dname(dtype)]["o"])
