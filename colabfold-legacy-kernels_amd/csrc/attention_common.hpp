@@ -346,7 +346,7 @@ struct LogitForm {
 // operand is [hi*I | lo*I] (hi + lo = 1/scale as two values of the input type, each product
 // with a bias value exact in float32) and whose B operand is the tile's bias, duplicated over
 // the two halves of the contraction; the tile then holds logit / scale, and
-// log2(e) * logit = cexp * S with cexp = scale * log2(e). No per-score instruction touches the bias. A bias of
+// log2(e) * logit = cexp * S with cexp = log2(e) / (hi + lo). No per-score instruction touches the bias. A bias of
 // magnitude above 3.4e38 * scale overflows there (float32 cannot hold bias / scale).
 struct BiasMfma {
     float hi, lo, bscale, cexp;
@@ -360,8 +360,11 @@ bool bias_mfma_for(float scale, BiasMfma* bm) {
     if (!(scale > 0.f) || !std::isfinite(scale)) return false;
     const float b = 1.f / scale;
     if (!std::isfinite(b) || b > 6.0e4f) return false;
-    const float hi = (float)(E)b;
-    *bm = {hi, (float)(E)(b - hi), b, scale * kLog2e};
+    const float hi = (float)(E)b, lo = (float)(E)(b - hi);
+    // The exponent's unit is that of hi + lo, not of 1/scale: the bias then enters exactly, whatever
+    // its size (additive masks of -1e4 and beyond), and the last rounding of the pair falls on the
+    // scale of q.k (relative 3e-7 in bfloat16 at D = 32, within float32's own rounding in float16).
+    *bm = {hi, lo, b, (float)((double)kLog2e / ((double)hi + lo))};
     return true;
 }
 
