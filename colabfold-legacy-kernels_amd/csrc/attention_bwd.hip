@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dq(
 #pragma unroll
                 for (int c = 0; c < 2; ++c) {
                     const int kk = k0 + 32 * c + 8 * g;
-                    load_bias8<TR>(brow_p, kk, Sk, vec_ok, bv[c]);
+                    load_bias8<TR>(brow_p, kk, Sk, bv[c]);
                     valid[c] = key_valid8(mp, kk, Sk, vec_ok);
                     all_valid = all_valid && valid[c] == 0xffu && kk + 8 <= Sk;
                 }
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv(
     const uint8_t* __restrict__ kmask, const typename TR::elem* __restrict__ dout,
     const float* __restrict__ lse, const float* __restrict__ di,
     typename TR::elem* __restrict__ dk, typename TR::elem* __restrict__ dv, int H, int Sq, int Sk,
-    float scale, int vec_ok) {
+    float scale) {
     using E = typename TR::elem;
     using V8 = typename TR::vec8;
     using G = AttnGeom<D>;
@@ -315,8 +315,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv(
             breg[i] = u32x4{0u, 0u, 0u, 0u};
             if (gq < Sq) {
                 const E* p = bhead + (size_t)gq * Sk + gk;
-                if (vec_ok && gk + 8 <= Sk) {
-                    breg[i] = ld16(p);
+                if (gk + 8 <= Sk) {
+                    breg[i] = ld16_a2(p);
                 } else {
                     E e[8];
 #pragma unroll
@@ -419,34 +419,6 @@ __global__ __launch_bounds__(256) void attn_bwd_dkv(
 // launch whose operands all arrive by direct global->LDS loads into static double buffers.
 // ---------------------------------------------------------------------------------------------
 
-// Bit j set when byte j of the eight is nonzero.
-__device__ __forceinline__ unsigned nonzero_bits8(u32x2 w) {
-    unsigned bits = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        bits |= (((w[0] >> (8 * j)) & 0xffu) != 0u ? 1u : 0u) << j;
-        bits |= (((w[1] >> (8 * j)) & 0xffu) != 0u ? 1u : 0u) << (4 + j);
-    }
-    return bits;
-}
-
-// Mask bytes of keys kk .. kk+7 of one mask row (0 past Sk; all present without a mask). VEC:
-// one 8-byte load (Sk % 8 == 0, 8-byte aligned rows), the address clamped into the row.
-template <bool VEC>
-__device__ __forceinline__ u32x2 mask_bytes8(const uint8_t* mrow, int kk, int Sk) {
-    if (!mrow) return u32x2{~0u, ~0u};
-    if constexpr (VEC) {
-        return *reinterpret_cast<const u32x2*>(mrow + min(kk, Sk - 8));
-    } else {
-        uint8_t b[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) b[j] = kk + j < Sk ? mrow[kk + j] : uint8_t(0);
-        u32x2 w;
-        __builtin_memcpy(&w, b, 8);
-        return w;
-    }
-}
-
 // Tile t (of H * tiles_q * tiles_k) of bias [H][Sq][Sk] -> bias_t [H][Sk][SqP] (SqP = Sq rounded
 // up to 64, padding zero), through the 64 x 64 LDS tile `tile`, by threads tid, tid + nthreads,
 // ... of the block. Returns after the stores are issued; the caller synchronises before `tile`
@@ -461,15 +433,14 @@ __device__ void transpose_bias_tile(const typename TR::elem* __restrict__ bias,
     t /= tiles_k;
     const int tq = t % tiles_q, h = t / tiles_q;
     const int q0 = tq * 64, k0 = tk * 64;
-    // Loads: 16-byte pieces of 8 keys of one query row when the piece lies inside the row and
-    // the rows are 16-byte aligned; element loads otherwise.
-    const bool vec = Sk % 8 == 0;
+    // Loads: 16-byte pieces of 8 keys of one query row when the piece lies inside the row (2-byte
+    // aligned for a ragged Sk); element loads otherwise.
     for (int ch = tid; ch < 512; ch += nthreads) {
         const int r = ch >> 3, c8 = (ch & 7) * 8;  // r: query, c8: first key
         const int qq = q0 + r, kk = k0 + c8;
         E e[8];
-        if (vec && qq < Sq && kk + 8 <= Sk) {
-            const u32x4 raw = ld16(bias + ((size_t)h * Sq + qq) * Sk + kk);
+        if (qq < Sq && kk + 8 <= Sk) {
+            const u32x4 raw = ld16_a2(bias + ((size_t)h * Sq + qq) * Sk + kk);
             __builtin_memcpy(e, &raw, 16);
         } else {
 #pragma unroll
@@ -522,7 +493,10 @@ __device__ __forceinline__ void stage_rows_wave(Rsrc r, int r0, int ld, char* ld
 // the wave computes S^T = K.Q^T and dP^T - D = V.dO^T - D (D_i = rowsum(dO*O) enters as the
 // accumulator input), dS, and dQ^T += K^T.dS^T. The four key-quarter waves of a query group
 // then add their dQ partials through LDS in a fixed order. Also writes lse*log2(e) and -D_i
-// per query for the column-owner pass.
+// per query for the column-owner pass. VEC: Sk % 8 == 0, so that the bias rows and the dBias rows
+// are 16-byte aligned; it only matters where a block loads its bias and stores its dBias. (Lse,
+// mask bytes and the masked bits read per row and lane, as a ragged Sk once did, cost 56 against
+// 37.5 us at 203 residues, 4 heads x 32.)
 template <typename TR, int D, int KCW, bool VEC, int QG, int QTW, bool NSHD>
 __global__ __launch_bounds__(256 * QG) void attn_bwd_dq2(
     const typename TR::elem* __restrict__ q, const typename TR::elem* __restrict__ k,
@@ -547,11 +521,11 @@ __global__ __launch_bounds__(256 * QG) void attn_bwd_dq2(
 
     __shared__ __attribute__((aligned(16))) char kv0[2 * KVB];
     __shared__ __attribute__((aligned(16))) char kv1[2 * KVB];
-    // Per-row extras staged with Q/dO/O when VEC: lse of the block's 64 queries (256 bytes),
+    // Per-row extras staged with Q/dO/O: lse of the block's 64 queries (256 bytes),
     // then the row's presence words of the key range (RK/64 64-bit words; one wave of 4-byte
     // loads, 256 bytes).
     static_assert(RK % 64 == 0 && RK / 32 <= 64, "presence words of a key range: one wave");
-    constexpr int XB = VEC ? 512 : 0;
+    constexpr int XB = 512;
     __shared__ __attribute__((aligned(16))) char qd0[3 * QB + XB];
     __shared__ __attribute__((aligned(16))) char qd1[3 * QB + XB];
     __shared__ __attribute__((aligned(16))) char xch_raw[NWV * QTW * DT * 64 * 16];
@@ -590,8 +564,7 @@ __global__ __launch_bounds__(256 * QG) void attn_bwd_dq2(
             if constexpr (VEC) {
                 unpack8<TR>(ld16(brow + min(kk, Sk - 8)), b);
             } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) b[j] = kk + j < Sk ? TR::to_f(brow[kk + j]) : 0.f;
+                load_bias8<TR>(brow, kk, Sk, b);
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j) bacc[i][qt][j >> 2][j & 3] = lf.bias_units(b[j]);
@@ -647,38 +620,23 @@ __global__ __launch_bounds__(256 * QG) void attn_bwd_dq2(
         } else {
             stage_rows_wave<D, BQ, HW>(buffer_rsrc(dout + qo, qb), q0, ld, qd + QB, wv - HW,
                                        lane);
-            if constexpr (VEC) {
-                // Queries past Sq and keys past Sk read zeros. Mask rows are 8-byte aligned.
-                char* ex = qd + 3 * QB;
-                const size_t nh = (size_t)n * H + h;
-                if (wv == HW)
-                    buf_dma4(buffer_rsrc(lse + nh * Sq, (uint32_t)Sq * 4), lane * 4, q0 * 4, ex);
-                // Words kbeg/64 .. of the row's presence bits (kbeg % 64 == 0); words past the
-                // row read zeros.
-                const int words = (Sk + 63) >> 6;
-                if (kmask && wv == HW + 1)
-                    buf_dma4(buffer_rsrc(mbits + (size_t)n * words, (uint32_t)words * 8),
-                             lane * 4, (kbeg >> 6) * 8, ex + 256);
-            }
-        }
-    };
-    // Per-row values kept in registers one row ahead when they are not staged (not VEC), raw:
-    // anything computed from them right after the load would wait for the row's direct-to-LDS
-    // loads too.
-    float lse_nx[VEC ? 1 : QTW], ml_nx = kMaskedLogit;
-    u32x2 mask_nx[VEC ? 1 : KCW];
-    auto prefetch = [&](int n) {
-        if constexpr (!VEC) {
+            // Queries past Sq and keys past Sk read zeros.
+            char* ex = qd + 3 * QB;
             const size_t nh = (size_t)n * H + h;
-#pragma unroll
-            for (int qt = 0; qt < QTW; ++qt) lse_nx[qt] = lse[nh * Sq + min(qrow[qt], Sq - 1)];
-            const uint8_t* mrow = kmask ? kmask + (size_t)n * Sk : nullptr;
-#pragma unroll
-            for (int i = 0; i < KCW; ++i)
-                mask_nx[i] = mask_bytes8<VEC>(mrow, kbeg + 32 * (i * KQ + kq) + 8 * g, Sk);
+            if (wv == HW)
+                buf_dma4(buffer_rsrc(lse + nh * Sq, (uint32_t)Sq * 4), lane * 4, q0 * 4, ex);
+            // Words kbeg/64 .. of the row's presence bits (kbeg % 64 == 0); words past the
+            // row read zeros.
+            const int words = (Sk + 63) >> 6;
+            if (kmask && wv == HW + 1)
+                buf_dma4(buffer_rsrc(mbits + (size_t)n * words, (uint32_t)words * 8),
+                         lane * 4, (kbeg >> 6) * 8, ex + 256);
         }
-        ml_nx = kmask ? row_logit[n] : kMaskedLogit;
     };
+    // The next row's masked logit, kept in a register one row ahead, raw: anything computed from
+    // it right after the load would wait for the row's direct-to-LDS loads too.
+    float ml_nx = kMaskedLogit;
+    auto prefetch = [&](int n) { ml_nx = kmask ? row_logit[n] : kMaskedLogit; };
 
     // dQ of the last row (this wave's slice), stored at the start of the next step by the waves
     // kq < QTW * DT: sub-tile dqt, head dims dd .. dd+3 of query qrow[dqt], at element offset
@@ -724,35 +682,26 @@ __global__ __launch_bounds__(256 * QG) void attn_bwd_dq2(
         const float mlc = ml_nx;
         // Presence bits of this wave's keys: chunk i in bits 8i .. 8i+7 (one register).
         unsigned vbits = 0;
-        if constexpr (VEC) {
-            const char* ex = qdc + 3 * QB;
+        const char* ex = qdc + 3 * QB;
 #pragma unroll
-            for (int qt = 0; qt < QTW; ++qt) {
-                // Read in every lane (queries past Sq read the staged zeros), then selected.
-                const float l = reinterpret_cast<const float*>(ex)[16 * QTW * qg + 16 * qt + r16];
-                lse2c[qt] = qrow[qt] < Sq ? l * kLog2e : INFINITY;
-            }
-            if (kmask) {
-                // Chunk i's 32 keys start at bit rel % 64 of staged word rel / 64 (rel = key
-                // offset in the range, a multiple of 32); the lane's 8 keys are bits 8g .. 8g+7
-                // of that. The word's address is the same in every lane (an LDS broadcast).
-                const unsigned long long* wd =
-                    reinterpret_cast<const unsigned long long*>(ex + 256);
+        for (int qt = 0; qt < QTW; ++qt) {
+            // Read in every lane (queries past Sq read the staged zeros), then selected.
+            const float l = reinterpret_cast<const float*>(ex)[16 * QTW * qg + 16 * qt + r16];
+            lse2c[qt] = qrow[qt] < Sq ? l * kLog2e : INFINITY;
+        }
+        if (kmask) {
+            // Chunk i's 32 keys start at bit rel % 64 of staged word rel / 64 (rel = key
+            // offset in the range, a multiple of 32); the lane's 8 keys are bits 8g .. 8g+7
+            // of that. The word's address is the same in every lane (an LDS broadcast).
+            const unsigned long long* wd = reinterpret_cast<const unsigned long long*>(ex + 256);
 #pragma unroll
-                for (int i = 0; i < KCW; ++i) {
-                    const int rel = 32 * (i * KQ + kq);
-                    const unsigned w32 = (unsigned)(wd[rel >> 6] >> (rel & 32));
-                    vbits |= ((w32 >> (8 * g)) & 0xffu) << (8 * i);
-                }
-            } else {
-                vbits = 0xffffffu;
+            for (int i = 0; i < KCW; ++i) {
+                const int rel = 32 * (i * KQ + kq);
+                const unsigned w32 = (unsigned)(wd[rel >> 6] >> (rel & 32));
+                vbits |= ((w32 >> (8 * g)) & 0xffu) << (8 * i);
             }
         } else {
-#pragma unroll
-            for (int qt = 0; qt < QTW; ++qt)
-                lse2c[qt] = qrow[qt] < Sq ? lse_nx[qt] * kLog2e : INFINITY;
-#pragma unroll
-            for (int i = 0; i < KCW; ++i) vbits |= nonzero_bits8(mask_nx[i]) << (8 * i);
+            vbits = 0xffffffu;
         }
 
         V8 qf[QTW], dof[QTW];
@@ -949,7 +898,7 @@ __global__ __launch_bounds__(256 * QG) void attn_bwd_dq2(
         }
         if (kmask) {
             // Also each row's presence bits, 64 keys per word (bit j of word i: key 64i + j is
-            // present), read by the row steps in place of the mask bytes (VEC); and, lane w
+            // present), read by the row steps in place of the mask bytes; and, lane w
             // holding word kbeg/64 + w of the key range, their OR and AND over this wave's rows.
             const int words = (Sk + 63) >> 6;
             unsigned long long seen = 0ull, always = ~0ull;
@@ -957,71 +906,62 @@ __global__ __launch_bounds__(256 * QG) void attn_bwd_dq2(
             for (int nr = n0 + wave; nr < n1; nr += NWV) {
                 const uint8_t* m = kmask + (size_t)nr * Sk;
                 bool any = false;
-                if constexpr (VEC) {
-                    unsigned long long mine = 0ull;  // this lane's word of the row
-                    for (int i = 0; i < words; ++i) {
-                        const int kk = 64 * i + lane;
-                        const unsigned long long b = __ballot(kk < Sk && m[kk] != 0);
-                        any |= b != 0ull;
-                        if (lane == 0) mbits[(size_t)nr * words + i] = b;
-                        if (lane == i - (kbeg >> 6)) mine = b;
-                    }
-                    if (any) {  // rows with a present key only
-                        seen |= mine;
-                        always &= mine;
-                    }
-                } else {
-                    for (int i = lane; i < Sk; i += 64) any |= m[i] != 0;
-                    any = __any(any);
+                unsigned long long mine = 0ull;  // this lane's word of the row
+                for (int i = 0; i < words; ++i) {
+                    const int kk = 64 * i + lane;
+                    const unsigned long long b = __ballot(kk < Sk && m[kk] != 0);
+                    any |= b != 0ull;
+                    if (lane == 0) mbits[(size_t)nr * words + i] = b;
+                    if (lane == i - (kbeg >> 6)) mine = b;
+                }
+                if (any) {  // rows with a present key only
+                    seen |= mine;
+                    always &= mine;
                 }
                 empty_row |= !any;
                 if (lane == 0) row_logit[nr] = any ? kMaskedLogit : 0.f;
             }
-            if constexpr (VEC) {
-                // The waves' words combined through the second Q/dO/O buffer (idle until the
-                // first row step stages row n0 + 1): the keys present in no row of the block
-                // (their bias becomes -inf), whether every key of the range is present in all
-                // rows that have a present key or in none of them, and whether a row has none.
-                constexpr int NWD = RK / 64;
-                unsigned long long* orw = reinterpret_cast<unsigned long long*>(qd1);
-                unsigned long long* andw = orw + NWV * NWD;
-                int* emptyw = reinterpret_cast<int*>(andw + NWV * NWD);
-                static_assert(sizeof(qd1) >= 2 * NWV * NWD * 8 + NWV * 4, "presence words fit");
-                if (lane < NWD) {
-                    orw[wave * NWD + lane] = seen;
-                    andw[wave * NWD + lane] = always;
-                }
-                if (lane == 0) emptyw[wave] = empty_row ? 1 : 0;
-                __syncthreads();
-#pragma unroll
-                for (int i = 0; i < KCW; ++i) {
-                    const int rel = 32 * (i * KQ + kq);
-                    unsigned long long w = 0ull;
-#pragma unroll
-                    for (int ww = 0; ww < NWV; ++ww) w |= orw[ww * NWD + (rel >> 6)];
-                    const unsigned bits = (unsigned)(w >> ((rel & 32) + 8 * g)) & 0xffu;
-                    cabs |= (~bits & 0xffu) << (8 * i);
-                }
-                bool mixed = false;
-                if (lane < NWD) {
-                    unsigned long long o = 0ull, a = ~0ull;
-#pragma unroll
-                    for (int ww = 0; ww < NWV; ++ww) {
-                        o |= orw[ww * NWD + lane];
-                        a &= andw[ww * NWD + lane];
-                    }
-                    const int lim = kend - (kbeg + 64 * lane);  // keys of the word in range
-                    const unsigned long long inr = lim >= 64 ? ~0ull : lim <= 0 ? 0ull
-                                                                      : (1ull << lim) - 1ull;
-                    mixed = ((o ^ a) & inr) != 0ull;
-                }
-                bool empty = false;
-#pragma unroll
-                for (int ww = 0; ww < NWV; ++ww) empty |= emptyw[ww] != 0;
-                block_rows = __any(mixed) ? kRowsMixed : empty ? kRowsEmpty : kRowsClean;
-            } else {
-                block_rows = kRowsMixed;
+            // The waves' words combined through the second Q/dO/O buffer (idle until the
+            // first row step stages row n0 + 1): the keys present in no row of the block
+            // (their bias becomes -inf), whether every key of the range is present in all
+            // rows that have a present key or in none of them, and whether a row has none.
+            constexpr int NWD = RK / 64;
+            unsigned long long* orw = reinterpret_cast<unsigned long long*>(qd1);
+            unsigned long long* andw = orw + NWV * NWD;
+            int* emptyw = reinterpret_cast<int*>(andw + NWV * NWD);
+            static_assert(sizeof(qd1) >= 2 * NWV * NWD * 8 + NWV * 4, "presence words fit");
+            if (lane < NWD) {
+                orw[wave * NWD + lane] = seen;
+                andw[wave * NWD + lane] = always;
             }
+            if (lane == 0) emptyw[wave] = empty_row ? 1 : 0;
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < KCW; ++i) {
+                const int rel = 32 * (i * KQ + kq);
+                unsigned long long w = 0ull;
+#pragma unroll
+                for (int ww = 0; ww < NWV; ++ww) w |= orw[ww * NWD + (rel >> 6)];
+                const unsigned bits = (unsigned)(w >> ((rel & 32) + 8 * g)) & 0xffu;
+                cabs |= (~bits & 0xffu) << (8 * i);
+            }
+            bool mixed = false;
+            if (lane < NWD) {
+                unsigned long long o = 0ull, a = ~0ull;
+#pragma unroll
+                for (int ww = 0; ww < NWV; ++ww) {
+                    o |= orw[ww * NWD + lane];
+                    a &= andw[ww * NWD + lane];
+                }
+                const int lim = kend - (kbeg + 64 * lane);  // keys of the word in range
+                const unsigned long long inr = lim >= 64 ? ~0ull : lim <= 0 ? 0ull
+                                                                  : (1ull << lim) - 1ull;
+                mixed = ((o ^ a) & inr) != 0ull;
+            }
+            bool empty = false;
+#pragma unroll
+            for (int ww = 0; ww < NWV; ++ww) empty |= emptyw[ww] != 0;
+            block_rows = __any(mixed) ? kRowsMixed : empty ? kRowsEmpty : kRowsClean;
             __syncthreads();  // this block's prefetches read them; the combined words are read
         }
     }
@@ -1072,9 +1012,7 @@ __global__ __launch_bounds__(256 * QG) void attn_bwd_dq2(
                     // kk % 4 == Sk % 4 == 0, so kk < Sk means kk + 4 <= Sk
                     if (kk < Sk) *reinterpret_cast<f32x4*>(drow + kk) = dbias[i][qt][t];
                 } else {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (kk + j < Sk) drow[kk + j] = dbias[i][qt][t][j];
+                    store4_below(drow, kk, Sk, dbias[i][qt][t]);
                 }
             }
         }
@@ -1110,7 +1048,7 @@ __device__ __forceinline__ void sum_slices(const f32x4* __restrict__ part, size_
 // global->LDS loads into the other buffer while the current tile is computed (one barrier per
 // tile). Per 32-query chunk: S = Q.K^T and dP - D = dO.V^T with the queries permuted so that P
 // and dS are directly the B operands of dV^T += dO^T.P and dK^T += Q^T.dS.
-template <typename TR, int D, int KSUB, int NW, bool VEC, bool NSHD>
+template <typename TR, int D, int KSUB, int NW, bool NSHD>
 __global__ __launch_bounds__(64 * NW) void attn_bwd_dkv2(
     const typename TR::elem* __restrict__ q, const typename TR::elem* __restrict__ k,
     const typename TR::elem* __restrict__ v, const typename TR::elem* __restrict__ bias_t,
@@ -1516,7 +1454,7 @@ void run_bwd_v1(hipStream_t st, const BwdPlan& p, const void* q, const void* k, 
         KernelTimer timer("attn_bwd_dkv", st);
         attn_bwd_dkv<TR, D, NSHD><<<grid, 256, 0, st>>>((const E*)q, (const E*)k, (const E*)v,
                                                   (const E*)bias, kmask, (const E*)dout, lse, di,
-                                                  (E*)dk, (E*)dv, H, Sq, Sk, scale, vec_ok);
+                                                  (E*)dk, (E*)dv, H, Sq, Sk, scale);
     }
     finish_partials<TR>(st, p, dbias_part, dq_part, dbias, dq, (size_t)H * Sq * Sk,
                         (size_t)rows * D);
@@ -1539,7 +1477,7 @@ void launch_dq2(hipStream_t st, const BwdPlan& p, const void* q, const void* k, 
         ceil_div(Sk, 64));
 }
 
-template <typename TR, int D, int KSUB, int NW, bool VEC, bool NSHD>
+template <typename TR, int D, int KSUB, int NW, bool NSHD>
 void launch_dkv2(hipStream_t st, const BwdPlan& p, const void* q, const void* k, const void* v,
                  const void* bias_t, const uint8_t* kmask, const void* dout, const float* lse2,
                  const float* ndi, const float* rowl, void* dk, void* dv, const float* dbias_part,
@@ -1552,14 +1490,14 @@ void launch_dkv2(hipStream_t st, const BwdPlan& p, const void* q, const void* k,
     const int extra =
         dbias_folded(p, count) ? (int)std::min<size_t>((vecs + per_block - 1) / per_block, 2048) : 0;
     KernelTimer timer("attn_bwd_dkv", st);
-    attn_bwd_dkv2<TR, D, KSUB, NW, VEC, NSHD><<<dim3(main_blocks + extra), 64 * NW, 0, st>>>(
+    attn_bwd_dkv2<TR, D, KSUB, NW, NSHD><<<dim3(main_blocks + extra), 64 * NW, 0, st>>>(
         (const E*)q, (const E*)k, (const E*)v, (const E*)bias_t, kmask, (const E*)dout, lse2,
         ndi, rowl, (E*)dk, (E*)dv, H, Sq, Sk, p.SqP, scale, main_blocks,
         reinterpret_cast<const f32x4*>(dbias_part), reinterpret_cast<f32x4*>(dbias), vecs,
         p.nchunks);
 }
 
-template <typename TR, int D, bool VEC, bool NSHD>
+template <typename TR, int D, bool NSHD>
 void run_bwd_v2(hipStream_t st, const BwdPlan& p, const void* q, const void* k, const void* v,
                 const void* bias, const uint8_t* kmask, const void* out, const void* dout,
                 const float* lse, void* dq, void* dk, void* dv, float* dbias, char* ws, int N,
@@ -1576,9 +1514,14 @@ void run_bwd_v2(hipStream_t st, const BwdPlan& p, const void* q, const void* k, 
     switch (p.KCW) {
 #define CLK_KCW(V)                                                                               \
     case V:                                                                                      \
-        launch_dq2<TR, D, V, VEC, NSHD>(st, p, q, k, v, bias, kmask, out, dout, lse, rowl,       \
-                                        mbits, lse2, ndi, dq, dq_part, dbias_dst, bias_t, N, H,  \
-                                        Sq, Sk, scale);                                          \
+        if (Sk % 8 == 0)                                                                         \
+            launch_dq2<TR, D, V, true, NSHD>(st, p, q, k, v, bias, kmask, out, dout, lse, rowl,  \
+                                             mbits, lse2, ndi, dq, dq_part, dbias_dst, bias_t,   \
+                                             N, H, Sq, Sk, scale);                               \
+        else                                                                                     \
+            launch_dq2<TR, D, V, false, NSHD>(st, p, q, k, v, bias, kmask, out, dout, lse, rowl, \
+                                              mbits, lse2, ndi, dq, dq_part, dbias_dst, bias_t,  \
+                                              N, H, Sq, Sk, scale);                              \
         break;
         CLK_KCW(1) CLK_KCW(2) CLK_KCW(3)
 #undef CLK_KCW
@@ -1586,7 +1529,7 @@ void run_bwd_v2(hipStream_t st, const BwdPlan& p, const void* q, const void* k, 
     switch (p.KSUB * 100 + p.KNW) {
 #define CLK_KSUB(V, W)                                                                           \
     case V * 100 + W:                                                                            \
-        launch_dkv2<TR, D, V, W, VEC, NSHD>(st, p, q, k, v, bias_t, kmask, dout, lse2, ndi,      \
+        launch_dkv2<TR, D, V, W, NSHD>(st, p, q, k, v, bias_t, kmask, dout, lse2, ndi,      \
                                             rowl, dk, dv, dbias_part, dbias, N, H, Sq, Sk,       \
                                             scale);                                              \
         break;
@@ -1603,13 +1546,8 @@ void run_bwd(hipStream_t st, const BwdPlan& p, const void* q, const void* k, con
              const float* lse, void* dq, void* dk, void* dv, float* dbias, char* ws, int N,
              int H, int Sq, int Sk, float scale) {
     if constexpr (D <= 32) {
-        const bool vec = Sk % 8 == 0 && (reinterpret_cast<uintptr_t>(kmask) & 7u) == 0;
-        if (vec)
-            run_bwd_v2<TR, D, true, NSHD>(st, p, q, k, v, bias, kmask, out, dout, lse, dq, dk, dv,
-                                          dbias, ws, N, H, Sq, Sk, scale);
-        else
-            run_bwd_v2<TR, D, false, NSHD>(st, p, q, k, v, bias, kmask, out, dout, lse, dq, dk,
-                                           dv, dbias, ws, N, H, Sq, Sk, scale);
+        run_bwd_v2<TR, D, NSHD>(st, p, q, k, v, bias, kmask, out, dout, lse, dq, dk, dv, dbias,
+                                ws, N, H, Sq, Sk, scale);
     } else {
         run_bwd_v1<TR, D, NSHD>(st, p, q, k, v, bias, kmask, out, dout, lse, dq, dk, dv, dbias,
                                 ws, N, H, Sq, Sk, scale);

@@ -25,13 +25,6 @@ struct AttnGeom {
 // Row of the 16-row operand tile t (0..3) of a 64-row tile that lane row r16 supplies. Inside
 // each 32-row chunk c = t/2 the rows are permuted so that the C tile of the product holds rows
 // 32c + 8*(l/16) + 0..7 in lane l: half t%2 covers +0..3, the other +4..7.
-// True when some byte of the eight is zero (an absent key).
-__device__ __forceinline__ bool has_zero_byte(u32x2 w) {
-    const unsigned a = (w[0] - 0x01010101u) & ~w[0] & 0x80808080u;
-    const unsigned b = (w[1] - 0x01010101u) & ~w[1] & 0x80808080u;
-    return (a | b) != 0u;
-}
-
 __device__ __forceinline__ int perm_key(int t, int r16) {
     return 32 * (t >> 1) + 8 * (r16 >> 2) + 4 * (t & 1) + (r16 & 3);
 }
@@ -118,20 +111,33 @@ __device__ __forceinline__ void zero_v_padding(E* lds) {
     }
 }
 
+// 16-byte load of eight 2-byte elements, and store of four floats, at any element alignment.
+typedef unsigned int u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ u32x4 ld16_a2(const void* p) {
+    return *reinterpret_cast<const u32x4_a2*>(p);
+}
+
 // Eight bias values bias_row[kk .. kk+7] as float (zero past Sk).
 template <typename TR>
 __device__ __forceinline__ void load_bias8(const typename TR::elem* row, int kk, int Sk,
-                                           int vec_ok, float* out) {
-    using E = typename TR::elem;
-    if (vec_ok && kk + 8 <= Sk) {
-        E e[8];
-        u32x4 raw = ld16(row + kk);
-        __builtin_memcpy(e, &raw, 16);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) out[j] = TR::to_f(e[j]);
+                                           float* out) {
+    if (kk + 8 <= Sk) {
+        unpack8<TR>(ld16_a2(row + kk), out);
     } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j) out[j] = (kk + j < Sk) ? TR::to_f(row[kk + j]) : 0.f;
+    }
+}
+
+// row[kk .. kk+3] = v, the entries below S only.
+__device__ __forceinline__ void store4_below(float* row, int kk, int S, f32x4 v) {
+    if (kk + 4 <= S) {
+        *reinterpret_cast<f32x4_a4*>(row + kk) = v;
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (kk + j < S) row[kk + j] = v[j];
     }
 }
 

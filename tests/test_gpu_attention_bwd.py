@@ -238,3 +238,33 @@ def test_attention_autograd_function(cuda):
     assert_close("q.grad", q.grad, rq, tol)
     assert_close("bias.grad", b.grad.float(), rb, tol)
     _ = np
+
+
+# (N, H, Sq, Sk, D): key counts that are no multiple of 8, around the edges of the 32-key chunks,
+# the 128-key groups and the 384-key ranges; odd query counts around the 64-query blocks.
+RAGGED_SHAPES = [(9, 2, 1, 1, 32), (9, 2, 3, 2, 16), (9, 2, 63, 31, 32), (9, 2, 65, 33, 8),
+                 (9, 3, 64, 127, 32), (9, 3, 127, 129, 32), (9, 2, 129, 255, 32),
+                 (9, 2, 66, 382, 32), (9, 2, 67, 385, 32), (9, 1, 65, 389, 16), (9, 2, 65, 66, 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=dname)
+@pytest.mark.parametrize("shape", RAGGED_SHAPES, ids=lambda c: "x".join(map(str, c)))
+def test_attention_bwd_ragged_keys(cuda, shape, dtype):
+    """Ragged key counts with per-row masks (all present, none, key 0 absent, only the last key
+    present, random holes) and without a mask, against the oracle."""
+    n, h, sq, sk, d = shape
+    inp = attention_inputs(n, h, sq, sk, d, dtype, seed=3 * sk + sq)
+    g = torch.Generator().manual_seed(sk + 5 * sq)
+    km = torch.ones((n, sk), dtype=torch.uint8)
+    km[1] = 0
+    km[2, 0] = 0
+    km[2, sk - 1] = 1
+    km[3, :sk - 1] = 0
+    km[4] = (torch.rand(sk, generator=g) > 0.3).to(torch.uint8)
+    km[4, sk // 2] = 1
+    tol = TOL[dname(dtype)]["grad"]
+    for mask in (km, torch.ones_like(km)):
+        inp["kmask"] = mask
+        _, _, _, grads = _run(inp, cuda)
+        for name, got, r in zip(("dQ", "dK", "dV", "dBias"), grads, _oracle(inp)):
+            assert_close(name, got, r, tol)
