@@ -22,10 +22,19 @@
 namespace clk {
 namespace {
 
-constexpr int kTriTile = 256;  // output tile edge
-constexpr int kTriK = 32;      // contraction depth of one half slice (two per stage)
+constexpr int kTriK = 32;  // contraction depth of one half slice (two per stage)
 
-// The twelve 16-byte fragments of one half slice (four B rows, eight A rows, 16-row blocks STRIDE
+// Output tile edge BT: 256 as above, or 128 with four waves of 64 x 64 (16 accumulators) and 64 KB
+// of LDS, two blocks per CU.
+template <int BT>
+struct TriShape {
+    static_assert(BT == 128 || BT == 256, "tile edge");
+    static constexpr int WJ = BT / 64;           // waves along j (64 columns each)
+    static constexpr int IT = BT == 256 ? 8 : 4;  // 16-row A fragments of a wave
+    static constexpr int NT = 64 * WJ * (BT / (16 * IT));
+};
+
+// The IT + 4 16-byte fragments of one half slice (four B rows, IT A rows, 16-row blocks STRIDE
 // bytes apart) read from LDS and waited for in one asm statement: the loop picks its stage at
 // run time, and a read the compiler can see would have to wait for every direct-to-LDS load in
 // flight. All outputs are complete when the statement ends, so no register is read before its
@@ -54,50 +63,90 @@ __device__ __forceinline__ void read_fragments_s(uint32_t ba, uint32_t bb, V8 (&
           "i"(5 * STRIDE), "i"(6 * STRIDE), "i"(7 * STRIDE)
         : "memory");
 }
+template <int STRIDE, typename V8>
+__device__ __forceinline__ void read_fragments_s(uint32_t ba, uint32_t bb, V8 (&fb)[4],
+                                                 V8 (&fa)[4]) {
+    asm volatile(
+        "ds_read_b128 %0, %9\n\t"
+        "ds_read_b128 %1, %9 offset:%10\n\t"
+        "ds_read_b128 %2, %9 offset:%11\n\t"
+        "ds_read_b128 %3, %9 offset:%12\n\t"
+        "ds_read_b128 %4, %8\n\t"
+        "ds_read_b128 %5, %8 offset:%10\n\t"
+        "ds_read_b128 %6, %8 offset:%11\n\t"
+        "ds_read_b128 %7, %8 offset:%12\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(fb[0]), "=&v"(fb[1]), "=&v"(fb[2]), "=&v"(fb[3]), "=&v"(fa[0]), "=&v"(fa[1]),
+          "=&v"(fa[2]), "=&v"(fa[3])
+        : "v"(ba), "v"(bb), "i"(STRIDE), "i"(2 * STRIDE), "i"(3 * STRIDE)
+        : "memory");
+}
 
-// The 24 transposed fragment reads of one TN slice (A: 8 fragments, B: 4, each two
-// ds_read_b64_tr_b16 of rows 8g+j and 8g+4+j, 2 KB apart) and their wait, as one asm statement.
+// The transposed fragment reads of one TN half slice (A: IT fragments, then B: 4, each two
+// ds_read_b64_tr_b16 of rows 8g+j and 8g+4+j, OFF bytes apart) and their wait, as one asm
+// statement.
+template <int OFF>
 __device__ __forceinline__ void read_tr_fragments(const uint32_t (&ad)[12], i16x4 (&r)[24]) {
     asm volatile(
-        "ds_read_b64_tr_b16 %0, %24\n\tds_read_b64_tr_b16 %1, %24 offset:2048\n\t"
-        "ds_read_b64_tr_b16 %2, %25\n\tds_read_b64_tr_b16 %3, %25 offset:2048\n\t"
-        "ds_read_b64_tr_b16 %4, %26\n\tds_read_b64_tr_b16 %5, %26 offset:2048\n\t"
-        "ds_read_b64_tr_b16 %6, %27\n\tds_read_b64_tr_b16 %7, %27 offset:2048\n\t"
-        "ds_read_b64_tr_b16 %8, %28\n\tds_read_b64_tr_b16 %9, %28 offset:2048\n\t"
-        "ds_read_b64_tr_b16 %10, %29\n\tds_read_b64_tr_b16 %11, %29 offset:2048\n\t"
-        "ds_read_b64_tr_b16 %12, %30\n\tds_read_b64_tr_b16 %13, %30 offset:2048\n\t"
-        "ds_read_b64_tr_b16 %14, %31\n\tds_read_b64_tr_b16 %15, %31 offset:2048\n\t"
-        "ds_read_b64_tr_b16 %16, %32\n\tds_read_b64_tr_b16 %17, %32 offset:2048\n\t"
-        "ds_read_b64_tr_b16 %18, %33\n\tds_read_b64_tr_b16 %19, %33 offset:2048\n\t"
-        "ds_read_b64_tr_b16 %20, %34\n\tds_read_b64_tr_b16 %21, %34 offset:2048\n\t"
-        "ds_read_b64_tr_b16 %22, %35\n\tds_read_b64_tr_b16 %23, %35 offset:2048\n\t"
+        "ds_read_b64_tr_b16 %0, %24\n\tds_read_b64_tr_b16 %1, %24 offset:%36\n\t"
+        "ds_read_b64_tr_b16 %2, %25\n\tds_read_b64_tr_b16 %3, %25 offset:%36\n\t"
+        "ds_read_b64_tr_b16 %4, %26\n\tds_read_b64_tr_b16 %5, %26 offset:%36\n\t"
+        "ds_read_b64_tr_b16 %6, %27\n\tds_read_b64_tr_b16 %7, %27 offset:%36\n\t"
+        "ds_read_b64_tr_b16 %8, %28\n\tds_read_b64_tr_b16 %9, %28 offset:%36\n\t"
+        "ds_read_b64_tr_b16 %10, %29\n\tds_read_b64_tr_b16 %11, %29 offset:%36\n\t"
+        "ds_read_b64_tr_b16 %12, %30\n\tds_read_b64_tr_b16 %13, %30 offset:%36\n\t"
+        "ds_read_b64_tr_b16 %14, %31\n\tds_read_b64_tr_b16 %15, %31 offset:%36\n\t"
+        "ds_read_b64_tr_b16 %16, %32\n\tds_read_b64_tr_b16 %17, %32 offset:%36\n\t"
+        "ds_read_b64_tr_b16 %18, %33\n\tds_read_b64_tr_b16 %19, %33 offset:%36\n\t"
+        "ds_read_b64_tr_b16 %20, %34\n\tds_read_b64_tr_b16 %21, %34 offset:%36\n\t"
+        "ds_read_b64_tr_b16 %22, %35\n\tds_read_b64_tr_b16 %23, %35 offset:%36\n\t"
         "s_waitcnt lgkmcnt(0)"
         : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]),
           "=&v"(r[6]), "=&v"(r[7]), "=&v"(r[8]), "=&v"(r[9]), "=&v"(r[10]), "=&v"(r[11]),
           "=&v"(r[12]), "=&v"(r[13]), "=&v"(r[14]), "=&v"(r[15]), "=&v"(r[16]), "=&v"(r[17]),
           "=&v"(r[18]), "=&v"(r[19]), "=&v"(r[20]), "=&v"(r[21]), "=&v"(r[22]), "=&v"(r[23])
         : "v"(ad[0]), "v"(ad[1]), "v"(ad[2]), "v"(ad[3]), "v"(ad[4]), "v"(ad[5]), "v"(ad[6]),
-          "v"(ad[7]), "v"(ad[8]), "v"(ad[9]), "v"(ad[10]), "v"(ad[11])
+          "v"(ad[7]), "v"(ad[8]), "v"(ad[9]), "v"(ad[10]), "v"(ad[11]), "i"(OFF)
+        : "memory");
+}
+template <int OFF>
+__device__ __forceinline__ void read_tr_fragments(const uint32_t (&ad)[8], i16x4 (&r)[16]) {
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %16\n\tds_read_b64_tr_b16 %1, %16 offset:%24\n\t"
+        "ds_read_b64_tr_b16 %2, %17\n\tds_read_b64_tr_b16 %3, %17 offset:%24\n\t"
+        "ds_read_b64_tr_b16 %4, %18\n\tds_read_b64_tr_b16 %5, %18 offset:%24\n\t"
+        "ds_read_b64_tr_b16 %6, %19\n\tds_read_b64_tr_b16 %7, %19 offset:%24\n\t"
+        "ds_read_b64_tr_b16 %8, %20\n\tds_read_b64_tr_b16 %9, %20 offset:%24\n\t"
+        "ds_read_b64_tr_b16 %10, %21\n\tds_read_b64_tr_b16 %11, %21 offset:%24\n\t"
+        "ds_read_b64_tr_b16 %12, %22\n\tds_read_b64_tr_b16 %13, %22 offset:%24\n\t"
+        "ds_read_b64_tr_b16 %14, %23\n\tds_read_b64_tr_b16 %15, %23 offset:%24\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]),
+          "=&v"(r[6]), "=&v"(r[7]), "=&v"(r[8]), "=&v"(r[9]), "=&v"(r[10]), "=&v"(r[11]),
+          "=&v"(r[12]), "=&v"(r[13]), "=&v"(r[14]), "=&v"(r[15])
+        : "v"(ad[0]), "v"(ad[1]), "v"(ad[2]), "v"(ad[3]), "v"(ad[4]), "v"(ad[5]), "v"(ad[6]),
+          "v"(ad[7]), "i"(OFF)
         : "memory");
 }
 
 // TN = false: X[c] = A[c] . B[c]^T for A, B, X [C][N][N] row-major (the contraction index
 // last). TN = true: X[c] = A[c]^T . B[c] (the contraction index first, A[c][k][i], B[c][k][j]):
-// a slice is 32 rows k of A (B) x the tile's 256 columns i (j), and the fragments are read
+// a slice is 64 rows k of A (B) x the tile's BT columns i (j), and the fragments are read
 // transposed with ds_read_b64_tr_b16, so the incoming direction needs no plane transposes.
 // N must be a multiple of 8.
-template <typename TR, bool TN>
-__global__ __launch_bounds__(512) void tri_einsum_kernel(const typename TR::elem* __restrict__ A,
+template <typename TR, bool TN, int BT>
+__global__ __launch_bounds__(TriShape<BT>::NT) void tri_einsum_kernel(const typename TR::elem* __restrict__ A,
                                                          const typename TR::elem* __restrict__ B,
                                                          typename TR::elem* __restrict__ X, int N,
                                                          int T, int ntiles) {
     using E = typename TR::elem;
     using V8 = typename TR::vec8;
-    constexpr int BT = kTriTile, KC = 2 * kTriK;
+    using SH = TriShape<BT>;
+    constexpr int KC = 2 * kTriK, IT = SH::IT;
     constexpr int NSTG = 2;  // two stages of 64 k
     constexpr int PR = KC / 8;             // 16-byte pieces per row slice
     constexpr int SLICE = BT * PR * 16;    // bytes of one operand slice
-    constexpr int NT = 512, DPW = 2 * BT * PR / NT;  // loads per lane and slice (A and B)
+    constexpr int NT = SH::NT, DPW = 2 * BT * PR / NT;  // loads per lane and slice (A and B)
     static_assert(BT * PR % NT == 0, "whole load rounds");
 
     constexpr int STAGE = 2 * SLICE;
@@ -106,7 +155,8 @@ __global__ __launch_bounds__(512) void tri_einsum_kernel(const typename TR::elem
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
-    const int wi = wave >> 2, wj = wave & 3;  // wave tile: rows 128*wi.., columns 64*wj..
+    // Wave tile: rows 16*IT*wi.., columns 64*wj..
+    const int wi = wave / SH::WJ, wj = wave % SH::WJ;
 
     const int w = xcd_contiguous(blockIdx.x, ntiles);
     const int c = w / (T * T), ti = (w / T) % T, tj = w % T;
@@ -126,7 +176,7 @@ __global__ __launch_bounds__(512) void tri_einsum_kernel(const typename TR::elem
 
     // Slice kk of both operands into buffer st: A rows at st, B rows at st + SLICE. Piece q of
     // LDS row r holds the row's 16-byte piece q ^ (r % 8); pieces past N read zeros.
-    // TN: LDS row r (k = kk*64 + r) holds the tile's 256 columns as 32 pieces; slot q holds
+    // TN: LDS row r (k = kk*64 + r) holds the tile's BT columns as BT/8 pieces; slot q holds
     // piece q ^ 2*(r % 4), so that the four rows of a transposed read fall in distinct banks.
     auto stage = [&](int kk, char* st) {
         const bool live = kk < nk;
@@ -150,11 +200,11 @@ __global__ __launch_bounds__(512) void tri_einsum_kernel(const typename TR::elem
         }
     };
 
-    f32x4 acc[4][8];
+    f32x4 acc[4][IT];
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
-        for (int b = 0; b < 8; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < IT; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // Operand reads (NT). Lane (r16, g) reads k 32h + 8g .. +7 (piece 4h + g) of row 16t + r16 of
     // its wave's rows; the swizzle term row % 8 is the same for every t, so one address per half
@@ -164,19 +214,19 @@ __global__ __launch_bounds__(512) void tri_einsum_kernel(const typename TR::elem
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const uint32_t rd = (uint32_t)(r16 * PR + ((4 * h + g) ^ (r16 & 7))) * 16;
-        rda2[h] = rd + 128 * wi * PR * 16;
+        rda2[h] = rd + 16 * IT * wi * PR * 16;
         rdb2[h] = rd + SLICE + 64 * wj * PR * 16;
     }
-    // TN: fragment f (it = 0..7 of A, then jt = 0..3 of B) is column block m0 = 128wi + 16it
+    // TN: fragment f (it = 0..IT-1 of A, then jt = 0..3 of B) is column block m0 = 16(IT*wi + it)
     // (64wj + 16jt); lane 4j + t reads row 8g + j (and + 4), columns m0 + 4t .. + 3.
-    uint32_t trd[12];
+    uint32_t trd[IT + 4];
     if constexpr (TN) {
         const int j = r16 >> 2, t = r16 & 3, row = 8 * g + j;
 #pragma unroll
-        for (int f = 0; f < 12; ++f) {
-            const int m0 = f < 8 ? 128 * wi + 16 * f : 64 * wj + 16 * (f - 8);
+        for (int f = 0; f < IT + 4; ++f) {
+            const int m0 = f < IT ? 16 * (IT * wi + f) : 64 * wj + 16 * (f - IT);
             const int piece = ((m0 + 4 * t) >> 3) ^ (2 * j);
-            trd[f] = (f < 8 ? 0 : SLICE) + row * (BT * 2) + piece * 16 + 8 * (t & 1);
+            trd[f] = (f < IT ? 0 : SLICE) + row * (BT * 2) + piece * 16 + 8 * (t & 1);
         }
     }
 
@@ -194,63 +244,66 @@ __global__ __launch_bounds__(512) void tri_einsum_kernel(const typename TR::elem
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            V8 fb[4], fa[8];
+            V8 fb[4], fa[IT];
             if constexpr (TN) {
                 // Rows 32h .. 32h+31 of the slice.
-                uint32_t ad[12];
+                uint32_t ad[IT + 4];
 #pragma unroll
-                for (int f = 0; f < 12; ++f) ad[f] = lds0 + cur * STAGE + trd[f] + h * 32 * BT * 2;
-                i16x4 r[24];
-                read_tr_fragments(ad, r);
+                for (int f = 0; f < IT + 4; ++f)
+                    ad[f] = lds0 + cur * STAGE + trd[f] + h * 32 * BT * 2;
+                i16x4 r[2 * (IT + 4)];
+                read_tr_fragments<4 * BT * 2>(ad, r);
 #pragma unroll
-                for (int f = 0; f < 12; ++f) {
+                for (int f = 0; f < IT + 4; ++f) {
                     const i16x4 lo = r[2 * f], hi = r[2 * f + 1];
                     typedef short i16x8 __attribute__((ext_vector_type(8)));
                     const i16x8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-                    if (f < 8) fa[f] = __builtin_bit_cast(V8, v);
-                    else fb[f - 8] = __builtin_bit_cast(V8, v);
+                    if (f < IT) fa[f] = __builtin_bit_cast(V8, v);
+                    else fb[f - IT] = __builtin_bit_cast(V8, v);
                 }
             } else {
                 read_fragments_s<16 * PR * 16>(lds0 + cur * STAGE + rda2[h],
                                                lds0 + cur * STAGE + rdb2[h], fb, fa);
             }
 #pragma unroll
-            for (int it = 0; it < 8; ++it)
+            for (int it = 0; it < IT; ++it)
 #pragma unroll
                 for (int jt = 0; jt < 4; ++jt) acc[jt][it] = TR::mfma(fb[jt], fa[it], acc[jt][it]);
         }
     }
 
-    // Lane (r16, g) of accumulator (jt, it) holds X[i][j..j+3] for i = i0 + 128wi + 16it + r16,
-    // j = j0 + 64wj + 16jt + 4g. The tile goes out through LDS (the two stages, 128 KB, are free
-    // once every wave's last loads have landed and its last reads are done): bf16 rows of 512
-    // bytes, 16-byte pieces XOR-swizzled by row % 32, then stored by the whole block as rows of
+    // Lane (r16, g) of accumulator (jt, it) holds X[i][j..j+3] for i = i0 + 16(IT*wi + it)
+    // + r16, j = j0 + 64wj + 16jt + 4g. The tile goes out through LDS (the two stages are free once
+    // every wave's last loads have landed and its last reads are done): rows of BT elements, their
+    // BT/8 16-byte pieces XOR-swizzled by the row, then stored by the whole block as rows of
     // whole cache lines (an 8-byte store per lane and accumulator writes a quarter line).
     // Rows past N fall outside the resource; columns past N (whole pieces, N being a multiple
     // of 8) are skipped.
     static_assert(BT * BT * 2 <= NSTG * STAGE, "the output tile fits the stages");
+    constexpr int OP = BT / 8;  // pieces per output row
     async_wait();
     lds_barrier();
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt)
 #pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            const int il = 128 * wi + 16 * it + r16, piece = 8 * wj + 2 * jt + (g >> 1);
+        for (int it = 0; it < IT; ++it) {
+            const int il = 16 * (IT * wi + it) + r16, piece = 8 * wj + 2 * jt + (g >> 1);
             E e[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) e[q] = TR::from_f(acc[jt][it][q]);
             u32x2 v;
             __builtin_memcpy(&v, e, 8);
-            *reinterpret_cast<u32x2*>(smem + (il * 32 + (piece ^ (il & 31))) * 16 + 8 * (g & 1)) =
-                v;
+            *reinterpret_cast<u32x2*>(smem + (il * OP + (piece ^ (il & (OP - 1)))) * 16 +
+                                      8 * (g & 1)) = v;
         }
     lds_barrier();
     const Rsrc rx = buffer_rsrc(X + c * plane + (size_t)i0 * N,
                                 (uint32_t)((size_t)min(BT, N - i0) * N * 2));
 #pragma unroll
     for (int k = 0; k < BT * BT / 8 / NT; ++k) {
-        const int f = k * NT + tid, row = f >> 5, piece = f & 31;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(smem + (row * 32 + (piece ^ (row & 31))) * 16);
+        const int f = k * NT + tid, row = f / OP, piece = f % OP;
+        const u32x4 v =
+            *reinterpret_cast<const u32x4*>(smem + (row * OP + (piece ^ (row & (OP - 1)))) * 16);
         if (j0 + 8 * piece < N) buf_st16_nt(rx, (row * N + j0 + 8 * piece) * 2, 0, v);
     }
 }
@@ -500,15 +553,32 @@ __global__ __launch_bounds__(512) void tri_out_kernel(TriOutParams<typename TR::
     async_wait();  // no direct-to-LDS load may still be in flight when the workgroup ends
 }
 
-template <typename TR, bool TN = false>
-clk_status launch_einsum(hipStream_t st, const void* a, const void* b, void* x, int C, int N) {
+template <typename TR, bool TN, int BT>
+clk_status launch_einsum_tiles(hipStream_t st, const void* a, const void* b, void* x, int C,
+                               int N) {
     using E = typename TR::elem;
-    const int T = (N + kTriTile - 1) / kTriTile;
+    const int T = (N + BT - 1) / BT;
     const int ntiles = C * T * T;
     KernelTimer timer("tri_einsum", st);
-    tri_einsum_kernel<TR, TN><<<ntiles, 512, 0, st>>>((const E*)a, (const E*)b, (E*)x, N, T,
-                                                       ntiles);
+    tri_einsum_kernel<TR, TN, BT><<<ntiles, TriShape<BT>::NT, 0, st>>>(
+        (const E*)a, (const E*)b, (E*)x, N, T, ntiles);
     return check_launch("triangle_einsum");
+}
+
+// The tile edge, by rounds of resident blocks (one 256-tile or two 128-tile blocks per CU): a
+// round of 128-tiles takes 0.57 of one of 256-tiles (14.3 against 25 us at N = 512, C = 128, where
+// the larger tile's fewer loads per product win: 50 against 57 us). So 128 where it leaves less of
+// its tiles empty or fills more CUs (C = 128: N = 104 10.5 -> 7.7, 200 15.4 -> 12.4, 320 29 -> 27,
+// 640 115 -> 104 us; C = 64, N = 256 14.5 -> 10.3), except that whole 256-tiles on half the CUs or
+// more are no slower (N = 256, C = 128: 15.0 and 15.6).
+template <typename TR, bool TN = false>
+clk_status launch_einsum(hipStream_t st, const void* a, const void* b, void* x, int C, int N) {
+    const int64_t big = (int64_t)C * ceil_div(N, 256) * ceil_div(N, 256);
+    const int64_t small = (int64_t)C * ceil_div(N, 128) * ceil_div(N, 128);
+    const int64_t rounds256 = (big + 255) / 256, rounds128 = (small + 511) / 512;
+    if (57 * rounds128 < 100 * rounds256 && !(N % 256 == 0 && big >= 128) && small <= INT32_MAX)
+        return launch_einsum_tiles<TR, TN, 128>(st, a, b, x, C, N);
+    return launch_einsum_tiles<TR, TN, 256>(st, a, b, x, C, N);
 }
 
 // Positions of an [N, N] grid of U-units (u units per position) copied to or from an [NP, NP]
@@ -570,8 +640,7 @@ extern "C" clk_status clk_triangle_einsum(hipStream_t stream, clk_dtype dtype, c
     if (C < 0 || N < 0) return fail(CLK_INVALID_ARGUMENT, "%s: bad dims", who);
     if (N % 8) return fail(CLK_INVALID_ARGUMENT, "%s: N=%lld is not a multiple of 8", who,
                            (long long)N);
-    if (N > 16384 || C * ((N + kTriTile - 1) / kTriTile) * ((N + kTriTile - 1) / kTriTile) >
-                         INT32_MAX)
+    if (N > 16384 || C * ((N + 255) / 256) * ((N + 255) / 256) > INT32_MAX)
         return fail(CLK_INVALID_ARGUMENT, "%s: dims too large", who);
     if (C == 0 || N == 0) return ok();
     if (!a || !b || !x) return fail(CLK_INVALID_ARGUMENT, "%s: null operand pointer", who);

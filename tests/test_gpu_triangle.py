@@ -139,3 +139,20 @@ def test_triangle_multiply_large_grid_sampled(cuda, n, outgoing):
                                  [np64(b) for b in bs], tuple(map(np64, ln_c)), pos, outgoing)
     got = torch.stack([out[i, j] for i, j in pos])
     assert_close("out", got, r, 2e-2)
+
+
+# Contraction shapes on either side of the choice between 128- and 256-wide output tiles, at the
+# edges of both: (C, N, channels compared).
+TILE_SHAPES = [(3, 120, (0, 2)), (3, 128, (0, 2)), (2, 136, (0, 1)), (2, 256, (0, 1)),
+               (128, 256, (0, 127)), (128, 264, (5, 127)), (128, 392, (0, 127)), (64, 640, (63,))]
+
+
+@pytest.mark.parametrize("c,n,chs", TILE_SHAPES, ids=str)
+def test_einsum_tile_choice(cuda, c, n, chs):
+    g = torch.Generator().manual_seed(c + n)
+    a = torch.randn((c, n, n), generator=g).to(torch.bfloat16)
+    b = torch.randn((c, n, n), generator=g).to(torch.bfloat16)
+    x = ops.triangle_einsum(a.to(cuda), b.to(cuda))
+    for ch in chs:
+        assert_close("x[%d]" % ch, x[ch], ref.einsum(np64(a[ch:ch + 1]), np64(b[ch:ch + 1]))[0],
+                     TOL["bf16"]["o"])
