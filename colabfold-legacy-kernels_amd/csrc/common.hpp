@@ -293,6 +293,39 @@ __device__ __forceinline__ int xcd_contiguous(int L, int T) {
     return xcd * per + min(xcd, rem) + slot;
 }
 
+// The pair positions (i, j) of an n x n grid as the rows of a zero-padded np x np one, np = n
+// rounded up to 8 (the channel planes of the triangle multiplication hold whole 16-byte pieces):
+// kernels that walk padded positions in 64-row tiles address the caller's n x n rows directly.
+struct PairGrid {
+    int n, np;
+    float inv;  // 1 / np
+};
+// A tile's first padded position: its grid row i0 and column j0, and a resource over the caller's
+// rows (`width` 2-byte elements each) from (i0, 0) on; rows outside the n x n grid read zeros and
+// drop stores.
+struct PairTile {
+    int i0, j0;
+    Rsrc r;
+};
+__device__ __forceinline__ PairTile pair_tile(const PairGrid& g, const void* base, int pos,
+                                              int width) {
+    PairTile t;
+    t.i0 = pos / g.np;
+    t.j0 = pos - t.i0 * g.np;
+    const size_t row_bytes = (size_t)g.n * width * 2;
+    const size_t left = t.i0 < g.n ? (size_t)(g.n - t.i0) * row_bytes : 0;
+    t.r = buffer_rsrc(left ? (const char*)base + t.i0 * row_bytes : base,
+                      (uint32_t)(left < (size_t)kPastEnd - 16 ? left : (size_t)kPastEnd - 16));
+    return t;
+}
+// Row of the caller's grid, counted from (i0, 0), of the tile's position r; -1 for a padded one.
+__device__ __forceinline__ int pair_row(const PairGrid& g, const PairTile& t, int r) {
+    const int x = t.j0 + r;  // < np + 64: the product's rounding cannot reach the next integer
+    const int q = (int)(((float)x + 0.5f) * g.inv);
+    const int j = x - q * g.np;
+    return j < g.n && t.i0 + q < g.n ? q * g.n + j : -1;
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 

@@ -364,12 +364,15 @@ __device__ __forceinline__ void lds_rows(uint32_t addr, u32x4 (&r)[N]) {
 // LN = false, NB = 1: the plain gated dual projection of one branch (x = z as it is; the four
 // staging waves only move z into the swizzled tile, and gamma, beta are not read).
 // Block: NB*N/32 MFMA waves, then 4 LayerNorm (staging) waves.
-template <typename TR, int C, int N, bool CM, bool LN = true, int NB = 2>
+// RAG (CM): z and mask hold a grid.n x grid.n pair grid and the rows walked are the positions of
+// the zero-padded grid.np x grid.np one (M = np^2); padded positions read zeros, mask included.
+template <typename TR, int C, int N, bool CM, bool LN = true, int NB = 2, bool RAG = false>
 __global__ __launch_bounds__(64 * NB * N / 32 + 256) void ln_gdp_kernel(
     const typename TR::elem* __restrict__ z, const float* __restrict__ gamma,
     const float* __restrict__ beta, LnGdpWeights<typename TR::elem> wb,
     const typename TR::elem* __restrict__ mask, typename TR::elem* __restrict__ outa,
-    typename TR::elem* __restrict__ outb, int M, float eps) {
+    typename TR::elem* __restrict__ outb, int M, float eps, PairGrid grid) {
+    static_assert(!RAG || CM, "padded pair grids are for the channel-major outputs");
     using E = typename TR::elem;
     using V8 = typename TR::vec8;
     constexpr int NWM = NB * N / 32;     // MFMA waves
@@ -453,6 +456,18 @@ __global__ __launch_bounds__(64 * NB * N / 32 + 256) void ln_gdp_kernel(
     };
     auto stage = [&](int j, char* zb) {
         const int t = tile_of(j);
+        if constexpr (RAG) {
+            PairTile pt = pair_tile(grid, z, j < mine ? t * R : 0, C);
+            if (j >= mine) pt.r = buffer_rsrc(z, 0);
+#pragma unroll
+            for (int k = 0; k < DPW; ++k) {
+                const int b = lw * 64 + k * NTL;
+                const int row = pair_row(grid, pt, (b + lane) / PL);
+                buf_dma16(pt.r, row < 0 ? kPastEnd : (row * PL + (b + lane) % PL) * 16, 0,
+                          zb + b * 16);
+            }
+            return;
+        }
         const int rows = j < mine ? min(R, M - t * R) : 0;
         const Rsrc rz = buffer_rsrc(rows > 0 ? z + (size_t)t * R * C : z, (uint32_t)rows * C * 2);
 #pragma unroll
@@ -464,6 +479,15 @@ __global__ __launch_bounds__(64 * NB * N / 32 + 256) void ln_gdp_kernel(
     auto load_mask = [&](int j, uint32_t (&mv)[PASSES]) {
         const uint16_t* m16 = reinterpret_cast<const uint16_t*>(mask);
         const int t = tile_of(j);
+        if constexpr (RAG) {
+            const PairTile pt = pair_tile(grid, mask, j < mine ? t * R : 0, 1);
+#pragma unroll
+            for (int p = 0; p < PASSES; ++p) {
+                const int row = pair_row(grid, pt, p * RPP + lt / LPR);
+                mv[p] = row < 0 ? 0u : m16[(size_t)pt.i0 * grid.n + row];
+            }
+            return;
+        }
 #pragma unroll
         for (int p = 0; p < PASSES; ++p) {
             const int64_t r = (int64_t)t * R + p * RPP + lt / LPR;
@@ -748,7 +772,7 @@ clk_status launch_gdp_resident(hipStream_t st, const void* x, const void* wp, co
     const int grid = ntiles < 256 * per_cu ? ntiles : 256 * per_cu;
     KernelTimer timer("gdp", st);
     ln_gdp_kernel<TR, K, N, false, false, 1><<<grid, 2 * N + 256, 0, st>>>(
-        (const E*)x, nullptr, nullptr, wb, (const E*)mask, (E*)out, nullptr, M, 0.f);
+        (const E*)x, nullptr, nullptr, wb, (const E*)mask, (E*)out, nullptr, M, 0.f, PairGrid{});
     return check_launch("gated_dual_proj");
 }
 
@@ -788,10 +812,10 @@ clk_status dispatch_gdp(hipStream_t st, const void* x, const void* wp, const voi
     return launch_gdp<TR, 64, true>(st, x, wp, bp, wg, bg, mask, out, M, K, N);
 }
 
-template <typename TR, int C, int N, bool CM = false>
+template <typename TR, int C, int N, bool CM = false, bool RAG = false>
 clk_status launch_ln_gdp(hipStream_t st, const void* z, const float* gamma, const float* beta,
                          const LnGdpWeights<typename TR::elem>& wb, const void* mask, void* a,
-                         void* b, int M, float eps) {
+                         void* b, int M, float eps, PairGrid pg = {}) {
     using E = typename TR::elem;
     // One 12-wave block per CU at N = C = 128 (its five 16 KB LDS tiles take half the CU's LDS,
     // its registers three waves per SIMD); narrower N runs more, smaller blocks per CU.
@@ -799,8 +823,8 @@ clk_status launch_ln_gdp(hipStream_t st, const void* z, const float* gamma, cons
     const int per_cu = LnGdpPlan<C, N, 2>::PER_CU;
     const int grid = ntiles < 256 * per_cu ? ntiles : 256 * per_cu;
     KernelTimer timer("ln_gdp", st);
-    ln_gdp_kernel<TR, C, N, CM><<<grid, 4 * N + 256, 0, st>>>((const E*)z, gamma, beta, wb,
-                                                     (const E*)mask, (E*)a, (E*)b, M, eps);
+    ln_gdp_kernel<TR, C, N, CM, true, 2, RAG><<<grid, 4 * N + 256, 0, st>>>(
+        (const E*)z, gamma, beta, wb, (const E*)mask, (E*)a, (E*)b, M, eps, pg);
     return check_launch("ln_gated_dual_proj");
 }
 
@@ -827,12 +851,14 @@ clk_status dispatch_ln_gdp(hipStream_t st, const void* z, const float* gamma, co
 
 }  // namespace
 
-// LayerNorm + both gated branches with channel-major outputs a, b [N][M], for the triangle-
-// multiplication contraction. Arguments checked by the caller; M % 64 == 0.
+// LayerNorm + both gated branches of the pair grid z [n, n, C] with channel-major outputs a, b
+// [N][np * np], np = n rounded up to 8 and zeros in the padding, for the triangle-multiplication
+// contraction. Arguments checked by the caller.
 clk_status ln_gdp_channel_major(hipStream_t st, clk_dtype dtype, const void* z,
                                 const float* gamma, const float* beta, const void* const* w,
-                                const void* const* bias, const void* mask, void* a, void* b, int M,
-                                int C, int N, float eps) {
+                                const void* const* bias, const void* mask, void* a, void* b,
+                                PairGrid pg, int C, int N, float eps) {
+    const int M = pg.np * pg.np;
     auto run = [&](auto tr) -> clk_status {
         using TR = decltype(tr);
         using E = typename TR::elem;
@@ -841,10 +867,14 @@ clk_status ln_gdp_channel_major(hipStream_t st, clk_dtype dtype, const void* z,
             wb.w[i] = static_cast<const E*>(w[i]);
             wb.b[i] = static_cast<const E*>(bias[i]);
         }
-        if (C == 128 && N == 128)
-            return launch_ln_gdp<TR, 128, 128, true>(st, z, gamma, beta, wb, mask, a, b, M, eps);
-        if (C == 64 && N == 64)
-            return launch_ln_gdp<TR, 64, 64, true>(st, z, gamma, beta, wb, mask, a, b, M, eps);
+#define CLK_LNCM(W)                                                                              \
+    if (C == W && N == W)                                                                        \
+        return pg.n == pg.np                                                                     \
+                   ? launch_ln_gdp<TR, W, W, true>(st, z, gamma, beta, wb, mask, a, b, M, eps)   \
+                   : launch_ln_gdp<TR, W, W, true, true>(st, z, gamma, beta, wb, mask, a, b, M, \
+                                                         eps, pg);
+        CLK_LNCM(128) CLK_LNCM(64)
+#undef CLK_LNCM
         return fail(CLK_INVALID_ARGUMENT, "ln_gdp_channel_major: C=%d, N=%d not supported", C, N);
     };
     return dtype == CLK_BF16 ? run(BF16{}) : run(F16{});

@@ -335,9 +335,12 @@ struct TriOutParams {
     E* out;
     int M;
     float eps;
+    PairGrid grid;  // RAG: z and out hold grid.n x grid.n rows, x the padded positions
 };
 
-template <typename TR, int C>
+// RAG: the positions are those of the padded grid (x's planes); z's and out's rows are addressed in
+// the caller's n x n grid, padded positions reading zeros and storing nothing.
+template <typename TR, int C, bool RAG>
 __global__ __launch_bounds__(512) void tri_out_kernel(TriOutParams<typename TR::elem> pr) {
     using E = typename TR::elem;
     using V8 = typename TR::vec8;
@@ -414,8 +417,14 @@ __global__ __launch_bounds__(512) void tri_out_kernel(TriOutParams<typename TR::
     // offsets stay below 8*M*2 bytes whatever C*M is.
     auto stage = [&](int t, char* xb, char* zb) {
         const bool live = t < ntiles;
-        const Rsrc rz = buffer_rsrc(live ? pr.z + (size_t)t * R * C : pr.z,
-                                    live ? (uint32_t)(R * C * 2) : 0u);
+        PairTile pz;
+        if constexpr (RAG) {
+            pz = pair_tile(pr.grid, pr.z, live ? t * R : 0, C);
+            if (!live) pz.r = buffer_rsrc(pr.z, 0);
+        } else {
+            pz.r = buffer_rsrc(live ? pr.z + (size_t)t * R * C : pr.z,
+                               live ? (uint32_t)(R * C * 2) : 0u);
+        }
 #pragma unroll
         for (int k = 0; k < DPX; ++k) {
             const int b = k * NT + wave * 64, c0 = b / (R / 8);
@@ -427,13 +436,32 @@ __global__ __launch_bounds__(512) void tri_out_kernel(TriOutParams<typename TR::
 #pragma unroll
         for (int k = 0; k < DPZ; ++k) {
             const int b = k * NT + wave * 64;
-            buf_dma16(rz, (b + lane) * 16, 0, zb + b * 16);
+            int voff = (b + lane) * 16;
+            if constexpr (RAG) {
+                const int row = pair_row(pr.grid, pz, (b + lane) / PL);
+                voff = row < 0 ? kPastEnd : (row * PL + (b + lane) % PL) * 16;
+            }
+            buf_dma16(pz.r, voff, 0, zb + b * 16);
         }
     };
     // The staged tile's output rows (an empty resource before the first tile), stored as whole
     // rows by all eight waves (NST instructions each).
-    Rsrc pend_out = buffer_rsrc(pr.out, 0);
-    auto flush = [&]() { store_staged_rows<R, C, OSTR, 8>(pend_out, ob, wave, lane); };
+    PairTile pend_out;
+    pend_out.i0 = pend_out.j0 = 0;
+    pend_out.r = buffer_rsrc(pr.out, 0);
+    auto flush = [&]() {
+        if constexpr (RAG) {
+#pragma unroll
+            for (int i = 0; i < NST; ++i) {
+                const int f = (i * 8 + wave) * 64 + lane, row = f / PL, piece = f % PL;
+                const int at = pair_row(pr.grid, pend_out, row);
+                buf_st16_nt(pend_out.r, at < 0 ? kPastEnd : (at * PL + piece) * 16, 0,
+                            *reinterpret_cast<const u32x4*>(ob + row * OSTR + piece * 16));
+            }
+        } else {
+            store_staged_rows<R, C, OSTR, 8>(pend_out.r, ob, wave, lane);
+        }
+    };
 
     auto tile = [&](int t, const char* xc, const char* zc, char* xn, char* zn) {
         vm_wait<NST + DPX + DPZ>();
@@ -505,7 +533,8 @@ __global__ __launch_bounds__(512) void tri_out_kernel(TriOutParams<typename TR::
         }
         lds_barrier();  // xh1, xh2 of tile t ready; xn, zn are free
         stage(t + 2 * gridDim.x, xn, zn);
-        pend_out = buffer_rsrc(pr.out + (size_t)t * R * C, R * C * 2);
+        if constexpr (RAG) pend_out = pair_tile(pr.grid, pr.out, t * R, C);
+        else pend_out.r = buffer_rsrc(pr.out + (size_t)t * R * C, R * C * 2);
 #pragma unroll
         for (int s = 0; s < SUBW; ++s) {
             const int xrow = 16 * (sh * SUBW + s) + r16;
@@ -581,42 +610,13 @@ clk_status launch_einsum(hipStream_t st, const void* a, const void* b, void* x, 
     return launch_einsum_tiles<TR, TN, 256>(st, a, b, x, C, N);
 }
 
-// Positions of an [N, N] grid of U-units (u units per position) copied to or from an [NP, NP]
-// grid (NP >= N): TO_PADDED fills the positions past N with zeros; otherwise only the N x N
-// positions are written back.
-template <typename U, bool TO_PADDED>
-__global__ __launch_bounds__(256) void pad_pairs(const U* __restrict__ src, U* __restrict__ dst,
-                                                 int N, int NP, int u) {
-    const int S = TO_PADDED ? NP : N;  // grid edge of the destination
-    const size_t total = (size_t)S * S * u;
-    for (size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x; idx < total;
-         idx += (size_t)gridDim.x * 256) {
-        const size_t pos = idx / u;
-        const int e = (int)(idx % u), i = (int)(pos / S), j = (int)(pos % S);
-        if constexpr (TO_PADDED) {
-            dst[idx] = (i < N && j < N) ? src[((size_t)i * N + j) * u + e] : U{};
-        } else {
-            dst[idx] = src[((size_t)i * NP + j) * u + e];
-        }
-    }
-}
-
-template <typename U, bool TO_PADDED>
-clk_status launch_pad(hipStream_t st, const void* src, void* dst, int N, int NP, int u) {
-    const int S = TO_PADDED ? NP : N;
-    const size_t total = (size_t)S * S * u;
-    const size_t blocks = (total + 255) / 256;
-    pad_pairs<U, TO_PADDED><<<(int)(blocks < 4096 ? blocks : 4096), 256, 0, st>>>(
-        static_cast<const U*>(src), static_cast<U*>(dst), N, NP, u);
-    return check_launch("triangle_multiply (padding)");
-}
-
 template <typename TR, int C>
 clk_status launch_tri_out(hipStream_t st, const TriOutParams<typename TR::elem>& pr) {
     const int ntiles = pr.M / 64;
     const int grid = ntiles < 256 ? ntiles : 256;
     KernelTimer timer("tri_out", st);
-    tri_out_kernel<TR, C><<<grid, 512, 0, st>>>(pr);
+    if (pr.grid.n == pr.grid.np) tri_out_kernel<TR, C, false><<<grid, 512, 0, st>>>(pr);
+    else tri_out_kernel<TR, C, true><<<grid, 512, 0, st>>>(pr);
     return check_launch("triangle_multiply (output)");
 }
 
@@ -624,8 +624,8 @@ clk_status launch_tri_out(hipStream_t st, const TriOutParams<typename TR::elem>&
 
 clk_status ln_gdp_channel_major(hipStream_t st, clk_dtype dtype, const void* z,
                                 const float* gamma, const float* beta, const void* const* w,
-                                const void* const* bias, const void* mask, void* a, void* b, int M,
-                                int C, int N, float eps);
+                                const void* const* bias, const void* mask, void* a, void* b,
+                                PairGrid pg, int C, int N, float eps);
 
 }  // namespace clk
 
@@ -653,28 +653,12 @@ extern "C" clk_status clk_triangle_einsum(hipStream_t stream, clk_dtype dtype, c
 namespace {
 // N rounded up to a multiple of 8: a ragged N runs the module on a zero-padded grid.
 int64_t padded_n(int64_t N) { return (N + 7) / 8 * 8; }
-size_t round256(size_t v) { return (v + 255) / 256 * 256; }
-// Workspace layout: left, right, x channel-major [C][NP][NP]; for a ragged N also the padded z,
-// mask and output.
-struct TriWorkspace {
-    size_t planes, zp, mp, outp, total;
-};
-TriWorkspace tri_workspace(int64_t N, int64_t C) {
-    const int64_t NP = padded_n(N);
-    const size_t plane_set = (size_t)C * NP * NP * 2;
-    TriWorkspace w;
-    w.planes = 0;
-    w.zp = round256(3 * plane_set);
-    w.mp = w.zp + (N % 8 ? round256(plane_set) : 0);
-    w.outp = w.mp + (N % 8 ? round256((size_t)NP * NP * 2) : 0);
-    w.total = w.outp + (N % 8 ? plane_set : 0);
-    return w;
-}
 }  // namespace
 
 extern "C" size_t clk_triangle_multiply_workspace_size(int64_t N, int64_t C) {
     if (N <= 0 || C <= 0) return 0;
-    return tri_workspace(N, C).total;
+    // left, right and x, channel-major [C][NP][NP].
+    return (size_t)3 * C * padded_n(N) * padded_n(N) * 2;
 }
 
 extern "C" clk_status clk_triangle_multiply(hipStream_t stream, clk_dtype dtype, const void* z,
@@ -705,43 +689,31 @@ extern "C" clk_status clk_triangle_multiply(hipStream_t stream, clk_dtype dtype,
     if (workspace_bytes < need)
         return fail(CLK_INVALID_ARGUMENT, "%s: workspace of %zu bytes, %zu needed", who,
                     workspace_bytes, need);
-    // A ragged N runs on a zero-padded NP x NP grid (mask 0 there, so the padded positions
-    // contribute nothing to the contraction) and copies the N x N outputs back.
-    const TriWorkspace lay = tri_workspace(N, C);
+    // The contraction runs on a zero-padded NP x NP grid (the first step writes zeros there, so
+    // the padding contributes nothing); z, mask and out keep the caller's N x N rows. Copying them
+    // to and from a padded grid around the same kernels took three more launches and 35 of 146 us
+    // at N = 389, C = 128.
     char* const ws = static_cast<char*>(workspace);
-    const bool ragged = N % 8 != 0;
-    const int64_t NP = padded_n(N);
-    if (ragged) {
-        clk_status ps = launch_pad<u32x4, true>(stream, z, ws + lay.zp, (int)N, (int)NP,
-                                                (int)C * 2 / 16);
-        if (ps == CLK_OK)
-            ps = launch_pad<uint16_t, true>(stream, mask, ws + lay.mp, (int)N, (int)NP, 1);
-        if (ps != CLK_OK) return ps;
-        z = ws + lay.zp;
-        mask = ws + lay.mp;
-    }
-    void* const out_final = out;
-    if (ragged) out = ws + lay.outp;
-    const int64_t N0 = N;  // the caller's grid edge
-    N = NP;
-    const int M = (int)(N * N), n = (int)N, c = (int)C;
+    const int NP = (int)padded_n(N);
+    const PairGrid grid{(int)N, NP, 1.f / (float)NP};
+    const int M = NP * NP, c = (int)C;
     const size_t plane_set = (size_t)C * M * 2;
-    char* wa = ws + lay.planes;
+    char* wa = ws;
     char* wb = wa + plane_set;
     char* wx = wb + plane_set;
     // 1. LN_in(z) and the four projections -> left (wa), right (wb), channel-major [C][N][N].
     const void* proj_w[4] = {w[0], w[2], w[1], w[3]};  // left proj, left gate, right proj, right gate
     const void* proj_b[4] = {b[0], b[2], b[1], b[3]};
     clk_status s = ln_gdp_channel_major(stream, dtype, z, ln[0], ln[1], proj_w, proj_b, mask, wa,
-                                        wb, M, c, c, eps);
+                                        wb, grid, c, c, eps);
     if (s != CLK_OK) return s;
     // 2. The contraction: outgoing x[c] = left[c] . right[c]^T; incoming x[c] = right[c]^T .
     //    left[c] (x[i,j] = sum_k left[k,j] right[k,i]), the contraction index first, read
     //    transposed from LDS.
     void* X = wx;
-    s = outgoing ? clk_triangle_einsum(stream, dtype, wa, wb, X, C, N)
-                 : (dtype == CLK_BF16 ? launch_einsum<BF16, true>(stream, wb, wa, X, c, n)
-                                      : launch_einsum<F16, true>(stream, wb, wa, X, c, n));
+    s = outgoing ? clk_triangle_einsum(stream, dtype, wa, wb, X, C, NP)
+                 : (dtype == CLK_BF16 ? launch_einsum<BF16, true>(stream, wb, wa, X, c, NP)
+                                      : launch_einsum<F16, true>(stream, wb, wa, X, c, NP));
     if (s != CLK_OK) return s;
     // 3. LN_c(x), output projection, output gate from LN_in(z).
     auto finish = [&](auto tr) -> clk_status {
@@ -761,9 +733,8 @@ extern "C" clk_status clk_triangle_multiply(hipStream_t stream, clk_dtype dtype,
         pr.out = static_cast<E*>(out);
         pr.M = M;
         pr.eps = eps;
+        pr.grid = grid;
         return c == 128 ? launch_tri_out<TR, 128>(stream, pr) : launch_tri_out<TR, 64>(stream, pr);
     };
-    s = dtype == CLK_BF16 ? finish(BF16{}) : finish(F16{});
-    if (s != CLK_OK || !ragged) return s;
-    return launch_pad<u32x4, false>(stream, out, out_final, (int)N0, (int)NP, (int)C * 2 / 16);
+    return dtype == CLK_BF16 ? finish(BF16{}) : finish(F16{});
 }

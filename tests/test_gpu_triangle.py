@@ -156,3 +156,28 @@ def test_einsum_tile_choice(cuda, c, n, chs):
     for ch in chs:
         assert_close("x[%d]" % ch, x[ch], ref.einsum(np64(a[ch:ch + 1]), np64(b[ch:ch + 1]))[0],
                      TOL["bf16"]["o"])
+
+
+# Ragged N around the 64-position tiles of the padded grid (rows shorter and longer than a tile)
+# and around the 128-wide contraction tiles: the kernels address the caller's rows in place.
+RAGGED_EDGES = [(2, 64), (7, 128), (57, 128), (63, 64), (65, 128), (123, 64), (129, 128)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=dname)
+@pytest.mark.parametrize("n,c", RAGGED_EDGES)
+def test_triangle_multiply_ragged_edges(cuda, n, c, dtype):
+    """Both directions against the oracle; the same values on a grid extended by masked
+    positions to a multiple of 8 give the same bits."""
+    z, mask, ln_in, ws, bs, ln_c = module_case(n, c, dtype, 3 * n + c, cuda)
+    p = (n + 7) // 8 * 8
+    zp = torch.zeros((p, p, c), dtype=dtype, device=cuda)
+    mp = torch.zeros((p, p), dtype=dtype, device=cuda)
+    zp[:n, :n], mp[:n, :n] = z, mask
+    for outgoing in (True, False):
+        out = ops.triangle_multiply(z, mask, ln_in, ws, bs, ln_c, outgoing)
+        r = ref.triangle_multiply(np64(z), np64(mask), tuple(map(np64, ln_in)),
+                                  [np64(w) for w in ws], [np64(b) for b in bs],
+                                  tuple(map(np64, ln_c)), outgoing)
+        assert_close("out", out, r, 2e-2 if dtype == torch.bfloat16 else 1e-2)
+        padded = ops.triangle_multiply(zp, mp, ln_in, ws, bs, ln_c, outgoing)
+        assert torch.equal(out, padded[:n, :n])
