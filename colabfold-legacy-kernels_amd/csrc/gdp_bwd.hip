@@ -3,10 +3,10 @@
 //   out = mask * p * s,  p = x.wp + bp,  s = sigmoid(x.wg + bg)
 //   dp = dout * mask * s,  dg = dout * mask * p * s * (1 - s)
 //   dx = dp.wp^T + dg.wg^T,  dwp = x^T.dp,  dwg = x^T.dg,  dbp = sum_m dp,  dbg = sum_m dg
-// Four kernels (three at K = N), deterministic (no float atomics):
+// At K = N one kernel, gdp_bwd_fused, does all but the last sum. Otherwise four kernels; all
+// deterministic (no float atomics):
 //   gdp_bwd_grad  recomputes p and the gate on MFMA (weights resident as in the forward) and
 //                 writes dpg = [dp | dg] (M x 2N, input dtype) and per-block column sums of dp, dg;
-//                 at K = N it also computes dx from the tile it holds;
 //   gdp_bwd_dx    dx = dpg . [wp | wg]^T, the transposed weights resident as MFMA A operands;
 //   gdp_bwd_dw    per-block partials of x^T . dpg over a contiguous range of rows, both operands
 //                 read transposed from LDS (ds_read_b64_tr_b16);
@@ -58,20 +58,14 @@ __device__ __forceinline__ void stage_swz(Rsrc rsrc, char* lds, int wave, int la
 // x arrives by buffer->LDS loads two tiles ahead and dout, mask of the next tile are loaded into
 // registers. A lane's accumulators hold 8 consecutive columns of one row, the layout of its
 // 16-byte dout vector and of its two 16-byte stores into dpg.
-// FDX (K == N): dx of the tile as well, so that dpg is not read back for it. The tile's
-// [dp | dg] rows go into LDS in the dx kernel's swizzled layout, and after a second barrier wave
-// w computes dx columns 32w..32w+31 = [dp | dg] . wcat^T's rows, held as A operands in registers
-// as in the dx kernel (with one wave per SIMD the registers allow it); dx is stored (or added to,
-// with accumulate) through a resource per tile.
 // ---------------------------------------------------------------------------------------------
-template <typename TR, int K, int N, bool FDX = false>
+template <typename TR, int K, int N>
 __global__ __launch_bounds__(2 * N) void gdp_bwd_grad_kernel(
     const typename TR::elem* __restrict__ x, const typename TR::elem* __restrict__ wp,
     const typename TR::elem* __restrict__ bp, const typename TR::elem* __restrict__ wg,
     const typename TR::elem* __restrict__ bg, const typename TR::elem* __restrict__ mask,
     const typename TR::elem* __restrict__ dout, typename TR::elem* __restrict__ dpg,
-    float* __restrict__ dbpart, int M, typename TR::elem* __restrict__ dx = nullptr,
-    int accumulate = 0) {
+    float* __restrict__ dbpart, int M) {
     using E = typename TR::elem;
     using V8 = typename TR::vec8;
     using S = SwzRows<K < 128 ? 128 : K>;  // K = 64 rows use a 128-wide tile (upper half zero)
@@ -80,32 +74,13 @@ __global__ __launch_bounds__(2 * N) void gdp_bwd_grad_kernel(
     constexpr int XB = R * KT * 2;
     constexpr int DPW = R * S::PL / NT;
 
-    static_assert(!FDX || K == N, "the fused dx takes one wave per 32 dx columns: K == N");
-    constexpr int W2 = 2 * N, KS2 = W2 / 32;
-    using S2 = SwzRows<W2>;
-
     __shared__ __attribute__((aligned(16))) char x0[XB];
     __shared__ __attribute__((aligned(16))) char x1[XB];
     __shared__ __attribute__((aligned(16))) char x2[XB];
-    __shared__ __attribute__((aligned(16))) char tg[FDX ? R * W2 * 2 : 16];  // [dp | dg] tile
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, g = lane >> 4;
-
-    // FDX: wcat^T's rows k = 32w + 8(r16/4) + 4h + r16%4 (8 consecutive n' per 16-byte load).
-    V8 wd[FDX ? 2 : 1][FDX ? KS2 : 1];
-    if constexpr (FDX) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int k = 32 * wave + 8 * (r16 >> 2) + 4 * h + (r16 & 3);
-#pragma unroll
-            for (int ks = 0; ks < KS2; ++ks) {
-                const int n = 32 * ks + 8 * g;
-                wd[h][ks] = bits_as<V8>(ld16(n < N ? wp + k * N + n : wg + k * N + (n - N)));
-            }
-        }
-    }
 
     V8 wa[2][2][KS];
     f32x4 binit[2][2];
@@ -223,40 +198,6 @@ __global__ __launch_bounds__(2 * N) void gdp_bwd_grad_kernel(
         }
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         store(out_rsrc(t));
-        if constexpr (FDX) {
-            // tg is free: every wave finished reading the previous tile's before this tile's
-            // first barrier.
-#pragma unroll
-            for (int sub = 0; sub < SUB; ++sub)
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-                    *reinterpret_cast<u32x4*>(
-                        tg + S2::piece_at(16 * sub + r16, (q * N + col0) / 8) * 16) = res[q][sub];
-            lds_barrier();
-            const Rsrc rdx = buffer_rsrc(rows > 0 ? dx + (size_t)t * R * K : dx,
-                                         (uint32_t)rows * K * 2);
-#pragma unroll
-            for (int sub = 0; sub < SUB; ++sub) {
-                const int xrow = 16 * sub + r16;
-                f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-                for (int ks = 0; ks < KS2; ++ks) {
-                    const V8 v = *reinterpret_cast<const V8*>(tg + S2::piece_at(xrow, 4 * ks + g) * 16);
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) acc[h] = TR::mfma(wd[h][ks], v, acc[h]);
-                }
-                float o[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) o[j] = acc[j >> 2][j & 3];
-                if (accumulate && xrow < rows) {
-                    float prev[8];
-                    unpack8<TR>(ld16(dx + ((size_t)t * R + xrow) * K + col0), prev);
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) o[j] += prev[j];
-                }
-                buf_st16(rdx, (xrow * K + col0) * 2, 0, pack8<TR>(o));
-            }
-        }
     };
 
     int t = blockIdx.x;
@@ -294,6 +235,289 @@ __global__ __launch_bounds__(2 * N) void gdp_bwd_grad_kernel(
             for (int j = 0; j < 8; ++j) o[q * N + col0 + j] = cs[q][j];
     }
     async_wait();
+}
+
+// ---------------------------------------------------------------------------------------------
+// The whole backward at K = N (64 or 128: the pair and template stacks) in one pass over x and
+// dout. A block has three kinds of waves, N/32 of each, and walks 64-row tiles:
+//   grad waves: wave w recomputes columns 32w..32w+31 of p and of the gate (weights resident as A
+//     operands), takes dout and the mask of the next tile into registers a tile ahead, and writes
+//     the tile's [dp | dg] rows to LDS (and keeps the column sums);
+//   dx waves, a step later: dx = [dp | dg] . wcat^T, the transposed weights resident as A operands;
+//   dW waves, a step later: dW += x^T . [dp | dg], both read transposed from LDS, the float32 sums
+//     of the block's rows resident in registers (64 k x N n' per wave). They also stage x by direct
+//     buffer->LDS loads two tiles ahead, four buffers deep (a tile is read in two steps).
+// One barrier per tile; the roles run separate loops with the same barrier count, so neither holds
+// the others' registers (three waves per SIMD, one of each role; with dx and dW in one role, at
+// two waves per SIMD, its resident operands and sums spill). HBM traffic is x, dout and dx once
+// and the blocks' weight partials. Kept apart, dpg = [dp | dg] went through memory between a grad
+// + dx kernel and a dW kernel: MEASURE_HERE
+// ---------------------------------------------------------------------------------------------
+template <typename TR, int N>
+__global__ __launch_bounds__(6 * N) __attribute__((amdgpu_waves_per_eu(3))) void gdp_bwd_fused_kernel(
+    const typename TR::elem* __restrict__ x, const typename TR::elem* __restrict__ wp,
+    const typename TR::elem* __restrict__ bp, const typename TR::elem* __restrict__ wg,
+    const typename TR::elem* __restrict__ bg, const typename TR::elem* __restrict__ mask,
+    const typename TR::elem* __restrict__ dout, typename TR::elem* __restrict__ dx,
+    float* __restrict__ part, float* __restrict__ dbpart, int M, int accumulate) {
+    using E = typename TR::elem;
+    using V8 = typename TR::vec8;
+    constexpr int K = N, W2 = 2 * N, NW = N / 32, R = kBwdRows, SUB = R / 16;
+    constexpr int KS = K / 32, KS2 = W2 / 32;
+    using S = SwzRows<K>;
+    using S2 = SwzRows<W2>;
+    constexpr int XB = R * K * 2, TB = R * W2 * 2;
+    constexpr int DPW = R * S::PL / (64 * NW);  // x loads per dW lane and tile
+    constexpr int WK = K / 64, WN = NW / WK;    // dW waves along k (64 each) and n'
+    constexpr int NTL = W2 / (16 * WN);         // 16-wide n' tiles per dW wave
+    static_assert(WK * WN == NW && DPW * 64 * NW == R * S::PL, "dW waves cover the tile");
+
+    // Separate objects: a read of one does not wait for the loads in flight into another.
+    __shared__ __attribute__((aligned(16))) char x0[XB];
+    __shared__ __attribute__((aligned(16))) char x1[XB];
+    __shared__ __attribute__((aligned(16))) char x2[XB];
+    __shared__ __attribute__((aligned(16))) char x3[XB];
+    __shared__ __attribute__((aligned(16))) char t0[TB];
+    __shared__ __attribute__((aligned(16))) char t1[TB];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    const int G = gridDim.x, ntiles = (M + R - 1) / R;
+    const int mine = (ntiles - (int)blockIdx.x + G - 1) / G;  // tiles of this block (>= 1)
+    // Steps 0 .. mine (step j: grad waves on tile j, the others on tile j - 1), rounded up to the
+    // loops' four copies; the extra steps are barriers only.
+    const int steps = (mine + 4) / 4 * 4;
+    auto tile_of = [&](int j) { return (int)blockIdx.x + j * G; };
+    // Rows [t*R, M) of a [M, W] matrix of 2-byte elements that lie in the block's tile j (rows past
+    // M, and every row of a tile past the block's last, read zeros and drop stores).
+    auto tile_rsrc = [&](const E* base, int W, int j) {
+        const int t = tile_of(j), rows = j < mine ? min(R, M - t * R) : 0;
+        return buffer_rsrc(rows > 0 ? base + (size_t)t * R * W : base, (uint32_t)rows * W * 2);
+    };
+
+    if (wave < NW) {
+        // ---- grad waves ----
+        const int col0 = 32 * wave + 8 * g;
+        V8 wa[2][2][KS];
+        f32x4 binit[2][2];
+#pragma unroll
+        for (int mat = 0; mat < 2; ++mat) {
+            const E* W = mat == 0 ? wp : wg;
+            const float fold = mat == 1 ? -kLog2e : 1.f;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int col = 32 * wave + 8 * (r16 >> 2) + 4 * h + (r16 & 3);
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        wa[mat][h][ks][j] =
+                            TR::from_f(fold * TR::to_f(W[(32 * ks + 8 * g + j) * N + col]));
+                const E* b = mat == 0 ? bp : bg;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) binit[mat][h][i] = fold * TR::to_f(b[col0 + 4 * h + i]);
+            }
+        }
+        float cs[2][8];  // column sums of dp, dg over this block's rows
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) cs[q][j] = 0.f;
+        // dout and mask of one 16-row sub-tile; each is loaded for the next tile as soon as the
+        // current tile's has been used.
+        u32x4 dv[SUB];
+        uint32_t mv[SUB];
+        auto load_rows = [&](int sub, Rsrc rd, Rsrc rm) {
+            const int row = 16 * sub + r16;
+            dv[sub] = __builtin_amdgcn_raw_buffer_load_b128(rd, (row * N + col0) * 2, 0, 0);
+            mv[sub] = __builtin_amdgcn_raw_buffer_load_b16(rm, row * 2, 0, 0);
+        };
+        auto step = [&](int j, const char* xc, char* tw) {
+            lds_barrier();  // x tile j in xc; the dx and dW waves are done with tw
+            if (j >= mine) return;
+            const Rsrc rd = tile_rsrc(dout, N, j + 1), rm = tile_rsrc(mask, 1, j + 1);
+#pragma unroll
+            for (int sub = 0; sub < SUB; ++sub) {
+                const int row = 16 * sub + r16;
+                f32x4 acc[2][2];
+#pragma unroll
+                for (int mat = 0; mat < 2; ++mat)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) acc[mat][h] = binit[mat][h];
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    const V8 xv =
+                        *reinterpret_cast<const V8*>(xc + S::piece_at(row, 4 * ks + g) * 16);
+#pragma unroll
+                    for (int mat = 0; mat < 2; ++mat)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h)
+                            acc[mat][h] = TR::mfma(wa[mat][h][ks], xv, acc[mat][h]);
+                }
+                float d[8], dp[8], dg[8];
+                unpack8<TR>(dv[sub], d);
+                const float m = TR::to_f(__builtin_bit_cast(E, (uint16_t)mv[sub]));
+                load_rows(sub, rd, rm);
+#pragma unroll
+                for (int j8 = 0; j8 < 8; ++j8) {
+                    const int h = j8 >> 2, i = j8 & 3;
+                    const float sg = fast_rcp(1.f + fast_exp2(acc[1][h][i]));
+                    const float dm = d[j8] * m;
+                    dp[j8] = dm * sg;
+                    dg[j8] = dp[j8] * acc[0][h][i] * (1.f - sg);
+                    cs[0][j8] += dp[j8];
+                    cs[1][j8] += dg[j8];
+                }
+                *reinterpret_cast<u32x4*>(tw + S2::piece_at(row, col0 / 8) * 16) = pack8<TR>(dp);
+                *reinterpret_cast<u32x4*>(tw + S2::piece_at(row, (N + col0) / 8) * 16) =
+                    pack8<TR>(dg);
+            }
+        };
+#pragma unroll
+        for (int sub = 0; sub < SUB; ++sub)
+            load_rows(sub, tile_rsrc(dout, N, 0), tile_rsrc(mask, 1, 0));
+        for (int j = 0; j < steps; j += 4) {
+            step(j, x0, t0);
+            step(j + 1, x1, t1);
+            step(j + 2, x2, t0);
+            step(j + 3, x3, t1);
+        }
+        // The 16 lanes of a lane group hold the same 8 columns of different rows.
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) cs[q][j] = group_sum<16>(cs[q][j]);
+        if (r16 == 0) {
+            float* o = dbpart + (size_t)blockIdx.x * W2;
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) o[q * N + col0 + j] = cs[q][j];
+        }
+        return;
+    }
+
+    if (wave < 2 * NW) {
+        // ---- dx waves ----
+        const int pw = wave - NW, col0 = 32 * pw + 8 * g;
+        V8 wd[2][KS2];  // wcat^T's rows k = 32pw + 8(r16/4) + 4h + r16%4
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int k = 32 * pw + 8 * (r16 >> 2) + 4 * h + (r16 & 3);
+#pragma unroll
+            for (int ks = 0; ks < KS2; ++ks) {
+                const int n = 32 * ks + 8 * g;
+                wd[h][ks] = bits_as<V8>(ld16(n < N ? wp + k * N + n : wg + k * N + (n - N)));
+            }
+        }
+        // The dx already there, a tile ahead (zeros from an empty resource without accumulate).
+        auto load_prev = [&](int j, u32x4 (&pv)[SUB]) {
+            const Rsrc r = accumulate ? tile_rsrc(dx, K, j) : buffer_rsrc(dx, 0);
+#pragma unroll
+            for (int sub = 0; sub < SUB; ++sub)
+                pv[sub] = __builtin_amdgcn_raw_buffer_load_b128(
+                    r, ((16 * sub + r16) * K + col0) * 2, 0, 0);
+        };
+        u32x4 pa[SUB], pb[SUB];
+        auto step = [&](int j, const char* tp, const u32x4 (&pc)[SUB], u32x4 (&pn)[SUB]) {
+            lds_barrier();  // tile j - 1 in tp
+            load_prev(j, pn);
+            if (j == 0 || j > mine) return;
+            const Rsrc rdx = tile_rsrc(dx, K, j - 1);
+#pragma unroll
+            for (int sub = 0; sub < SUB; ++sub) {
+                const int row = 16 * sub + r16;
+                f32x4 da[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+                for (int ks = 0; ks < KS2; ++ks) {
+                    const V8 v =
+                        *reinterpret_cast<const V8*>(tp + S2::piece_at(row, 4 * ks + g) * 16);
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) da[h] = TR::mfma(wd[h][ks], v, da[h]);
+                }
+                float o[8], pv[8];
+                unpack8<TR>(pc[sub], pv);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) o[i] = da[i >> 2][i & 3] + pv[i];
+                buf_st16(rdx, (row * K + col0) * 2, 0, pack8<TR>(o));
+            }
+        };
+        for (int j = 0; j < steps; j += 2) {
+            step(j, t1, pb, pa);
+            step(j + 1, t0, pa, pb);
+        }
+        return;
+    }
+
+    // ---- dW waves ----
+    const int pw = wave - 2 * NW, wk = pw % WK, wn = pw / WK;
+    f32x4 acc[NTL][4];
+#pragma unroll
+    for (int a = 0; a < NTL; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto stage = [&](int j, char* xb) {
+        stage_swz<K, R, 64 * NW>(tile_rsrc(x, K, j), xb, pw, lane);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    };
+    // Step j: x tile j has landed; tile j + 2 goes into xn; tile j - 1 (xp, tp) is multiplied.
+    auto step = [&](int j, const char* xp, char* xn, const char* tp) {
+        vm_wait<DPW>();
+        lds_barrier();
+        stage(j + 2, xn);
+        if (j == 0 || j > mine) return;
+        // Transposed operand: lane (r16, g) gets column 16a + r16 of rows ms + 8g .. + 7 (two 4-row
+        // reads). Its pieces 2a + (r16 & 3)/2 of rows r and r + 4 sit at piece ^ (r & 7), so four
+        // lane offsets (a % 4) serve a whole tile with immediate offsets: the upper read of a is
+        // the lower one of a ^ 2 four rows on. Formed from an opaque lane index: held in registers
+        // across the steps they would spill.
+        int lr = lane;
+        asm volatile("" : "+v"(lr));
+        const int m = (lr >> 2) & 3, trow = 8 * (lr >> 4) + m;
+        int xo[4], to[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int at = 16 * ((2 * q + ((lr >> 1) & 1)) ^ m) + 8 * (lr & 1);
+            xo[q] = trow * (2 * K) + at;
+            to[q] = trow * (2 * W2) + at;
+        }
+        auto tr_operand = [&](const char* base, const int (&off)[4], int pitch, int ms, int a) {
+            const char* at = base + ms * pitch + (a >> 2) * 128;
+            return lds_tr8<V8>(at + off[a & 3], at + 4 * pitch + off[(a & 3) ^ 2]);
+        };
+#pragma unroll
+        for (int ms = 0; ms < R; ms += 32) {
+            V8 ax[4];
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt)
+                ax[kt] = tr_operand(xp + wk * 128, xo, 2 * K, ms, kt);
+#pragma unroll
+            for (int a = 0; a < NTL; ++a) {
+                const V8 bt = tr_operand(tp + wn * (NTL * 32), to, 2 * W2, ms, a);
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt) acc[a][kt] = TR::mfma(ax[kt], bt, acc[a][kt]);
+                if (a & 1) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    stage(0, x0);
+    stage(1, x1);
+    for (int j = 0; j < steps; j += 4) {
+        step(j, x3, x2, t1);
+        step(j + 1, x0, x3, t0);
+        step(j + 2, x1, x0, t1);
+        step(j + 3, x2, x1, t0);
+    }
+    // Lane (r16, g) of accumulator (a, kt): n' = (NTL*wn + a)*16 + r16, k = 64wk + 16kt + 4g + q.
+    float* pb = part + (size_t)blockIdx.x * (W2 * K + W2);
+#pragma unroll
+    for (int a = 0; a < NTL; ++a)
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+            *reinterpret_cast<f32x4*>(pb + ((NTL * wn + a) * 16 + r16) * K + 64 * wk + 16 * kt +
+                                      4 * g) = acc[a][kt];
+    async_wait();  // no direct-to-LDS load may still be in flight when the workgroup ends
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -794,16 +1018,18 @@ struct BwdGeom {
     size_t dpg_off, part_off, dbpart_off, total;
 };
 
+// K == N: one fused kernel, so no dpg, and its blocks' partials are both the weights' and the
+// biases' (two 64 KB blocks share a CU at 64, one of 128 KB at 128).
 BwdGeom bwd_geom(int64_t M, int K, int N) {
     BwdGeom g;
     const int64_t ntiles = (M + kBwdRows - 1) / kBwdRows;
     const int per_cu = 128 / N;
     g.grad_blocks = (int)(ntiles < 256 * per_cu ? ntiles : 256 * per_cu);
-    g.dw_blocks = (int)(ntiles < 256 ? ntiles : 256);
+    g.dw_blocks = K == N ? g.grad_blocks : (int)(ntiles < 256 ? ntiles : 256);
     g.dw_tiles = (int)((ntiles + g.dw_blocks - 1) / g.dw_blocks);
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
     g.dpg_off = 0;
-    g.part_off = up((size_t)M * 2 * N * 2);
+    g.part_off = K == N ? 0 : up((size_t)M * 2 * N * 2);
     g.dbpart_off = g.part_off + up((size_t)g.dw_blocks * (2 * N * K + 2 * N) * 4);
     g.total = g.dbpart_off + up((size_t)g.grad_blocks * 2 * N * 4);
     return g;
@@ -816,30 +1042,29 @@ clk_status run_gdp_bwd(hipStream_t st, const void* x, const void* wp, const void
                        int accumulate) {
     using E = typename TR::elem;
     const BwdGeom gm = bwd_geom(M, K, N);
-    E* dpg = reinterpret_cast<E*>(ws + gm.dpg_off);
     float* part = reinterpret_cast<float*>(ws + gm.part_off);
     float* dbpart = reinterpret_cast<float*>(ws + gm.dbpart_off);
     if constexpr (K == N) {
-        // dx computed by the grad kernel from the tile it already holds.
-        KernelTimer timer("gdp_bwd_grad", st);
-        gdp_bwd_grad_kernel<TR, K, N, true><<<gm.grad_blocks, 2 * N, 0, st>>>(
+        KernelTimer timer("gdp_bwd", st);
+        gdp_bwd_fused_kernel<TR, N><<<gm.grad_blocks, 6 * N, 0, st>>>(
             (const E*)x, (const E*)wp, (const E*)bp, (const E*)wg, (const E*)bg, (const E*)mask,
-            (const E*)dout, dpg, dbpart, M, (E*)dx, accumulate);
+            (const E*)dout, (E*)dx, part, dbpart, M, accumulate);
     } else {
+        E* dpg = reinterpret_cast<E*>(ws + gm.dpg_off);
         {
             KernelTimer timer("gdp_bwd_grad", st);
             gdp_bwd_grad_kernel<TR, K, N><<<gm.grad_blocks, 2 * N, 0, st>>>(
                 (const E*)x, (const E*)wp, (const E*)bp, (const E*)wg, (const E*)bg,
                 (const E*)mask, (const E*)dout, dpg, dbpart, M);
         }
-        const int ntiles = (M + kBwdRows - 1) / kBwdRows;
-        const int per_cu = 128 / K;
-        const int grid = ntiles < 256 * per_cu ? ntiles : 256 * per_cu;
-        KernelTimer timer("gdp_bwd_dx", st);
-        gdp_bwd_dx_kernel<TR, K, N><<<grid, 2 * K, 0, st>>>(dpg, (const E*)wp, (const E*)wg,
-                                                           (E*)dx, M, accumulate);
-    }
-    {
+        {
+            const int ntiles = (M + kBwdRows - 1) / kBwdRows;
+            const int per_cu = 128 / K;
+            const int grid = ntiles < 256 * per_cu ? ntiles : 256 * per_cu;
+            KernelTimer timer("gdp_bwd_dx", st);
+            gdp_bwd_dx_kernel<TR, K, N><<<grid, 2 * K, 0, st>>>(dpg, (const E*)wp, (const E*)wg,
+                                                               (E*)dx, M, accumulate);
+        }
         KernelTimer timer("gdp_bwd_dw", st);
         gdp_bwd_dw_kernel<TR, K, N><<<gm.dw_blocks, 512, 0, st>>>((const E*)x, dpg, part, M,
                                                                   gm.dw_tiles);
