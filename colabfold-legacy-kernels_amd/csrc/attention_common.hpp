@@ -111,13 +111,6 @@ __device__ __forceinline__ void zero_v_padding(E* lds) {
     }
 }
 
-// 16-byte load of eight 2-byte elements, and store of four floats, at any element alignment.
-typedef unsigned int u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
-typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ u32x4 ld16_a2(const void* p) {
-    return *reinterpret_cast<const u32x4_a2*>(p);
-}
-
 // Eight bias values bias_row[kk .. kk+7] as float (zero past Sk).
 template <typename TR>
 __device__ __forceinline__ void load_bias8(const typename TR::elem* row, int kk, int Sk,

@@ -80,6 +80,16 @@ __device__ __forceinline__ u32x2 ld8(const void* p) {
 }
 __device__ __forceinline__ void st8(void* p, u32x2 v) { *reinterpret_cast<u32x2*>(p) = v; }
 
+// 16-byte accesses of eight 2-byte elements, and of four floats, at any element alignment.
+typedef unsigned int u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ u32x4 ld16_a2(const void* p) {
+    return *reinterpret_cast<const u32x4_a2*>(p);
+}
+__device__ __forceinline__ f32x4 ld4f(const float* p) {
+    return *reinterpret_cast<const f32x4_a4*>(p);
+}
+
 template <typename V>
 __device__ __forceinline__ V bits_as(u32x4 v) {
     return __builtin_bit_cast(V, v);
@@ -97,6 +107,33 @@ __device__ __forceinline__ V lds_tr8(const void* p_lo, const void* p_hi) {
     typedef short i16x8 __attribute__((ext_vector_type(8)));
     i16x8 r = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
     return __builtin_bit_cast(V, r);
+}
+
+// MFMA A operands W^T of one wave's 32 output columns, for the kernels that keep their weights in
+// registers: W has 32*KS rows, `ldw` elements apart; w points at the wave's first column. Operand
+// (h, ks), lane (r16, g): column 8*(r16/4) + 4h + r16%4, rows 32ks + 8g .. + 7. The rows arrive as
+// 16-byte pieces (any element alignment) and are transposed through `scratch`, 2*KS KB of LDS of
+// the wave's own (in order within the wave, so no barrier). Read straight from memory the
+// operands are 64*KS two-byte loads per lane, which held up the kernels' small calls and spilled
+// the larger ones (triangle multiplication at N = 203, C = 128 45 -> 41 us, at 512 1-2% faster).
+template <int KS, typename V8, typename E>
+__device__ __forceinline__ void load_weight_columns(const E* w, int ldw, char* scratch, int lane,
+                                                    V8 (&out)[2][KS]) {
+    const int r16 = lane & 15, g = lane >> 4;
+    u32x4 raw[2 * KS];
+#pragma unroll
+    for (int i = 0; i < 2 * KS; ++i)
+        raw[i] = ld16_a2(w + (size_t)(16 * i + (lane >> 2)) * ldw + 8 * (lane & 3));
+#pragma unroll
+    for (int i = 0; i < 2 * KS; ++i)
+        *reinterpret_cast<u32x4*>(scratch + (16 * i + (lane >> 2)) * 64 + 16 * (lane & 3)) = raw[i];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const char* lo = scratch + (32 * ks + 8 * g + (r16 >> 2)) * 64 + 16 * (r16 & 3) + 8 * h;
+            out[h][ks] = lds_tr8<V8>(lo, lo + 4 * 64);
+        }
 }
 
 // Eight 2-byte elements (one 16-byte load) as floats.

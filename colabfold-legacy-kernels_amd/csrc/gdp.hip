@@ -412,24 +412,44 @@ __global__ __launch_bounds__(64 * NB * N / 32 + 256) void ln_gdp_kernel(
     V8 wa[2][2][KS];
     f32x4 binit[2][2];
     if (mfma_wave) {
+        // The weights' transpose scratch: the output staging buffers, or the normalised tiles
+        // (neither is written before the first barrier).
+        constexpr int HALF = (NWM + 1) / 2;
+        static_assert(HALF * C * 64 <= (OST ? PLAN::OBB : ZB), "the waves' scratch fits");
+        char* const scratch = (wave < HALF ? (OST ? ob0 : xh0) : (OST ? ob1 : xh1)) +
+                              (wave % HALF) * (C * 64);
 #pragma unroll
         for (int mat = 0; mat < 2; ++mat) {
-            const E* W = wb.w[2 * br + mat];
             const float fold = mat == 1 ? -kLog2e : 1.f;
+            load_weight_columns<KS>(wb.w[2 * br + mat] + 32 * cb, N, scratch, lane, wa[mat]);
+            float part[2] = {0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+                f32x4 ga[2], be[2];
+                if constexpr (LN) {
+                    const int k = 32 * ks + 8 * g;
+                    ga[0] = ld4f(gamma + k);
+                    ga[1] = ld4f(gamma + k + 4);
+                    be[0] = ld4f(beta + k);
+                    be[1] = ld4f(beta + k + 4);
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const float v = TR::to_f(wa[mat][h][ks][j]);
+                        if constexpr (LN) {
+                            wa[mat][h][ks][j] = TR::from_f(ga[j >> 2][j & 3] * v * fold);
+                            part[h] = fmaf(be[j >> 2][j & 3], v, part[h]);
+                        } else if (mat == 1) {
+                            wa[mat][h][ks][j] = TR::from_f(v * fold);
+                        }
+                    }
+            }
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int col = 32 * cb + 8 * (r16 >> 2) + 4 * h + (r16 & 3);
-                float part = 0.f;
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const int k = 32 * ks + 8 * g + j;
-                        const float v = TR::to_f(W[(size_t)k * N + col]);
-                        wa[mat][h][ks][j] = TR::from_f((LN ? gamma[k] : 1.f) * v * fold);
-                        if constexpr (LN) part = fmaf(beta[k], v, part);
-                    }
-                const float bcol = (xgroup_sum(part) + TR::to_f(wb.b[2 * br + mat][col])) * fold;
+                const float bcol = (xgroup_sum(part[h]) + TR::to_f(wb.b[2 * br + mat][col])) * fold;
                 if constexpr (CM) {
                     binit[mat][h] = f32x4{bcol, bcol, bcol, bcol};
                 } else {

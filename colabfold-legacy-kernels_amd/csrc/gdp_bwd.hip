@@ -301,20 +301,21 @@ __global__ __launch_bounds__(6 * N) __attribute__((amdgpu_waves_per_eu(3))) void
         const int col0 = 32 * wave + 8 * g;
         V8 wa[2][2][KS];
         f32x4 binit[2][2];
+        static_assert(NW * K * 64 <= TB, "the waves' transpose scratch fits");
 #pragma unroll
         for (int mat = 0; mat < 2; ++mat) {
-            const E* W = mat == 0 ? wp : wg;
+            load_weight_columns<KS>((mat == 0 ? wp : wg) + 32 * wave, N, t0 + wave * (K * 64), lane,
+                                    wa[mat]);
             const float fold = mat == 1 ? -kLog2e : 1.f;
+            const E* b = mat == 0 ? bp : bg;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int col = 32 * wave + 8 * (r16 >> 2) + 4 * h + (r16 & 3);
+                if (mat == 1)
 #pragma unroll
-                for (int ks = 0; ks < KS; ++ks)
+                    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        wa[mat][h][ks][j] =
-                            TR::from_f(fold * TR::to_f(W[(32 * ks + 8 * g + j) * N + col]));
-                const E* b = mat == 0 ? bp : bg;
+                        for (int j = 0; j < 8; ++j)
+                            wa[mat][h][ks][j] = TR::from_f(fold * TR::to_f(wa[mat][h][ks][j]));
 #pragma unroll
                 for (int i = 0; i < 4; ++i) binit[mat][h][i] = fold * TR::to_f(b[col0 + 4 * h + i]);
             }

@@ -384,27 +384,36 @@ __global__ __launch_bounds__(512) void tri_out_kernel(TriOutParams<typename TR::
     // biases (bc . w_out + b_out, -log2(e) (bin . w_g + b_g)) in C-tile layout.
     V8 wa[2][2][KS];
     f32x4 binit[2][2];
+    // Their transpose scratch, two waves to a buffer, is not written before the first barrier.
+    static_assert(2 * C * 64 <= ZB && ZB <= XB, "the waves' scratch fits");
+    char* const scratch =
+        (wave < 2 ? z2 : wave < 4 ? x2 : wave < 6 ? xh1 : xh2) + (wave & 1) * (C * 64);
 #pragma unroll
     for (int mat = 0; mat < 2; ++mat) {
-        const E* W = mat == 0 ? pr.wout : pr.wg;
         const float* gam = mat == 0 ? pr.gc : pr.gin;
         const float* bet = mat == 0 ? pr.bc : pr.bin;
         const float fold = mat == 1 ? -kLog2e : 1.f;
+        load_weight_columns<KS>((mat == 0 ? pr.wout : pr.wg) + 32 * cb, C, scratch, lane, wa[mat]);
+        float part[2] = {0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int k = 32 * ks + 8 * g;
+            const f32x4 g2[2] = {ld4f(gam + k), ld4f(gam + k + 4)};
+            const f32x4 b2[2] = {ld4f(bet + k), ld4f(bet + k + 4)};
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const float v = TR::to_f(wa[mat][h][ks][j]);
+                    wa[mat][h][ks][j] = TR::from_f(g2[j >> 2][j & 3] * v * fold);
+                    part[h] = fmaf(b2[j >> 2][j & 3], v, part[h]);
+                }
+        }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int col = 32 * cb + 8 * (r16 >> 2) + 4 * h + (r16 & 3);
-            float part = 0.f;
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int k = 32 * ks + 8 * g + j;
-                    const float v = TR::to_f(W[k * C + col]);
-                    wa[mat][h][ks][j] = TR::from_f(gam[k] * v * fold);
-                    part = fmaf(bet[k], v, part);
-                }
             const E* bias = mat == 0 ? pr.bout : pr.bg;
-            const float bcol = (xgroup_sum(part) + TR::to_f(bias[col])) * fold;
+            const float bcol = (xgroup_sum(part[h]) + TR::to_f(bias[col])) * fold;
 #pragma unroll
             for (int i = 0; i < 4; ++i) binit[mat][h][i] = __shfl(bcol, 4 * g + i);
         }

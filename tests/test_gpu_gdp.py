@@ -323,3 +323,47 @@ def test_gdp_bwd_beyond_two_gib(cuda):
         sums = list(r) if sums is None else [u + v for u, v in zip(sums, r)]
     for name, got, want in zip(("dwp", "dbp", "dwg", "dbg"), (dwp, dbp, dwg, dbg), sums):
         assert_close(name, got, want, tol)
+
+
+# Row counts around the fused backward's block and tile structure at K = N: one tile and one more
+# row, then 1, 2, 3, 4 and 5 tiles per block (its loops run four steps at a time).
+FUSED_ROWS = [(64, 128), (65, 128), (256 * 64 + 1, 128), (3 * 256 * 64 - 63, 128),
+              (4 * 256 * 64 + 130, 128), (130, 64), (512 * 64 * 2 + 7, 64)]
+
+
+@pytest.mark.parametrize("m,k", FUSED_ROWS)
+def test_gdp_bwd_fused_tiles(cuda, m, k):
+    """Every gradient against the oracle, with dx added into an existing one."""
+    dt = torch.bfloat16
+    li = layer_norm_inputs(m, k, dt, seed=m + k, device=cuda)
+    w = [t.to(cuda) for t in gdp_weights(k, k, dt, seed=k, bias_std=0.3)]
+    g = torch.Generator(device=cuda).manual_seed(m)
+    dout = torch.randn((m, k), generator=g, device=cuda).to(dt)
+    prev = torch.randn((m, k), generator=g, device=cuda).to(dt)
+    got = ops.gated_dual_proj_bwd(li["x"], *w, li["mask"], dout, dx=prev.clone())
+    r = list(ref.gated_dual_proj_bwd(np64(li["x"]), *(np64(t) for t in w), np64(li["mask"]),
+                                     np64(dout)))
+    r[0] = r[0] + np64(prev)
+    for name, a, b in zip(("dx", "dwp", "dbp", "dwg", "dbg"), got, r):
+        assert_close(name, a, b, TOL["bf16"]["grad"])
+
+
+def _offset_by_one(t):
+    """A contiguous copy of t one element past a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 8, device=t.device, dtype=t.dtype)
+    buf[1:1 + t.numel()] = t.reshape(-1)
+    return buf[1:1 + t.numel()].view(t.shape)
+
+
+@pytest.mark.parametrize("c,n", [(128, 128), (64, 64), (128, 64), (32, 32), (96, 32), (32, 128)])
+def test_ln_gdp_weights_at_any_alignment(cuda, c, n):
+    """Weights, biases and LayerNorm parameters need no alignment: the same bits one element past
+    a 16-byte boundary."""
+    dt = torch.bfloat16
+    li = layer_norm_inputs(130, c, dt, seed=c + n, device=cuda)
+    wa, wb = ([t.to(cuda) for t in gdp_weights(c, n, dt, seed=s, bias_std=0.3)] for s in (1, 2))
+    a, b = ops.ln_gated_dual_proj(li["x"], li["scale"], li["offset"], wa, wb, li["mask"])
+    off = lambda ts: [_offset_by_one(t) for t in ts]  # noqa: E731
+    a2, b2 = ops.ln_gated_dual_proj(li["x"], *off((li["scale"], li["offset"])), off(wa), off(wb),
+                                    _offset_by_one(li["mask"]))
+    assert torch.equal(a, a2) and torch.equal(b, b2)
