@@ -265,7 +265,6 @@ __global__ __launch_bounds__(6 * N) __attribute__((amdgpu_waves_per_eu(3))) void
     constexpr int K = N, W2 = 2 * N, NW = N / 32, R = kBwdRows, SUB = R / 16;
     constexpr int KS = K / 32, KS2 = W2 / 32;
     using S = SwzRows<K>;
-    using S2 = SwzRows<W2>;
     constexpr int XB = R * K * 2, TB = R * W2 * 2;
     constexpr int DPW = R * S::PL / (64 * NW);  // x loads per dW lane and tile
     constexpr int WK = K / 64, WN = NW / WK;    // dW waves along k (64 each) and n'
@@ -295,6 +294,17 @@ __global__ __launch_bounds__(6 * N) __attribute__((amdgpu_waves_per_eu(3))) void
         const int t = tile_of(j), rows = j < mine ? min(R, M - t * R) : 0;
         return buffer_rsrc(rows > 0 ? base + (size_t)t * R * W : base, (uint32_t)rows * W * 2);
     };
+
+    // Byte offsets of the lane's row operand in a tile of 16-byte pieces at piece ^ (row & 7): row
+    // 16*sub + r16, piece 4ks + g. Two lane offsets (ks even, odd) serve a tile with immediate
+    // offsets (a spilled address would be reloaded behind the row loads in flight).
+    int rx[2], rt[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int at = 16 * ((4 * q + g) ^ (r16 & 7));
+        rx[q] = r16 * (2 * K) + at;
+        rt[q] = r16 * (2 * W2) + at;
+    }
 
     if (wave < NW) {
         // ---- grad waves ----
@@ -334,13 +344,14 @@ __global__ __launch_bounds__(6 * N) __attribute__((amdgpu_waves_per_eu(3))) void
             dv[sub] = __builtin_amdgcn_raw_buffer_load_b128(rd, (row * N + col0) * 2, 0, 0);
             mv[sub] = __builtin_amdgcn_raw_buffer_load_b16(rm, row * 2, 0, 0);
         };
+        // The lane's piece of dp (of dg: 2*N bytes on) in row 16*sub + r16 of the gradient tile.
+        const int wt = r16 * (2 * W2) + 16 * ((4 * wave + g) ^ (r16 & 7));
         auto step = [&](int j, const char* xc, char* tw) {
             lds_barrier();  // x tile j in xc; the dx and dW waves are done with tw
             if (j >= mine) return;
             const Rsrc rd = tile_rsrc(dout, N, j + 1), rm = tile_rsrc(mask, 1, j + 1);
 #pragma unroll
             for (int sub = 0; sub < SUB; ++sub) {
-                const int row = 16 * sub + r16;
                 f32x4 acc[2][2];
 #pragma unroll
                 for (int mat = 0; mat < 2; ++mat)
@@ -348,8 +359,8 @@ __global__ __launch_bounds__(6 * N) __attribute__((amdgpu_waves_per_eu(3))) void
                     for (int h = 0; h < 2; ++h) acc[mat][h] = binit[mat][h];
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
-                    const V8 xv =
-                        *reinterpret_cast<const V8*>(xc + S::piece_at(row, 4 * ks + g) * 16);
+                    const V8 xv = *reinterpret_cast<const V8*>(xc + rx[ks & 1] + (ks >> 1) * 128 +
+                                                               sub * 16 * (2 * K));
 #pragma unroll
                     for (int mat = 0; mat < 2; ++mat)
 #pragma unroll
@@ -370,9 +381,9 @@ __global__ __launch_bounds__(6 * N) __attribute__((amdgpu_waves_per_eu(3))) void
                     cs[0][j8] += dp[j8];
                     cs[1][j8] += dg[j8];
                 }
-                *reinterpret_cast<u32x4*>(tw + S2::piece_at(row, col0 / 8) * 16) = pack8<TR>(dp);
-                *reinterpret_cast<u32x4*>(tw + S2::piece_at(row, (N + col0) / 8) * 16) =
-                    pack8<TR>(dg);
+                char* const at = tw + wt + sub * 16 * (2 * W2);
+                *reinterpret_cast<u32x4*>(at) = pack8<TR>(dp);
+                *reinterpret_cast<u32x4*>(at + 2 * N) = pack8<TR>(dg);
             }
         };
 #pragma unroll
@@ -432,8 +443,8 @@ __global__ __launch_bounds__(6 * N) __attribute__((amdgpu_waves_per_eu(3))) void
                 f32x4 da[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
                 for (int ks = 0; ks < KS2; ++ks) {
-                    const V8 v =
-                        *reinterpret_cast<const V8*>(tp + S2::piece_at(row, 4 * ks + g) * 16);
+                    const V8 v = *reinterpret_cast<const V8*>(tp + rt[ks & 1] + (ks >> 1) * 128 +
+                                                              sub * 16 * (2 * W2));
 #pragma unroll
                     for (int h = 0; h < 2; ++h) da[h] = TR::mfma(wd[h][ks], v, da[h]);
                 }
@@ -471,9 +482,9 @@ __global__ __launch_bounds__(6 * N) __attribute__((amdgpu_waves_per_eu(3))) void
         // Transposed operand: lane (r16, g) gets column 16a + r16 of rows ms + 8g .. + 7 (two 4-row
         // reads). Its pieces 2a + (r16 & 3)/2 of rows r and r + 4 sit at piece ^ (r & 7), so four
         // lane offsets (a % 4) serve a whole tile with immediate offsets: the upper read of a is
-        // the lower one of a ^ 2 four rows on. Formed from an opaque lane index: held in registers
-        // across the steps they would spill.
-        int lr = lane;
+        // the lower one of a ^ 2 four rows on. Formed in every step, from a lane index that is itself
+        // counted anew: held across the steps they spill, and a reload waits for the x loads.
+        int lr = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
         asm volatile("" : "+v"(lr));
         const int m = (lr >> 2) & 3, trow = 8 * (lr >> 4) + m;
         int xo[4], to[4];
