@@ -2,17 +2,17 @@
 // Replaces VoltaMma (cuda/volta_mma_attn.cu:70-351) and VoltaWmma (cuda/volta_wmma_attn.cu:
 // 47-311) with one kernel for f16 and bf16 on MFMA 16x16x32 with float32 accumulation.
 //
-// Work split: a block of 4 waves owns (query tile of 64*QT rows, head h, row n); each wave owns
-// 16*QT queries and streams the keys in tiles of 64 through double-buffered LDS: tile kt+1 is
-// fetched with direct global->LDS loads (K, V and the bias rows) while tile kt is computed, so
-// each tile costs one barrier. Which tiles contain an absent key is worked out once per block
-// from the mask row; the others skip the mask entirely.
+// Work split: a block of 4 waves owns (query tile of 64*QT rows, head h, row n), QT chosen by
+// fwd_small_blocks; each wave owns 16*QT queries and streams the keys in tiles of 64 through
+// double-buffered LDS: tile kt+1 is fetched with direct global->LDS loads (K, V and the bias
+// rows) while tile kt is computed, so each tile costs one barrier. Which tiles contain an absent
+// key is worked out once per block from the mask row; the others skip the mask entirely.
 //
 // Any even Sk, and any odd one (by query parity, the ODD form below), loads its bias through LDS.
 // Reading bias and mask element by element, as a ragged Sk once did, left the kernel waiting on
 // sixteen 2-byte loads per lane and tile: triangle attention of 757 residues (4 heads x 32)
 // 2395 -> 550 us, 1024 sequences of 300 residues (8 heads x 8) 965 -> 292 us, 203 residues
-// 65 -> 29 us. That path remains for what the direct loads cannot take (launch_fwd_qt).
+// 65 -> 29 us. That path remains for what the direct loads cannot take (fwd_form).
 //
 // Per 64-key tile and 16-query sub-tile a wave computes S^T = K . Q^T with the keys of each
 // 32-key chunk permuted so that lane l's accumulator holds keys 8*(l/16)+0..7 of the chunk for
@@ -739,23 +739,57 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     }
 }
 
+// How a call's bias reaches the kernel.
+struct FwdForm {
+    BiasMfma bm{};
+    bool bmf, odd, vec;
+};
+
+// The bias tile through LDS (vec: direct loads of 4-byte aligned pieces): at most kPresWords key
+// tiles (masked bias tiles are changed in LDS from presence words kept there). An even Sk
+// aligns every bias row. An odd one takes the parity form of the bias-MFMA kernel, when the
+// bias is a whole number of dwords (no load then reaches past its end). Other odd cases
+// (scale <= 0, one head or an odd number of them with an odd Sq) and longer rows read bias and
+// mask element by element, about four times slower (2395 against 550 us at 757 residues).
+template <typename TR>
+FwdForm fwd_form(int H, int Sq, int Sk, float scale) {
+    FwdForm f;
+    f.bmf = bias_mfma_for<TR>(scale, &f.bm);
+    const bool odd = Sk % 2 && f.bmf && (size_t)H * Sq * Sk % 2 == 0;
+    f.vec = (Sk % 2 == 0 || odd) && Sk + (odd ? 1 : 0) <= kPresWords * 64;
+    f.odd = f.vec && odd;
+    return f;
+}
+
+// Query blocks of one (row, head) at 64*QT queries each.
+int fwd_qtiles(const FwdForm& f, int Sq, int QT) {
+    return f.odd ? 2 * ceil_div((Sq + 1) / 2, 64 * QT) : ceil_div(Sq, 64 * QT);
+}
+
+// Queries per block: 64 (one 16-query sub-tile a wave) or 128 (two, which share each K, V and
+// presence read). Per query the smaller block costs 0-3% more time at D <= 16, 10% at D = 32 and
+// 40% at D = 64, so it is taken (us, smaller against larger block, bf16)
+//  - where its finer rounding saves more than that: an odd number m of 64-query tiles (m + 1 are
+//    run otherwise) at D <= 16, and m <= 7 at D = 32. D = 8, 300 queries 270 against 297; D = 16,
+//    300 38.6 against 47.5, 400 83 against 99; D = 32, 192 15.8 / 17.1, 300 47.4 / 50.8, 400
+//    110.4 / 111.9, but 704 116 / 114. An even m: 512 135 / 137 at D = 16, 182 / 163 at D = 32.
+//  - where all the smaller blocks are resident at once, so that a call lasts one block and half
+//    the block is nearly half the time: 4 per CU, 2 at D = 64 (gated, D = 32, 1024 blocks 11.9
+//    against 15.0, but 1536 16.7 / 15.3; D = 64, 512 blocks 13.1 / 15.7, but 768 17.4 / 15.8).
+bool fwd_small_blocks(const FwdForm& f, int D, int64_t NH, int Sq) {
+    if (Sq <= 64) return true;
+    if (!f.vec) return false;
+    const int m = fwd_qtiles(f, Sq, 1);
+    if (NH * m <= (D == 64 ? 512 : 1024)) return true;
+    return m < 2 * fwd_qtiles(f, Sq, 2) && (D <= 16 || (D == 32 && m <= 7));
+}
+
 template <typename TR, int D, int QT, bool GATE, bool NSHD>
 void launch_fwd_qt(hipStream_t st, const void* q, const void* k, const void* v, const void* bias,
                    const uint8_t* kmask, void* out, float* lse, int N, int H, int Sq, int Sk,
-                   float scale, GateArgs<typename TR::elem> ga) {
+                   float scale, GateArgs<typename TR::elem> ga, const FwdForm& f) {
     using E = typename TR::elem;
-    // The bias tile through LDS (direct loads of 4-byte aligned pieces): at most kPresWords key
-    // tiles (masked bias tiles are changed in LDS from presence words kept there). An even Sk
-    // aligns every bias row. An odd one takes the parity form of the bias-MFMA kernel, when the
-    // bias is a whole number of dwords (no load then reaches past its end). Other odd cases
-    // (scale <= 0, one head or an odd number of them with an odd Sq) and longer rows read bias and
-    // mask element by element, about four times slower (2395 against 550 us at 757 residues).
-    BiasMfma bm{};
-    const bool bmf = bias_mfma_for<TR>(scale, &bm);
-    const bool odd = Sk % 2 && bmf && (size_t)H * Sq * Sk % 2 == 0;
-    const bool vec = (Sk % 2 == 0 || odd) && Sk + (odd ? 1 : 0) <= kPresWords * 64;
-    const int BQ = 64 * QT;
-    const int qtiles = vec && odd ? 2 * ceil_div((Sq + 1) / 2, BQ) : ceil_div(Sq, BQ);
+    const int qtiles = fwd_qtiles(f, Sq, QT);
     const dim3 grid(qtiles * H * N);
     // The head-outer work-item order when the bias of all heads passes half of an XCD's 4 MB L2,
     // in groups of rows whose query tiles make about 48 work items, half an XCD's resident
@@ -766,13 +800,13 @@ void launch_fwd_qt(hipStream_t st, const void* q, const void* k, const void* v, 
     const int grp = head_outer ? max(1, min(N, 48 / qtiles)) : 0;
     auto run = [&](auto kernel) {
         kernel<<<grid, 256, 0, st>>>((const E*)q, (const E*)k, (const E*)v, (const E*)bias, kmask,
-                                     (E*)out, lse, H, Sq, Sk, scale, ga, bm, grp);
+                                     (E*)out, lse, H, Sq, Sk, scale, ga, f.bm, grp);
     };
-    if (vec && odd)
+    if (f.odd)
         run(attn_fwd_kernel<TR, D, QT, true, GATE, true, NSHD, true>);
-    else if (vec && bmf)
+    else if (f.vec && f.bmf)
         run(attn_fwd_kernel<TR, D, QT, true, GATE, true, NSHD, false>);
-    else if (vec)
+    else if (f.vec)
         run(attn_fwd_kernel<TR, D, QT, true, GATE, false, NSHD, false>);
     else
         run(attn_fwd_kernel<TR, D, QT, false, GATE, false, NSHD, false>);
@@ -783,24 +817,24 @@ void launch_fwd(hipStream_t st, const void* q, const void* k, const void* v, con
                 const uint8_t* kmask, void* out, float* lse, int N, int H, int Sq, int Sk,
                 float scale, GateArgs<typename TR::elem> ga, int nshd) {
     KernelTimer timer(GATE ? "attn_fwd_gated" : "attn_fwd", st);
+    const FwdForm f = fwd_form<TR>(H, Sq, Sk, scale);
+    const bool small = fwd_small_blocks(f, D, (int64_t)N * H, Sq);
+    auto launch = [&](auto qt, auto rows_nshd) {
+        launch_fwd_qt<TR, D, decltype(qt)::value, GATE, decltype(rows_nshd)::value>(
+            st, q, k, v, bias, kmask, out, lse, N, H, Sq, Sk, scale, ga, f);
+    };
+    using One = std::integral_constant<int, 1>;
+    using Two = std::integral_constant<int, 2>;
     // The [N, S, H, D] layout only for the ungated forward.
     if constexpr (!GATE) {
         if (nshd) {
-            if (Sq <= 64)
-                launch_fwd_qt<TR, D, 1, GATE, true>(st, q, k, v, bias, kmask, out, lse, N, H, Sq,
-                                                    Sk, scale, ga);
-            else
-                launch_fwd_qt<TR, D, 2, GATE, true>(st, q, k, v, bias, kmask, out, lse, N, H, Sq,
-                                                    Sk, scale, ga);
+            if (small) launch(One{}, std::true_type{});
+            else launch(Two{}, std::true_type{});
             return;
         }
     }
-    if (Sq <= 64)
-        launch_fwd_qt<TR, D, 1, GATE, false>(st, q, k, v, bias, kmask, out, lse, N, H, Sq, Sk,
-                                             scale, ga);
-    else
-        launch_fwd_qt<TR, D, 2, GATE, false>(st, q, k, v, bias, kmask, out, lse, N, H, Sq, Sk,
-                                             scale, ga);
+    if (small) launch(One{}, std::false_type{});
+    else launch(Two{}, std::false_type{});
 }
 
 template <typename TR, bool GATE>

@@ -314,3 +314,35 @@ def test_attention_fwd_ragged_keys(cuda, shape, dtype):
     neg = {**inp, "scale": -inp["scale"]}
     out_n = ops.attention(g["q"], g["k"], g["v"], g["bias"], g["kmask"], neg["scale"])
     assert_close("O (negative scale)", out_n, _oracle(neg)[0], TOL[dname(dtype)]["o"])
+
+
+# (Sq, Sk, D): one and two 64-query tiles past a block, odd and even numbers of tiles (odd ones
+# round up to two per block in the larger blocks), both key parities, every head dim.
+BLOCK_SHAPES = [(65, 66, 32), (128, 128, 16), (127, 129, 32), (130, 70, 64), (250, 96, 8),
+                (193, 192, 32), (257, 64, 64), (300, 300, 16), (300, 65, 8), (513, 64, 32)]
+
+
+@pytest.mark.parametrize("shape", BLOCK_SHAPES, ids=lambda c: "x".join(map(str, c)))
+def test_attention_fwd_query_block_choice(cuda, shape):
+    """Few rows run 64-query blocks, many rows the size that suits the shape: the same bits for
+    every row either way, in both layouts and gated; the few rows against the oracle."""
+    sq, sk, d = shape
+    n, h = 5, 2
+    inp = attention_inputs(n, h, sq, sk, d, torch.bfloat16, seed=sq + sk, masked_tail=0.2,
+                           masked_rows=1, with_dout=False)
+    x, wg, bg = (t.to(cuda) for t in gate_inputs(n, sq, 64, h * d, torch.bfloat16, seed=sk))
+    g = {k: (v.to(cuda) if isinstance(v, torch.Tensor) else v) for k, v in inp.items()}
+    out, lse = ops.attention_fwd(g["q"], g["k"], g["v"], g["bias"], g["kmask"], g["scale"])
+    assert_close("O", out, _oracle(inp)[0], TOL["bf16"]["o"])
+    gated = ops.attention_gated(g["q"], g["k"], g["v"], g["bias"], g["kmask"], x, wg, bg,
+                                g["scale"])
+    reps = 1100 // (n * h * ((sq + 63) // 64)) + 1
+    many = [t.repeat(reps, *[1] * (t.dim() - 1)) for t in (g["q"], g["k"], g["v"], g["kmask"], x)]
+    q, k, v, km, xm = many
+    t = lambda a: a.transpose(1, 2).contiguous()  # noqa: E731
+    out_m, lse_m = ops.attention_fwd(q, k, v, g["bias"], km, g["scale"])
+    out_s = ops.attention_nshd(t(q), t(k), t(v), g["bias"], km, g["scale"])[0]
+    gated_m = ops.attention_gated(q, k, v, g["bias"], km, xm, wg, bg, g["scale"])
+    for name, got, want in (("O", out_m, out), ("lse", lse_m, lse), ("O nshd", t(out_s), out),
+                            ("gated", gated_m, gated)):
+        assert torch.equal(got.reshape(reps, *want.shape), want.expand(reps, *want.shape)), name
