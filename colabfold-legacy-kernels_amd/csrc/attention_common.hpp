@@ -193,19 +193,21 @@ struct SwzTile {
 // covers its S rows, so rows past S read zeros, as do the padding pieces of D < 16) into a
 // swizzled LDS tile. ROWS*PL must be a multiple of 64. Every thread of the block calls it;
 // completion is awaited with async_wait() before a barrier.
-template <int D, int ROWS, int NTHREADS>
+template <int D, int ROWS, int NTHREADS, bool SW = false>
 __device__ __forceinline__ void stage_rows(Rsrc r, int r0, char* lds) {
     using T = SwzTile<D>;
     constexpr int SLOTS = ROWS * T::PL;
     static_assert(SLOTS % 64 == 0, "tile must be whole wave instructions");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-    for (int b = wave * 64; b < SLOTS; b += NTHREADS) {
+    for (int i = 0; i < (SLOTS + NTHREADS - 1) / NTHREADS; ++i) {
+        const int b = wave * 64 + i * NTHREADS;
+        if (SLOTS % NTHREADS != 0 && b >= SLOTS) break;
         const int slot = b + lane;
         const int row = slot / T::PL;
         const int piece = (slot % T::PL) ^ T::swz(row);
         const int voff = piece < T::P ? (row * D + piece * 8) * 2 : kPastEnd;
-        buf_dma16(r, voff, r0 * D * 2, lds + b * 16);
+        buf_dma16(r, voff, r0 * D * 2, lds + (SW ? __builtin_amdgcn_readfirstlane(b) : b) * 16);
     }
 }
 
@@ -213,7 +215,7 @@ __device__ __forceinline__ void stage_rows(Rsrc r, int r0, char* lds) {
 // row-major matrix): row r of the resource starts at byte 2*r*ld. Rows past the resource read
 // zeros. `tid` is the thread's index in the block (taken as an argument so that a caller can
 // keep its offsets from being shared with, and kept live across, earlier code).
-template <int D, int ROWS, int NTHREADS>
+template <int D, int ROWS, int NTHREADS, bool SW = false>
 __device__ __forceinline__ void stage_rows_ld(Rsrc r, int r0, int ld, char* lds, int tid) {
     using T = SwzTile<D>;
     constexpr int SLOTS = ROWS * T::PL;
@@ -227,12 +229,12 @@ __device__ __forceinline__ void stage_rows_ld(Rsrc r, int r0, int ld, char* lds,
         const int row = slot / T::PL;
         const int piece = (slot % T::PL) ^ T::swz(row);
         const int voff = piece < T::P ? (row * ld + piece * 8) * 2 : kPastEnd;
-        buf_dma16(r, voff, r0 * ld * 2, lds + b * 16);
+        buf_dma16(r, voff, r0 * ld * 2, lds + (SW ? __builtin_amdgcn_readfirstlane(b) : b) * 16);
     }
 }
 
 // stage_rows_ld from a first row r0 that may be negative: rows below 0 read zeros.
-template <int D, int ROWS, int NTHREADS>
+template <int D, int ROWS, int NTHREADS, bool SW = false>
 __device__ __forceinline__ void stage_rows_from(Rsrc r, int r0, int ld, char* lds, int tid) {
     using T = SwzTile<D>;
     constexpr int SLOTS = ROWS * T::PL;
@@ -247,7 +249,7 @@ __device__ __forceinline__ void stage_rows_from(Rsrc r, int r0, int ld, char* ld
         const int piece = (slot % T::PL) ^ T::swz(row);
         const int voff = piece < T::P && r0 + row >= 0 ? ((r0 + row) * ld + piece * 8) * 2
                                                        : kPastEnd;
-        buf_dma16(r, voff, 0, lds + b * 16);
+        buf_dma16(r, voff, 0, lds + (SW ? __builtin_amdgcn_readfirstlane(b) : b) * 16);
     }
 }
 

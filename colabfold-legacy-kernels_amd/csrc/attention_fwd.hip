@@ -14,6 +14,14 @@
 // 2395 -> 550 us, 1024 sequences of 300 residues (8 heads x 8) 965 -> 292 us, 203 residues
 // 65 -> 29 us. That path remains for what the direct loads cannot take (fwd_form).
 //
+// A block runs only 5 to 16 key tiles, so what it does before and after them counts: of 22600
+// cycles at 384 residues, 4600 passed before the first tile was there (2500 before its loads went
+// out) and 1100 after the last. The work item comes from prepared multipliers, the arguments in
+// one round of scalar loads, the mask, Q and tile loads carry no branch (a row or key that does
+// not exist reads zero), and the presence words wait for the mask bytes alone: D = 32, 300
+// residues 47.2 -> 45.1 us, 384 72.2 -> 69.4, 757 537 -> 515; D = 16, 300 40.5 -> 36.9;
+// D = 64, 300 91.3 -> 85.5.
+//
 // Per 64-key tile and 16-query sub-tile a wave computes S^T = K . Q^T with the keys of each
 // 32-key chunk permuted so that lane l's accumulator holds keys 8*(l/16)+0..7 of the chunk for
 // query l%16. Those eight values are exactly the B operand of O^T = V^T . P^T for that chunk, so
@@ -145,6 +153,14 @@ struct GateArgs {
     int C, HD;
 };
 
+// A block's work item a * outer.d + b * inner.d + c from its index, the divisors prepared at
+// launch: (a, b, c) are (row, head, query tile), or with grp > 0 (head, group of rows, place in it).
+struct FwdItems {
+    FastDiv outer, inner;     // items of one a, of one b
+    FastDiv rows, last_rows;  // grp > 0: rows of a group, of the last group
+    int grp, nrows;
+};
+
 // ODD (VEC and BM): Sk is odd. The direct-to-LDS loads of the bias need 4-byte aligned addresses,
 // and every other bias row starts half a dword off. A block then owns queries of one parity
 // (query q0 + 2i for its i-th row), whose bias rows are all aligned or all off by one element;
@@ -157,7 +173,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     const typename TR::elem* __restrict__ v, const typename TR::elem* __restrict__ bias,
     const uint8_t* __restrict__ kmask, typename TR::elem* __restrict__ out,
     float* __restrict__ lse, int H, int Sq, int Sk, float scale,
-    GateArgs<typename TR::elem> ga, BiasMfma bm, int grp) {
+    GateArgs<typename TR::elem> ga, BiasMfma bm, FwdItems items) {
     static_assert(!BM || VEC, "the bias MFMA reads the bias tile from LDS");
     static_assert(!ODD || BM, "odd key counts run the bias-MFMA form");
     static_assert(!(NSHD && GATE), "the gated entry takes the [N, H, S, D] layout");
@@ -169,10 +185,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     // changed in LDS before use -- a large negative bias for an absent key (P = 0 after the
     // exponential once the row's max comes from a present key): the masked logit -1e9 in
     // bfloat16, float16's lowest value -65504 in float16 (the reference's own masked logit is
-    // -1e4); 0 for every key in range in a row without any present key (whose Q^T is zero, so
-    // every logit is that row's masked logit 0) -- and the scores need no per-key select, so the
-    // tile's MFMAs and exponentials stay one straight-line block. (No larger magnitude: the
-    // exponent's FMA against the running max leaves a rounding residue of about 2^-24 of the
+    // -1e4) -- and the scores need no per-key select, so the tile's MFMAs and exponentials stay
+    // one straight-line block. (A row without any present key computes no scores: tile_empty.)
+    // (No larger magnitude: the exponent's FMA against the running max leaves a rounding residue of about 2^-24 of the
     // logit, which must stay far below float32's exponent range.)
     constexpr bool PATCH = VEC;
     using PF = TilePrefetch<TR, QT>;
@@ -187,6 +202,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     __shared__ __attribute__((aligned(16))) char kv0[2 * TILE + BTILE];  // K rows, V rows, bias
     __shared__ __attribute__((aligned(16))) char kv1[2 * TILE + BTILE];
 
+    // The arguments of the set-up in one round of scalar loads: left to itself the compiler loads
+    // each where it is first needed, four rounds in a row before the first tile's loads go out.
+    asm volatile("" ::"s"(q), "s"(k), "s"(v), "s"(bias), "s"(kmask), "s"(H), "s"(Sq), "s"(Sk),
+                 "s"(items.outer.d), "s"(items.outer.m), "s"(items.outer.s), "s"(items.inner.d),
+                 "s"(items.inner.m), "s"(items.inner.s), "s"(items.grp), "s"(gridDim.x));
+
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, g = lane >> 4;
     // 1-D grid of (query tile, head, row) work items, placed so that each XCD runs a contiguous
@@ -198,32 +219,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     // blocks then read one head's bias rows (the same for every row n) and the K and V of a few
     // rows, both of which stay in its L2.
     // ODD: the even and the odd queries of a range of 2*BQ are neighbouring work items.
-    const int qtiles = QS * (((Sq + QS - 1) / QS + BQ - 1) / BQ);
     const int item = xcd_contiguous(blockIdx.x, gridDim.x);
-    int q0, h, n;
-    if (grp == 0) {
-        q0 = item % qtiles;
-        h = (item / qtiles) % H;
-        n = item / (qtiles * H);
-    } else {
-        const int nrows = gridDim.x / (qtiles * H), per_head = qtiles * nrows;
-        h = item / per_head;
-        const int rem = item - h * per_head;
-        const int gi = rem / (grp * qtiles), nb = gi * grp, gsz = min(grp, nrows - nb);
-        q0 = (rem - gi * grp * qtiles) / gsz;
-        n = nb + (rem - gi * grp * qtiles) % gsz;
+    const int a = div_by(item, items.outer), rem = item - a * items.outer.d;
+    const int b = div_by(rem, items.inner), at = rem - b * items.inner.d;
+    int q0 = at, h = b, n = a;  // grp == 0
+    if (items.grp > 0) {
+        const int nb = b * items.grp;
+        const FastDiv rows = items.nrows - nb < items.grp ? items.last_rows : items.rows;
+        h = a;
+        q0 = div_by(at, rows);
+        n = nb + at - q0 * rows.d;
     }
     q0 = ODD ? (q0 >> 1) * 2 * BQ + (q0 & 1) : q0 * BQ;
-    const size_t nh = (size_t)n * H + h;
+    const size_t nh = (uint32_t)(n * H + h);  // below 2^31 (validate_attention)
     // Rows of one (n, h) in q, k, v and out: [N, H, S, D] (rows D apart), or with NSHD
     // [N, S, H, D] (rows H*D apart, head h at column block h).
     const int ld = NSHD ? H * D : D;
-    const E* qp = q + (NSHD ? ((size_t)n * Sq * H + h) * D : nh * Sq * D);
-    const E* kp = k + (NSHD ? ((size_t)n * Sk * H + h) * D : nh * Sk * D);
-    const E* vp = v + (NSHD ? ((size_t)n * Sk * H + h) * D : nh * Sk * D);
-    E* const op = out ? out + (NSHD ? ((size_t)n * Sq * H + h) * D : nh * Sq * D) : nullptr;
-    const E* bp = bias + (size_t)h * Sq * Sk;
-    const uint8_t* mp = kmask ? kmask + (size_t)n * Sk : nullptr;
+    const E* qp = q + (NSHD ? ((size_t)n * Sq * H + h) * D : nh * (uint32_t)Sq * D);
+    const E* kp = k + (NSHD ? ((size_t)n * Sk * H + h) * D : nh * (uint32_t)Sk * D);
+    const E* vp = v + (NSHD ? ((size_t)n * Sk * H + h) * D : nh * (uint32_t)Sk * D);
+    E* const op = out ? out + (NSHD ? ((size_t)n * Sq * H + h) * D : nh * (uint32_t)Sq * D) : nullptr;
+    const E* bp = bias + (size_t)(uint32_t)h * (uint32_t)Sq * (uint32_t)Sk;
+    const uint8_t* mp = kmask ? kmask + (size_t)(uint32_t)n * (uint32_t)Sk : nullptr;
     const int qbase = q0 + wave * 16 * QT * QS;
     // Keys the block's tiles start before key 0 (0 or 1; every row of the block agrees).
     const int shift = ODD ? (h * Sq + q0) & 1 : 0;
@@ -238,7 +255,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     // first. Its end is rounded up to a dword (loads are range-checked by dword): for ODD the bias
     // of all heads is an even number of elements, so that dword lies inside it.
     const int brows = min(BQ, (Sq - q0 + QS - 1) / QS);
-    const Rsrc rb = buffer_rsrc(bp + (size_t)q0 * Sk - shift,
+    const Rsrc rb = buffer_rsrc(bp + (size_t)(uint32_t)q0 * (uint32_t)Sk - shift,
                                 brows > 0 ? (uint32_t)((((brows - 1) * QS * Sk + Sk + shift) * 2 + 3) & ~3)
                                           : 0u);
     // Head h's D columns of the gate weight: row c (channel) starts HD elements after row c-1.
@@ -246,54 +263,57 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
                          : rb;
     auto stage = [&](int k0, char* kv) {
         if (ODD && k0 == 0) {  // row -1 (shift = 1) reads zeros
-            stage_rows_from<D, BK, 256>(rk, -shift, ld, kv, threadIdx.x);
-            stage_rows_from<D, BK, 256>(rv, -shift, ld, kv + TILE, threadIdx.x);
+            stage_rows_from<D, BK, 256, true>(rk, -shift, ld, kv, threadIdx.x);
+            stage_rows_from<D, BK, 256, true>(rv, -shift, ld, kv + TILE, threadIdx.x);
         } else if constexpr (NSHD) {
-            stage_rows_ld<D, BK, 256>(rk, k0 - shift, ld, kv, threadIdx.x);
-            stage_rows_ld<D, BK, 256>(rv, k0 - shift, ld, kv + TILE, threadIdx.x);
+            stage_rows_ld<D, BK, 256, true>(rk, k0 - shift, ld, kv, threadIdx.x);
+            stage_rows_ld<D, BK, 256, true>(rv, k0 - shift, ld, kv + TILE, threadIdx.x);
         } else {
-            stage_rows<D, BK, 256>(rk, k0 - shift, kv);
-            stage_rows<D, BK, 256>(rv, k0 - shift, kv + TILE);
+            stage_rows<D, BK, 256, true>(rk, k0 - shift, kv);
+            stage_rows<D, BK, 256, true>(rv, k0 - shift, kv + TILE);
         }
         if constexpr (VEC) {
             // The block's bias rows, keys k0 - shift .. + 63 as eight 16-byte pieces per row; piece
             // p of row r sits at position p ^ (r & 7), so a 16-row operand read is conflict-free.
             // Rows past Sq read zeros; keys past Sk (last tile) and key -1 read what lies there,
             // and are patched.
+            const int row = threadIdx.x >> 3, piece = (threadIdx.x & 7) ^ (row & 7);
+            const int voff = (row * QS * Sk + 8 * piece) * 2;
+            // The later loads' offsets as sums with an opaque zero: held in registers through the
+            // loop they cost the kernel two spilled ones.
+            int step = 64 * QS * Sk;
+            asm volatile("" : "+s"(step));
+            char* const dst = kv + 2 * TILE + __builtin_amdgcn_readfirstlane(wave) * 1024;
 #pragma unroll
-            for (int b = wave * 64; b < BQ * 8; b += 256) {
-                const int slot = b + lane;
-                const int row = slot >> 3, piece = (slot & 7) ^ (row & 7);
-                buf_dma16(rb, (row * QS * Sk + 8 * piece) * 2, k0 * 2, kv + 2 * TILE + b * 16);
-            }
+            for (int i = 0; i < BQ * 8 / 256; ++i)
+                buf_dma16(rb, voff + i * step, k0 * 2, dst + i * 4096);
         }
     };
-    // PATCH: this wave's mask bytes of its first two key tiles (t = wave, wave + 4; lane l:
-    // key 64t + l - shift), loaded before anything else so that the presence words below wait for them
-    // alone.
-    uint32_t mb[2] = {0u, 0u};
+    // PATCH: this wave's mask bytes of its first kPre key tiles (t = wave + 4*i; lane l: key
+    // 64t + l - shift), loaded before anything else so that the presence words below wait for
+    // them alone. Out of range (key -1 too, a negative offset) reads zero.
+    constexpr int kPre = 4;
+    uint32_t mb[kPre];
     if constexpr (PATCH) {
+        const Rsrc rm = buffer_rsrc(mp ? (const void*)mp : (const void*)bp, mp ? (uint32_t)Sk : 0u);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int kk = (wave + 4 * i) * BK + lane - shift;
-            if (kk >= 0 && kk < Sk) mb[i] = mp ? mp[kk] : 1u;
-        }
+        for (int i = 0; i < kPre; ++i) mb[i] = buf_ld1(rm, (wave + 4 * i) * BK + lane - shift);
     }
-    if (ntiles > 0) stage(0, kv0);
-
     // B operand Q^T: lane (query r16, group g) holds head dims 32*ks + 8*g + 0..7.
     V8 qf[QT][G::KS];
+    const Rsrc rq = buffer_rsrc(qp, NSHD ? (uint32_t)(((size_t)(Sq - 1) * ld + D) * 2)
+                                         : (uint32_t)Sq * D * 2);
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         const int row = qbase + (qt * 16 + r16) * QS;
 #pragma unroll
         for (int ks = 0; ks < G::KS; ++ks) {
             const int d0 = ks * 32 + g * 8;
-            u32x4 raw = {0u, 0u, 0u, 0u};
-            if (row < Sq && d0 < D) raw = ld16(qp + (size_t)row * ld + d0);
-            qf[qt][ks] = bits_as<V8>(raw);
+            qf[qt][ks] = bits_as<V8>(buf_ld16(rq, d0 < D ? (row * ld + d0) * 2 : kPastEnd));
         }
     }
+    // (With no keys at all the resources are empty and the tile reads zeros.)
+    stage(0, kv0);
 
     // Not PATCH: bias rows of the lane's queries (clamped inside [0, Sq)), keys 32c + 8g + 0..7
     // per tile.
@@ -313,15 +333,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     if constexpr (PATCH) {
         int last = 0;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int t = wave + 4 * i;
-            if (t < ntiles) {
-                const unsigned long long b = __ballot(mb[i] != 0u);
-                if (b != 0ull) last = t + 1;
-                if (lane == 0) pres[t] = b;
-            }
+        for (int i = 0; i < kPre; ++i) {
+            const int t = wave + 4 * i, kk = t * BK + lane - shift;
+            const unsigned long long b = __ballot(mp ? mb[i] != 0u : kk >= 0 && kk < Sk);
+            if (b != 0ull) last = t + 1;
+            if (lane == 0) pres[t] = b;  // (past the last tile: no key, a zero nobody reads)
         }
-        for (int t = wave + 8; t < ntiles; t += 4) {
+        for (int t = wave + 4 * kPre; t < ntiles; t += 4) {
             const int kk = t * BK + lane - shift;
             const unsigned long long b = __ballot(kk < Sk && (mp == nullptr || mp[kk] != 0));
             if (b != 0ull) last = t + 1;
@@ -329,23 +347,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
         }
         if (lane == 0) wave_last[wave] = last;
     }
-    // PATCH: a row without any present key: every logit is its masked logit 0, so Q^T = 0 and
-    // the changed bias tiles hold 0 in range. Otherwise the key tiles after the row's last
-    // present key (a padding tail) add P = 0 to O and l and are not run at all: after the row's
-    // max is set their P underflows to 0.
+    // PATCH: a row without any present key runs tile_empty below. Otherwise the key tiles after
+    // the row's last present key (a padding tail) add P = 0 to O and l and are not run at all:
+    // after the row's max is set their P underflows to 0.
     bool row_empty = false;
     int nrun = ntiles;  // key tiles the loop runs
     if constexpr (PATCH) {
-        __syncthreads();  // the presence words and counts are visible
+        lds_barrier();  // the presence words and counts are visible (the loads stay in flight)
         const int last = max(max(wave_last[0], wave_last[1]), max(wave_last[2], wave_last[3]));
         row_empty = mp && last == 0;
         if (!row_empty) nrun = last;
-        if (row_empty) {
-#pragma unroll
-            for (int qt = 0; qt < QT; ++qt)
-#pragma unroll
-                for (int ks = 0; ks < G::KS; ++ks) qf[qt][ks] = V8{};
-        }
     }
     // PATCH: lane (row r16 of each sub-tile, group g) changes 16-byte pieces 4c + g (keys
     // k0 + 32c + 8g + 0..7) of its rows of tile kt's bias: all its pieces are read, changed and
@@ -391,10 +402,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     // 8g .. 8g+7, so its one nonzero is element r16 % 8 when g % 2 == r16 / 8.
     V8 idn;
     if constexpr (BM) {
+        const uint32_t v = (uint32_t)__builtin_bit_cast(uint16_t, TR::from_f(g < 2 ? bm.hi : bm.lo))
+                           << (16 * (r16 & 1));
+        const int at = (g & 1) == (r16 >> 3) ? (r16 & 7) >> 1 : -1;
+        u32x4 bits;
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-            idn[j] = TR::from_f((j == (r16 & 7) && (g & 1) == (r16 >> 3)) ? (g < 2 ? bm.hi : bm.lo)
-                                                                      : 0.f);
+        for (int i = 0; i < 4; ++i) bits[i] = i == at ? v : 0u;
+        idn = bits_as<V8>(bits);
     }
 
     // Running max, and O^T plus one extra accumulator per sub-tile: the MFMA of an all-ones
@@ -637,6 +651,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             tile(kt, kv0, kv1, ca, cb);
             if (kt + 1 < nrun) tile(kt + 1, kv1, kv0, cb, ca);
         }
+        if (nrun == 0) async_wait();  // no load into LDS outlives the block
     }
 
     // Gate pre-activations in O^T's accumulator layout (lane: rows 16*dt + 4*g + i of head h's
@@ -798,9 +813,16 @@ void launch_fwd_qt(hipStream_t st, const void* q, const void* k, const void* v, 
     // inside the row: the MSA shapes' gate rows and [N, S, H, D] rows are shared by the heads.
     const bool head_outer = (size_t)H * Sq * Sk * 2 > (2u << 20);
     const int grp = head_outer ? max(1, min(N, 48 / qtiles)) : 0;
+    FwdItems items{};
+    items.grp = grp;
+    items.nrows = N;
+    items.outer = fast_div(qtiles * (grp ? N : H));
+    items.inner = fast_div(qtiles * (grp ? grp : 1));
+    items.rows = fast_div(grp ? grp : 1);
+    items.last_rows = fast_div(grp && N % grp ? N % grp : max(1, grp));
     auto run = [&](auto kernel) {
         kernel<<<grid, 256, 0, st>>>((const E*)q, (const E*)k, (const E*)v, (const E*)bias, kmask,
-                                     (E*)out, lse, H, Sq, Sk, scale, ga, f.bm, grp);
+                                     (E*)out, lse, H, Sq, Sk, scale, ga, f.bm, items);
     };
     if (f.odd)
         run(attn_fwd_kernel<TR, D, QT, true, GATE, true, NSHD, true>);

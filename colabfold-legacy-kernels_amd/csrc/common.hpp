@@ -221,6 +221,15 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
+// Buffer loads of 16 bytes and of one byte: zero where the offset falls past the resource's range,
+// so a row that does not exist takes no branch (and the loads around it stay countable).
+__device__ __forceinline__ u32x4 buf_ld16(Rsrc r, int voff) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0);
+}
+__device__ __forceinline__ uint32_t buf_ld1(Rsrc r, int voff) {
+    return __builtin_amdgcn_raw_buffer_load_b8(r, voff, 0, 0);
+}
+
 // 16-byte buffer store; a store whose offset falls past the resource's range is dropped.
 __device__ __forceinline__ void buf_st16(Rsrc r, int voff, int soff, u32x4 v) {
     __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, soff, 0);
@@ -325,9 +334,24 @@ __device__ __forceinline__ float group_sum(float v) {
 // of [0, T): results never depend on it, only the L2 hit rate does.
 constexpr int kXcds = 8;
 __device__ __forceinline__ int xcd_contiguous(int L, int T) {
-    const int xcd = L % kXcds, slot = L / kXcds;
-    const int per = T / kXcds, rem = T % kXcds;
+    const int xcd = (unsigned)L % kXcds, slot = (unsigned)L / kXcds;
+    const int per = (unsigned)T / kXcds, rem = (unsigned)T % kXcds;
     return xcd * per + min(xcd, rem) + slot;
+}
+
+// Division of 0 <= n < 2^31 by a divisor fixed at launch, as a multiply and a shift: with
+// 2^s >= d and m = ceil(2^(31+s) / d), n*m / 2^(31+s) exceeds n/d by less than 1/d. (A division
+// by a kernel argument is some 25 dependent scalar instructions.)
+struct FastDiv {
+    uint32_t d, m, s;
+};
+inline FastDiv fast_div(uint32_t d) {
+    uint32_t s = 0;
+    while ((1ull << s) < d) ++s;
+    return {d, (uint32_t)(((1ull << (31 + s)) + d - 1) / d), s};
+}
+__device__ __forceinline__ uint32_t div_by(uint32_t n, FastDiv f) {
+    return __umulhi(2 * n, f.m) >> f.s;
 }
 
 // The pair positions (i, j) of an n x n grid as the rows of a zero-padded np x np one, np = n
