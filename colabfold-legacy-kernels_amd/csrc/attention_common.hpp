@@ -270,12 +270,12 @@ struct HeadRows {
 };
 
 // stage_rows over the rows of one (n, h) in either layout (`r` from HeadRows' offset and bytes).
-template <int D, int ROWS, int NTHREADS, bool NSHD>
+template <int D, int ROWS, int NTHREADS, bool NSHD, bool SW = false>
 __device__ __forceinline__ void stage_head_rows(Rsrc r, int r0, int H, char* lds) {
     if constexpr (NSHD)
-        stage_rows_ld<D, ROWS, NTHREADS>(r, r0, H * D, lds, threadIdx.x);
+        stage_rows_ld<D, ROWS, NTHREADS, SW>(r, r0, H * D, lds, threadIdx.x);
     else
-        stage_rows<D, ROWS, NTHREADS>(r, r0, lds);
+        stage_rows<D, ROWS, NTHREADS, SW>(r, r0, lds);
 }
 
 // Row operand from a swizzled tile: row `row`, head dims 32*ks + 8*g + 0..7 (zero beyond D).

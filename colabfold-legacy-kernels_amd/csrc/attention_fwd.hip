@@ -309,7 +309,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
 #pragma unroll
         for (int ks = 0; ks < G::KS; ++ks) {
             const int d0 = ks * 32 + g * 8;
-            qf[qt][ks] = bits_as<V8>(buf_ld16(rq, d0 < D ? (row * ld + d0) * 2 : kPastEnd));
+            qf[qt][ks] = bits_as<V8>(buf_ld16(rq, d0 < D ? (row * ld + d0) * 2 : kNoRow));
         }
     }
     // (With no keys at all the resources are empty and the tile reads zeros.)

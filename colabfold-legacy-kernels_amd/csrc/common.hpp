@@ -184,6 +184,8 @@ __device__ __forceinline__ Rsrc buffer_rsrc(const void* base, uint32_t bytes) {
 }
 // A per-lane offset that every slice resource treats as out of range (resources cover < 2^30).
 constexpr int kPastEnd = 1 << 30;
+// The same for resources of up to 2^31 bytes (for loads without a scalar offset).
+constexpr int kNoRow = -(1 << 30);
 
 // Direct buffer->LDS loads: lane i's 16 (4) bytes at byte voff + soff of the resource land at
 // lds_window + 16*i (4*i); lds_window must be wave-uniform.
@@ -221,10 +223,13 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
-// Buffer loads of 16 bytes and of one byte: zero where the offset falls past the resource's range,
+// Buffer loads of 16, 4 and 1 bytes: zero where the offset falls past the resource's range,
 // so a row that does not exist takes no branch (and the loads around it stay countable).
 __device__ __forceinline__ u32x4 buf_ld16(Rsrc r, int voff) {
     return __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0);
+}
+__device__ __forceinline__ uint32_t buf_ld4(Rsrc r, int voff) {
+    return __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0);
 }
 __device__ __forceinline__ uint32_t buf_ld1(Rsrc r, int voff) {
     return __builtin_amdgcn_raw_buffer_load_b8(r, voff, 0, 0);
