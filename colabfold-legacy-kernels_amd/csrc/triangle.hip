@@ -340,6 +340,65 @@ struct TriOutParams {
 
 // RAG: the positions are those of the padded grid (x's planes); z's and out's rows are addressed in
 // the caller's n x n grid, padded positions reading zeros and storing nothing.
+// LDS reads of the output stage's LayerNorms as single asm statements with their own wait. Issued
+// as plain reads, the compiler cannot tell the three staging buffers apart here and puts a wait for
+// the next tile's direct-to-LDS loads in front of them, so that only one tile was ever in flight
+// (at N = 512, C = 64 28.2 -> 24.4 us; at C = 128, where the arithmetic between two barriers takes
+// longer, 49.8 -> 48.9).
+//
+// Channel slab: lane (r16, g) of a wave gets four consecutive channels per pair of dwords,
+// NQ transposed reads of channels 4q .. 4q + 3 from the lane group's first (`at`: the lane's own
+// 8 bytes of the first read; rows of 128 bytes, 16 bytes of padding every eight).
+template <int NQ>
+__device__ __forceinline__ void slab_read(uint32_t at, uint32_t (&vp)[2 * NQ]) {
+    static_assert(NQ == 4 || NQ == 8, "C = 64 or 128");
+    u32x2 v[8];
+    if constexpr (NQ == 8)
+        asm volatile(
+            "ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %1, %8 offset:512\n\t"
+            "ds_read_b64_tr_b16 %2, %8 offset:1040\n\tds_read_b64_tr_b16 %3, %8 offset:1552\n\t"
+            "ds_read_b64_tr_b16 %4, %8 offset:2080\n\tds_read_b64_tr_b16 %5, %8 offset:2592\n\t"
+            "ds_read_b64_tr_b16 %6, %8 offset:3120\n\tds_read_b64_tr_b16 %7, %8 offset:3632\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]),
+              "=&v"(v[6]), "=&v"(v[7])
+            : "v"(at)
+            : "memory");
+    else
+        asm volatile(
+            "ds_read_b64_tr_b16 %0, %4\n\tds_read_b64_tr_b16 %1, %4 offset:512\n\t"
+            "ds_read_b64_tr_b16 %2, %4 offset:1040\n\tds_read_b64_tr_b16 %3, %4 offset:1552\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+            : "v"(at)
+            : "memory");
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        vp[2 * q] = v[q][0];
+        vp[2 * q + 1] = v[q][1];
+    }
+}
+// NP 16-byte pieces, 4096 bytes apart.
+template <int NP>
+__device__ __forceinline__ void rows_read(uint32_t at, u32x4 (&v)[NP]) {
+    static_assert(NP == 2 || NP == 4, "C = 64 or 128");
+    if constexpr (NP == 4)
+        asm volatile(
+            "ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:4096\n\t"
+            "ds_read_b128 %2, %4 offset:8192\n\tds_read_b128 %3, %4 offset:12288\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+            : "v"(at)
+            : "memory");
+    else
+        asm volatile(
+            "ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:4096\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(v[0]), "=&v"(v[1])
+            : "v"(at)
+            : "memory");
+}
+
 template <typename TR, int C, bool RAG>
 __global__ __launch_bounds__(512) void tri_out_kernel(TriOutParams<typename TR::elem> pr) {
     using E = typename TR::elem;
@@ -488,14 +547,11 @@ __global__ __launch_bounds__(512) void tri_out_kernel(TriOutParams<typename TR::
                 return TR::to_f(__builtin_bit_cast(E, (uint16_t)((j & 1) ? w2 >> 16 : w2)));
             };
             float sum = 0.f;
+            slab_read<CPG / 4>(lds_addr(xc) + (CPG * g + (r16 >> 2)) * (R * 2) + CPG / 8 * g * 16 +
+                                   (16 * wave + 4 * (r16 & 3)) * 2,
+                               vp);
 #pragma unroll
-            for (int j = 0; j < CPG; j += 2) {
-                const char* at = xc + (CPG * g + j) * (R * 2) + ((CPG * g + j) / 8) * 16 + p * 2;
-                const uint32_t lo = *reinterpret_cast<const uint16_t*>(at);
-                const uint32_t hi = *reinterpret_cast<const uint16_t*>(at + R * 2);
-                vp[j >> 1] = lo | (hi << 16);
-                sum += val(j) + val(j + 1);
-            }
+            for (int j = 0; j < CPG; j += 2) sum += val(j) + val(j + 1);
             const float mean = xgroup_sum(sum) * (1.f / C);
             float m2 = 0.f;
 #pragma unroll
@@ -517,11 +573,14 @@ __global__ __launch_bounds__(512) void tri_out_kernel(TriOutParams<typename TR::
             // LN_in over the z rows: LPR lanes per row, 8 channels each.
             const int lt = tid - 256, lr = lt % LPR;
             constexpr int RPP = 256 / LPR;
+            static_assert(RPP * C * 2 == 4096, "rows_read's step");
+            u32x4 zr[R / RPP];
+            rows_read<R / RPP>(lds_addr(zc) + lt * 16, zr);
 #pragma unroll
             for (int pass = 0; pass < R / RPP; ++pass) {
                 const int row = pass * RPP + lt / LPR;
                 float v[8];
-                unpack8<TR>(*reinterpret_cast<const u32x4*>(zc + row * C * 2 + lr * 16), v);
+                unpack8<TR>(zr[pass], v);
                 float sum = 0.f;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) sum += v[j];
