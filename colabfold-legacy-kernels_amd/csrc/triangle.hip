@@ -721,12 +721,17 @@ extern "C" clk_status clk_triangle_einsum(hipStream_t stream, clk_dtype dtype, c
 namespace {
 // N rounded up to a multiple of 8: a ragged N runs the module on a zero-padded grid.
 int64_t padded_n(int64_t N) { return (N + 7) / 8 * 8; }
+size_t round256(size_t v) { return (v + 255) / 256 * 256; }
 }  // namespace
 
 extern "C" size_t clk_triangle_multiply_workspace_size(int64_t N, int64_t C) {
     if (N <= 0 || C <= 0) return 0;
-    // left, right and x, channel-major [C][NP][NP].
-    return (size_t)3 * C * padded_n(N) * padded_n(N) * 2;
+    // left, right and x, channel-major [C][NP][NP]. The size of a ragged N is part of the
+    // interface (a smaller workspace is refused) and counts padded copies of z, the mask and the
+    // output as well; the kernels address the caller's rows and leave that part alone.
+    const size_t np = padded_n(N), planes = (size_t)C * np * np * 2;
+    if (N % 8 == 0) return 3 * planes;
+    return round256(3 * planes) + round256(planes) + round256(np * np * 2) + planes;
 }
 
 extern "C" clk_status clk_triangle_multiply(hipStream_t stream, clk_dtype dtype, const void* z,

@@ -310,7 +310,8 @@ clk_status clk_triangle_einsum(hipStream_t stream, clk_dtype dtype, const void* 
  * gate, each [C,C] row-major (input channel first); b[0..5] their [C] biases; ln[0..3] = LN_in
  * scale, offset, LN_c scale, offset (float32 [C]). z, mask, weights, biases and out of dtype
  * CLK_F16 or CLK_BF16. C = 64 or 128; N up to 16384. The workspace holds left, right and x
- * channel-major on a grid of N rounded up to 8, zero in the padding
+ * channel-major on a grid of N rounded up to 8, zero in the padding; for a ragged N its size
+ * also counts padded copies of z, mask and output, which are not written
  * (clk_triangle_multiply_workspace_size bytes).
  */
 size_t clk_triangle_multiply_workspace_size(int64_t N, int64_t C);
