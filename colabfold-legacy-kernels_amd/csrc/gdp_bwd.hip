@@ -1031,19 +1031,30 @@ struct BwdGeom {
 };
 
 // K == N: one fused kernel, so no dpg, and its blocks' partials are both the weights' and the
-// biases' (two 64 KB blocks share a CU at 64, one of 128 KB at 128).
+// biases' (two 64 KB blocks share a CU at 64, one of 128 KB at 128). The size is part of the
+// interface (a smaller workspace is refused) and that of the three-kernel form, dpg included; the
+// partials of the fused kernel's blocks fit it but for one block in some 500 at K = N = 64.
 BwdGeom bwd_geom(int64_t M, int K, int N) {
     BwdGeom g;
     const int64_t ntiles = (M + kBwdRows - 1) / kBwdRows;
     const int per_cu = 128 / N;
     g.grad_blocks = (int)(ntiles < 256 * per_cu ? ntiles : 256 * per_cu);
-    g.dw_blocks = K == N ? g.grad_blocks : (int)(ntiles < 256 ? ntiles : 256);
+    g.dw_blocks = (int)(ntiles < 256 ? ntiles : 256);
     g.dw_tiles = (int)((ntiles + g.dw_blocks - 1) / g.dw_blocks);
     auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    const size_t part = (size_t)(2 * N * K + 2 * N) * 4, dbpart = (size_t)2 * N * 4;
     g.dpg_off = 0;
-    g.part_off = K == N ? 0 : up((size_t)M * 2 * N * 2);
-    g.dbpart_off = g.part_off + up((size_t)g.dw_blocks * (2 * N * K + 2 * N) * 4);
-    g.total = g.dbpart_off + up((size_t)g.grad_blocks * 2 * N * 4);
+    g.part_off = up((size_t)M * 2 * N * 2);
+    g.dbpart_off = g.part_off + up(g.dw_blocks * part);
+    g.total = g.dbpart_off + up(g.grad_blocks * dbpart);
+    if (K == N) {
+        // part and dbpart are multiples of 256 bytes.
+        const size_t fit = g.total / (part + dbpart);
+        if (fit < (size_t)g.grad_blocks) g.grad_blocks = (int)fit;
+        g.dw_blocks = g.grad_blocks;
+        g.part_off = 0;
+        g.dbpart_off = g.grad_blocks * part;
+    }
     return g;
 }
 

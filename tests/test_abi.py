@@ -291,6 +291,19 @@ def test_triangle_multiply_validation(kw, msg):
     assert msg in _native.last_error()
 
 
+@pytest.mark.parametrize("k,n", [(64, 64), (128, 128), (128, 64), (64, 128)])
+def test_gated_dual_proj_bwd_workspace_sizes(k, n):
+    """The workspace of every form is that of the three-kernel one: the gradient rows [M, 2N] in the
+    input type, [2N, K] and [2N] float32 partials of at most 256 blocks, the column sums of the
+    gradient kernel's blocks, each rounded up to 256 bytes."""
+    size = _native.lib().clk_gated_dual_proj_bwd_workspace_size
+    up = lambda v: (v + 255) // 256 * 256  # noqa: E731
+    for m in (1, 63, 64, 65, 1000, 16384, 16385, 32209, 32768, 90601, 512 * 512):
+        tiles = (m + 63) // 64
+        assert size(m, k, n) == (up(m * 4 * n) + up(min(tiles, 256) * (2 * n * k + 2 * n) * 4) +
+                                 up(min(tiles, 256 * (128 // n)) * 8 * n)), m
+
+
 def test_triangle_multiply_sizes():
     """The largest grid is accepted up to the workspace check; its workspace holds three
     channel-major plane sets of 2 bytes per element (ragged N adds the padded z, mask, out)."""
