@@ -57,14 +57,17 @@ __global__ __launch_bounds__(2 * HD) void attn_gate_kernel(
     // Resident A operands -log2(e) * wg^T and the matching bias.
     V8 wa[2][KS];
     f32x4 binit[2];
+    // (Transposed through the output tile's buffer, 4 KB a wave; it is not written before the first
+    // barrier.)
+    constexpr int KSC = KS % 2 == 0 ? 2 : 1;
+    static_assert(NW * 2048 * KSC <= R * OSTR, "the waves' scratch fits");
+    load_weight_columns<KS, KSC>(wg + 32 * wave, HD, ob + wave * 2048 * KSC, lane, wa);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        const int col = 32 * wave + 8 * (r16 >> 2) + 4 * h + (r16 & 3);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                wa[h][ks][j] = TR::from_f(-kLog2e * TR::to_f(wg[(32 * ks + 8 * g + j) * HD + col]));
+            for (int j = 0; j < 8; ++j) wa[h][ks][j] = TR::from_f(-kLog2e * TR::to_f(wa[h][ks][j]));
         // C lane (r16, g) holds the columns 32w + 8g + 4h + i.
 #pragma unroll
         for (int i = 0; i < 4; ++i)

@@ -112,28 +112,36 @@ __device__ __forceinline__ V lds_tr8(const void* p_lo, const void* p_hi) {
 // MFMA A operands W^T of one wave's 32 output columns, for the kernels that keep their weights in
 // registers: W has 32*KS rows, `ldw` elements apart; w points at the wave's first column. Operand
 // (h, ks), lane (r16, g): column 8*(r16/4) + 4h + r16%4, rows 32ks + 8g .. + 7. The rows arrive as
-// 16-byte pieces (any element alignment) and are transposed through `scratch`, 2*KS KB of LDS of
-// the wave's own (in order within the wave, so no barrier). Read straight from memory the
+// 16-byte pieces (any element alignment) and are transposed KSC row groups at a time through
+// `scratch`, 2*KSC KB of LDS of the wave's own (in order within the wave, so no barrier). Read straight from memory the
 // operands are 64*KS two-byte loads per lane, which held up the kernels' small calls and spilled
-// the larger ones (triangle multiplication at N = 203, C = 128 45 -> 41 us, at 512 1-2% faster).
-template <int KS, typename V8, typename E>
+// the larger ones (triangle multiplication at N = 203, C = 128 45 -> 41 us, at 512 1-2% faster;
+// the attention gate of 512 x 256 rows, 256 channels 44.8 -> 43.1 us, of 32 x 128 11.2 -> 10.5,
+// its backward's recompute 70.1 -> 67.8 and 12.2 -> 11.6).
+template <int KS, int KSC = KS, typename V8, typename E>
 __device__ __forceinline__ void load_weight_columns(const E* w, int ldw, char* scratch, int lane,
                                                     V8 (&out)[2][KS]) {
+    static_assert(KS % KSC == 0);
     const int r16 = lane & 15, g = lane >> 4;
     u32x4 raw[2 * KS];
 #pragma unroll
     for (int i = 0; i < 2 * KS; ++i)
         raw[i] = ld16_a2(w + (size_t)(16 * i + (lane >> 2)) * ldw + 8 * (lane & 3));
 #pragma unroll
-    for (int i = 0; i < 2 * KS; ++i)
-        *reinterpret_cast<u32x4*>(scratch + (16 * i + (lane >> 2)) * 64 + 16 * (lane & 3)) = raw[i];
+    for (int c = 0; c < KS; c += KSC) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+        for (int i = 0; i < 2 * KSC; ++i)
+            *reinterpret_cast<u32x4*>(scratch + (16 * i + (lane >> 2)) * 64 + 16 * (lane & 3)) =
+                raw[2 * c + i];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const char* lo = scratch + (32 * ks + 8 * g + (r16 >> 2)) * 64 + 16 * (r16 & 3) + 8 * h;
-            out[h][ks] = lds_tr8<V8>(lo, lo + 4 * 64);
-        }
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int ks = 0; ks < KSC; ++ks) {
+                const char* lo =
+                    scratch + (32 * ks + 8 * g + (r16 >> 2)) * 64 + 16 * (r16 & 3) + 8 * h;
+                out[h][c + ks] = lds_tr8<V8>(lo, lo + 4 * 64);
+            }
+    }
 }
 
 // Eight 2-byte elements (one 16-byte load) as floats.

@@ -569,14 +569,16 @@ __global__ __launch_bounds__(2 * N) void gate_bwd_grad_kernel(
     // Resident A operands -log2(e) * wg^T and the matching bias, as in the forward gate.
     V8 wa[2][KS];
     f32x4 binit[2];
+    // (Transposed through x2, which no load fills before the first barrier.)
+    constexpr int KSC = KS % 2 == 0 && NT / 64 * 4096 <= XB ? 2 : 1;
+    static_assert(NT / 64 * 2048 * KSC <= XB, "the waves' scratch fits");
+    load_weight_columns<KS, KSC>(wg + 32 * wave, N, x2 + wave * 2048 * KSC, lane, wa);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        const int col = 32 * wave + 8 * (r16 >> 2) + 4 * h + (r16 & 3);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                wa[h][ks][j] = TR::from_f(-kLog2e * TR::to_f(wg[(32 * ks + 8 * g + j) * N + col]));
+            for (int j = 0; j < 8; ++j) wa[h][ks][j] = TR::from_f(-kLog2e * TR::to_f(wa[h][ks][j]));
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             binit[h][i] = -kLog2e * TR::to_f(bg[32 * wave + 8 * g + 4 * h + i]);
