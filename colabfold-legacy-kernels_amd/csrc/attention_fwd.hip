@@ -291,7 +291,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     };
     // PATCH: this wave's mask bytes of its first kPre key tiles (t = wave + 4*i; lane l: key
     // 64t + l - shift), loaded before anything else so that the presence words below wait for
-    // them alone. Out of range (key -1 too, a negative offset) reads zero.
+    // them alone. Out of range (key -1 too, a negative offset) reads zero. (That lane's later keys
+    // are the same register plus an instruction offset; the sum wraps at 32 bits, as tested.)
     constexpr int kPre = 4;
     uint32_t mb[kPre];
     if constexpr (PATCH) {

@@ -346,3 +346,22 @@ def test_attention_fwd_query_block_choice(cuda, shape):
     for name, got, want in (("O", out_m, out), ("lse", lse_m, lse), ("O nshd", t(out_s), out),
                             ("gated", gated_m, gated)):
         assert torch.equal(got.reshape(reps, *want.shape), want.expand(reps, *want.shape)), name
+
+
+@pytest.mark.parametrize("sk", [1023, 1022, 131])
+def test_attention_fwd_picks_any_key(cuda, sk):
+    """A bias that leaves one key's weight (exp(-300) for the others is below float32's smallest
+    number): every row is that key's V, exactly, for keys at the edges of 64-key tiles that start
+    at key 0 or -1 and of the groups of tiles whose mask bytes one lane loads."""
+    n, h, sq, d = 2, 2, 131, 32
+    inp = attention_inputs(n, h, sq, sk, d, torch.bfloat16, seed=sk, with_dout=False)
+    g = {k: (v.to(cuda) if isinstance(v, torch.Tensor) else v) for k, v in inp.items()}
+    km = torch.ones((n, sk), dtype=torch.uint8, device=cuda)
+    for key in (0, 62, 63, 64, 127, 128, 254, 255, 256, 511, 512, 767, 768, sk - 2, sk - 1):
+        if key >= sk:
+            continue
+        bias = torch.full((h, sq, sk), -300.0, dtype=torch.bfloat16, device=cuda)
+        bias[:, :, key] = 0.0
+        out, _ = ops.attention_fwd(g["q"], g["k"], g["v"], bias, km, g["scale"])
+        want = g["v"][:, :, key:key + 1].expand_as(out)
+        assert torch.equal(out, want), key
