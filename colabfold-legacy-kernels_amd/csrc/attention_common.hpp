@@ -3,6 +3,7 @@
 #pragma once
 
 #include <cmath>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -340,33 +341,51 @@ struct LogitForm {
     }
 };
 
-// How the logits reach the softmax in the kernels that stream bias tiles through LDS (the
-// forward and the dK/dV kernel). Plain: logit = fmaf(q.k, scale, bias) per score (bias unpacked
-// to float32). Bias MFMA (when scale > 0): the accumulator of each 16x16 score tile starts as
-// bias / scale, added by one more MFMA per 16x16 tile whose A
-// operand is [hi*I | lo*I] (hi + lo = 1/scale as two values of the input type, each product
-// with a bias value exact in float32) and whose B operand is the tile's bias, duplicated over
-// the two halves of the contraction; the tile then holds logit / scale, and
-// log2(e) * logit = cexp * S with cexp = log2(e) / (hi + lo). No per-score instruction touches the bias. A bias of
-// magnitude above 3.4e38 * scale overflows there (float32 cannot hold bias / scale).
+// How the logits reach the softmax in the forward, which streams bias tiles through LDS. Plain:
+// logit = fmaf(q.k, scale, bias) per score (bias unpacked to float32). Bias MFMA (when scale > 0):
+// the accumulator of each 16x16 score tile starts as bias / scale, added by one more MFMA per 16x16
+// tile whose A operand is [hi*I | lo*I] (hi + lo = 1/scale as two values of the input type, each
+// product with a bias value exact in float32) and whose B operand is the tile's bias, duplicated
+// over the two halves of the contraction; the tile then holds logit / scale, and
+// log2(e) * logit = cexp * S. No per-score instruction touches the bias. A bias of magnitude above
+// 3.4e38 * scale overflows there (float32 cannot hold bias / scale).
+//
+// Ragged key counts hold scale and bias to float32: where the pair is further than 2^-24 from
+// 1/scale (bfloat16 at D = 8 and 32: 2.9e-7), a third value lo2 enters by an MFMA of its own
+// ([lo2*I | 0], three terms), and cexp = log2(e) / (hi + lo + lo2), so that the bias enters exactly
+// and q.k to the rounding of cexp (757 residues, 4 heads x 32: 550 us, 517 with the pair alone). At
+// multiples of 8 the pair alone is used, its error (up to 7.6e-6 of the bias in bfloat16) on the
+// bias, and cexp = scale * log2(e).
 struct BiasMfma {
-    float hi, lo, bscale, cexp;
+    float hi, lo, lo2, bscale, cexp;
 };
 
-// The bias-MFMA constants for `scale`, when that form applies: scale > 0 with 1/scale finite
-// and within the input type's range (hi + lo = 1/scale to about 16 bits).
+// The terms (2 or 3) of the bias MFMA for `scale`, and its constants; 0 where the form does not
+// apply: scale <= 0, 1/scale past the input type's range, or too small to be held in it (float16:
+// scale above some hundreds, or for `exact` some tens).
 template <typename TR>
-bool bias_mfma_for(float scale, BiasMfma* bm) {
+int bias_mfma_for(float scale, bool exact, BiasMfma* bm) {
     using E = typename TR::elem;
-    if (!(scale > 0.f) || !std::isfinite(scale)) return false;
+    if (!(scale > 0.f) || !std::isfinite(scale)) return 0;
     const float b = 1.f / scale;
-    if (!std::isfinite(b) || b > 6.0e4f) return false;
-    const float hi = (float)(E)b, lo = (float)(E)(b - hi);
-    // The exponent's unit is that of hi + lo, not of 1/scale: the bias then enters exactly, whatever
-    // its size (additive masks of -1e4 and beyond), and the last rounding of the pair falls on the
-    // scale of q.k (relative 3e-7 in bfloat16 at D = 32, within float32's own rounding in float16).
-    *bm = {hi, lo, b, (float)((double)kLog2e / ((double)hi + lo))};
-    return true;
+    if (!std::isfinite(b) || b > 6.0e4f) return 0;
+    if (!exact) {
+        const float hi = (float)(E)b, lo = (float)(E)(b - hi);
+        *bm = {hi, lo, 0.f, b, scale * kLog2e};
+        return std::fabs(b - hi - lo) <= 0x1p-16f * b ? 2 : 0;
+    }
+    const double want = 1.0 / scale;
+    double sum = 0.0;
+    float part[3];
+    for (int terms = 1; terms <= 3; ++terms) {
+        part[terms - 1] = (float)(E)(float)(want - sum);
+        sum += part[terms - 1];
+        if (terms < 2 || std::fabs(want - sum) > 0x1p-24 * want) continue;
+        *bm = {part[0], part[1], terms == 3 ? part[2] : 0.f, b, (float)(1.4426950408889634 / sum)};
+        // (float16's third value would lie below its smallest number.)
+        return terms == 2 || std::is_same<TR, BF16>::value ? terms : 0;
+    }
+    return 0;
 }
 
 // Host-side shape/dtype validation shared by the forward and backward entry points. The

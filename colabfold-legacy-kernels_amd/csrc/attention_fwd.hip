@@ -167,13 +167,15 @@ struct FwdItems {
 // in the second case its key tiles start one key early (tile kt: keys 64kt - 1 ...), which
 // aligns every load, and key -1 is an absent key. So the loop is the even one, with no shifting
 // of bias pieces.
-template <typename TR, int D, int QT, bool VEC, bool GATE, bool BM, bool NSHD, bool ODD>
+// TERMS: the terms of the bias MFMA (BM), 0 without it.
+template <typename TR, int D, int QT, bool VEC, bool GATE, int TERMS, bool NSHD, bool ODD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && VEC ? 3 : 1))) void attn_fwd_kernel(
     const typename TR::elem* __restrict__ q, const typename TR::elem* __restrict__ k,
     const typename TR::elem* __restrict__ v, const typename TR::elem* __restrict__ bias,
     const uint8_t* __restrict__ kmask, typename TR::elem* __restrict__ out,
     float* __restrict__ lse, int H, int Sq, int Sk, float scale,
     GateArgs<typename TR::elem> ga, BiasMfma bm, FwdItems items) {
+    constexpr bool BM = TERMS > 0;
     static_assert(!BM || VEC, "the bias MFMA reads the bias tile from LDS");
     static_assert(!ODD || BM, "odd key counts run the bias-MFMA form");
     static_assert(!(NSHD && GATE), "the gated entry takes the [N, H, S, D] layout");
@@ -401,15 +403,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     const float xs = BM ? bm.cexp : kLog2e;
     // A operand [hi*I | lo*I] of the bias MFMA: lane (row r16, group g) holds columns
     // 8g .. 8g+7, so its one nonzero is element r16 % 8 when g % 2 == r16 / 8.
-    V8 idn;
+    // (Three terms: a second operand [lo2*I | 0].)
+    V8 idn, idn2;
     if constexpr (BM) {
-        const uint32_t v = (uint32_t)__builtin_bit_cast(uint16_t, TR::from_f(g < 2 ? bm.hi : bm.lo))
-                           << (16 * (r16 & 1));
-        const int at = (g & 1) == (r16 >> 3) ? (r16 & 7) >> 1 : -1;
-        u32x4 bits;
+        auto diagonal = [&](float upper, float lower) {
+            const uint32_t v =
+                (uint32_t)__builtin_bit_cast(uint16_t, TR::from_f(g < 2 ? upper : lower))
+                << (16 * (r16 & 1));
+            const int at = (g & 1) == (r16 >> 3) ? (r16 & 7) >> 1 : -1;
+            u32x4 bits;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) bits[i] = i == at ? v : 0u;
-        idn = bits_as<V8>(bits);
+            for (int i = 0; i < 4; ++i) bits[i] = i == at ? v : 0u;
+            return bits_as<V8>(bits);
+        };
+        idn = diagonal(bm.hi, bm.lo);
+        if constexpr (TERMS == 3) idn2 = diagonal(bm.lo2, 0.f);
     }
 
     // Running max, and O^T plus one extra accumulator per sub-tile: the MFMA of an all-ones
@@ -491,7 +499,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
                 for (int t = 0; t < 4; ++t) {
                     const u32x4 raw = *reinterpret_cast<const u32x4*>(
                         brow_l + 16 * ((2 * t + (g & 1)) ^ (row & 7)));
-                    s[qt][t] = TR::mfma(idn, bits_as<V8>(raw), f32x4{0.f, 0.f, 0.f, 0.f});
+                    f32x4 low = {0.f, 0.f, 0.f, 0.f};
+                    if constexpr (TERMS == 3) low = TR::mfma(idn2, bits_as<V8>(raw), low);
+                    s[qt][t] = TR::mfma(idn, bits_as<V8>(raw), low);
                 }
             }
         }
@@ -755,23 +765,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     }
 }
 
-// How a call's bias reaches the kernel.
+// How a call's bias reaches the kernel (terms: those of the bias MFMA, 0 without it).
 struct FwdForm {
     BiasMfma bm{};
-    bool bmf, odd, vec;
+    int terms;
+    bool odd, vec;
 };
 
 // The bias tile through LDS (vec: direct loads of 4-byte aligned pieces): at most kPresWords key
 // tiles (masked bias tiles are changed in LDS from presence words kept there). An even Sk
 // aligns every bias row. An odd one takes the parity form of the bias-MFMA kernel, when the
 // bias is a whole number of dwords (no load then reaches past its end). Other odd cases
-// (scale <= 0, one head or an odd number of them with an odd Sq) and longer rows read bias and
-// mask element by element, about four times slower (2395 against 550 us at 757 residues).
+// (scale <= 0 or without a bias MFMA, one head or an odd number of them with an odd Sq) and longer
+// rows read bias and mask element by element, about four times slower (2395 against 550 us at 757
+// residues).
 template <typename TR>
 FwdForm fwd_form(int H, int Sq, int Sk, float scale) {
     FwdForm f;
-    f.bmf = bias_mfma_for<TR>(scale, &f.bm);
-    const bool odd = Sk % 2 && f.bmf && (size_t)H * Sq * Sk % 2 == 0;
+    f.terms = bias_mfma_for<TR>(scale, Sk % 8 != 0, &f.bm);
+    const bool odd = Sk % 2 && f.terms && (size_t)H * Sq * Sk % 2 == 0;
     f.vec = (Sk % 2 == 0 || odd) && Sk + (odd ? 1 : 0) <= kPresWords * 64;
     f.odd = f.vec && odd;
     return f;
@@ -825,14 +837,20 @@ void launch_fwd_qt(hipStream_t st, const void* q, const void* k, const void* v, 
         kernel<<<grid, 256, 0, st>>>((const E*)q, (const E*)k, (const E*)v, (const E*)bias, kmask,
                                      (E*)out, lse, H, Sq, Sk, scale, ga, f.bm, items);
     };
-    if (f.odd)
-        run(attn_fwd_kernel<TR, D, QT, true, GATE, true, NSHD, true>);
-    else if (f.vec && f.bmf)
-        run(attn_fwd_kernel<TR, D, QT, true, GATE, true, NSHD, false>);
-    else if (f.vec)
-        run(attn_fwd_kernel<TR, D, QT, true, GATE, false, NSHD, false>);
-    else
-        run(attn_fwd_kernel<TR, D, QT, false, GATE, false, NSHD, false>);
+    auto run_terms = [&](auto terms) {
+        if (f.odd)
+            run(attn_fwd_kernel<TR, D, QT, true, GATE, decltype(terms)::value, NSHD, true>);
+        else
+            run(attn_fwd_kernel<TR, D, QT, true, GATE, decltype(terms)::value, NSHD, false>);
+    };
+    if (!f.vec)
+        run(attn_fwd_kernel<TR, D, QT, false, GATE, 0, NSHD, false>);
+    else if (f.terms == 0)
+        run(attn_fwd_kernel<TR, D, QT, true, GATE, 0, NSHD, false>);
+    else if (f.terms == 2)
+        run_terms(std::integral_constant<int, 2>{});
+    else if constexpr (std::is_same<TR, BF16>::value)
+        run_terms(std::integral_constant<int, 3>{});
 }
 
 template <typename TR, int D, bool GATE>

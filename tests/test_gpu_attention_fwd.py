@@ -365,3 +365,37 @@ def test_attention_fwd_picks_any_key(cuda, sk):
         out, _ = ops.attention_fwd(g["q"], g["k"], g["v"], bias, km, g["scale"])
         want = g["v"][:, :, key:key + 1].expand_as(out)
         assert torch.equal(out, want), key
+
+
+# (dtype, scale, q, k): scales whose inverse two values of the type hold to 3e-7 (bfloat16, head
+# dims 8 and 32), to 7e-6, or not at all (float16), and one dominating q.k of about 600 / scale.
+SCALES = [(torch.bfloat16, 32 ** -0.5, 64.0, 56.0), (torch.bfloat16, 0.4989, 32.0, 40.0),
+          (torch.bfloat16, 0.3, 32.0, 64.0), (torch.bfloat16, 0.25, 64.0, 40.0),
+          (torch.bfloat16, 3e4, 0.125, 0.15625), (torch.float16, 32 ** -0.5, 64.0, 56.0),
+          (torch.float16, 100.0, 2.0, 3.0), (torch.float16, 1e5, 0.0625, 0.09375),
+          (torch.float16, 1e8, 2.0 ** -9, 1.5 * 2.0 ** -9)]
+
+
+@pytest.mark.parametrize("sk", [64, 66, 67])
+@pytest.mark.parametrize("dtype,scale,qv,kv", SCALES, ids=lambda v: str(v).replace("torch.", ""))
+def test_attention_fwd_logits_are_float32(cuda, dtype, scale, qv, kv, sk):
+    """A row with one key far above the others has that key's logit as its lse: scale * q.k and
+    the bias both enter it as float32 values. The bound is eight roundings of 2^-24: the constants
+    of the score's unit and of the two logarithms, the products and the sums. (At a multiple of
+    eight keys only q.k is held to it.)"""
+    n, h, sq, d = 1, 2, 6, 32
+    q = torch.zeros((n, h, sq, d), dtype=dtype)
+    k = torch.zeros((n, h, sk, d), dtype=dtype)
+    v = torch.ones((n, h, sk, d), dtype=dtype)
+    bias = torch.zeros((h, sq, sk), dtype=dtype)
+    q[:, :, :3, 1] = qv
+    k[:, :, sk - 1, 1] = kv
+    bias[:, 3:, 5] = 600.0
+    args = [t.to(cuda) for t in (q, k, v, bias)]
+    _, lse = ops.attention_fwd(*args, None, scale)
+    s32 = float(np.float32(scale))
+    want = torch.tensor([qv * kv * s32] * 3 + [600.0] * 3, dtype=torch.float64)
+    err = ((lse.cpu().double() - want) / want).abs().amax((0, 1))
+    print("relative", err.tolist())
+    held = err if sk % 8 else err[:3]
+    assert (held <= 8 * 2.0 ** -24).all(), held.tolist()
