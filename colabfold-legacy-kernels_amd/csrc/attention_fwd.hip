@@ -662,8 +662,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             tile(kt, kv0, kv1, ca, cb);
             if (kt + 1 < nrun) tile(kt + 1, kv1, kv0, cb, ca);
         }
-        if (nrun == 0) async_wait();  // no load into LDS outlives the block
     }
+    if (nrun == 0) async_wait();  // no keys: tile 0's loads end before the block (or its gate)
 
     // Gate pre-activations in O^T's accumulator layout (lane: rows 16*dt + 4*g + i of head h's
     // columns, query r16), so gate and O pair up element for element.

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from _util import TOL, assert_close, dname, np64
-from colabfold_legacy_kernels import ops
+from colabfold_legacy_kernels import _native, ops
 from colabfold_legacy_kernels.workloads import attention_inputs, attention_workload, gate_inputs
 from oracle import attention as ref
 
@@ -399,3 +399,34 @@ def test_attention_fwd_logits_are_float32(cuda, dtype, scale, qv, kv, sk):
     print("relative", err.tolist())
     held = err if sk % 8 else err[:3]
     assert (held <= 8 * 2.0 ** -24).all(), held.tolist()
+
+
+@pytest.mark.parametrize("masked", [False, True])
+def test_attention_fwd_without_keys(cuda, masked):
+    """No keys at all (the C entries take such a call): O = 0 and lse = +inf, ungated in both
+    layouts and gated, in the neighbourhood of an ordinary call on the same stream."""
+    n, h, sq, d, c = 300, 4, 130, 32, 64
+    inp = attention_inputs(n, h, sq, 64, d, torch.bfloat16, seed=3, with_dout=False)
+    g = {k: (v.to(cuda) if isinstance(v, torch.Tensor) else v) for k, v in inp.items()}
+    x, wg, bg = (t.to(cuda) for t in gate_inputs(n, sq, c, h * d, torch.bfloat16, seed=4))
+    lib, stream = _native.lib(), torch.cuda.current_stream().cuda_stream
+    ptr = lambda t: t.data_ptr()  # noqa: E731
+    km = ptr(g["kmask"]) if masked else None
+    want = ops.attention(g["q"], g["k"], g["v"], g["bias"], None, g["scale"])
+    for entry in ("plain", "nshd", "gated"):
+        out = torch.full_like(g["q"], 7.0)
+        gated = torch.full((n, sq, h * d), 7.0, dtype=out.dtype, device=cuda)
+        lse = torch.zeros((n, h, sq), device=cuda)
+        head = (stream, _native.BF16, ptr(g["q"]), ptr(g["k"]), ptr(g["v"]), ptr(g["bias"]), km)
+        if entry == "plain":
+            status = lib.clk_attention_fwd(*head, ptr(out), ptr(lse), n, h, sq, 0, d, 0.125, 64, 64)
+        elif entry == "nshd":
+            status = lib.clk_attention_fwd_nshd(*head, ptr(out), ptr(lse), n, h, sq, 0, d, 0.125)
+        else:
+            status = lib.clk_attention_fwd_gated(*head, ptr(x), ptr(wg), ptr(bg), ptr(gated),
+                                                 ptr(out), ptr(lse), n, h, sq, 0, d, c, 0.125)
+            assert not gated.any()
+        assert status == _native.OK, _native.last_error()
+        after = ops.attention(g["q"], g["k"], g["v"], g["bias"], None, g["scale"])
+        assert not out.any() and bool((lse == np.inf).all())
+        assert torch.equal(after, want)
