@@ -347,8 +347,8 @@ struct LogitForm {
 // tile whose A operand is [hi*I | lo*I] (hi + lo = 1/scale as two values of the input type, each
 // product with a bias value exact in float32) and whose B operand is the tile's bias, duplicated
 // over the two halves of the contraction; the tile then holds logit / scale, and
-// log2(e) * logit = cexp * S. No per-score instruction touches the bias. A bias of magnitude above
-// 3.4e38 * scale overflows there (float32 cannot hold bias / scale).
+// log2(e) * logit = cexp * S. No per-score instruction touches the bias. A bias whose bias / scale
+// float32 cannot hold, -inf among them, leaves NaN, and its block is redone in the plain form.
 //
 // Ragged key counts hold scale and bias to float32: where the pair is further than 2^-24 from
 // 1/scale (bfloat16 at D = 8 and 32: 2.9e-7), a third value lo2 enters by an MFMA of its own

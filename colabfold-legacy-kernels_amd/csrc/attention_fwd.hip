@@ -442,7 +442,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
         for (int dt = 0; dt < G::DT; ++dt) acc[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-    auto tile = [&](int kt, const char* kvc, char* kvn, PF& cur, PF& nxt) {
+    // PLAIN (PATCH): the same tile with the bias as it is added to each score, and a select per
+    // absent key, for blocks whose bias holds -inf (below).
+    auto tile = [&](int kt, const char* kvc, char* kvn, PF& cur, PF& nxt, auto plain_tag) {
+        constexpr bool PLAIN = decltype(plain_tag)::value;
+        constexpr bool BMT = BM && !PLAIN;  // the bias through the MFMA
+        const float xt = PLAIN ? kLog2e : xs;
         const int k0 = kt * BK;
         async_wait();
         __syncthreads();  // tile kt visible; every wave is done with the other buffer
@@ -465,7 +470,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             stage_rows_ld<D, kGateChannels, 256>(rw, 0, ga.HD, kvn, t);
         }
         // Each wave reads only its own rows of the bias tile: no barrier after the change.
-        if (PATCH && need_mask) {
+        if (PATCH && !PLAIN && need_mask) {
             patch(kvc, kt);
             // Nothing of the tile's work is interleaved with the change (registers).
             __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -486,7 +491,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
 
         // S^T = K . Q^T for the four 16-key sub-tiles (chunk c = t/2, half t%2).
         f32x4 s[QT][4];
-        if constexpr (BM) {
+        if constexpr (BMT) {
             // Bias / scale first. S^T tile t holds keys 16t + 0..15 of the key tile here, so
             // rows 8g' + j of the B operand (g' = g % 2, duplicated for the lo half) are keys
             // 16t + 8g' + 0..7 of the lane's query row: one 16-byte piece, 2t + g', of the
@@ -512,7 +517,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
 #pragma unroll
                 for (int qt = 0; qt < QT; ++qt)
                     s[qt][t] = TR::mfma(kf[t][ks], qf[qt][ks],
-                                        (BM || ks > 0) ? s[qt][t] : f32x4{0.f, 0.f, 0.f, 0.f});
+                                        (BMT || ks > 0) ? s[qt][t] : f32x4{0.f, 0.f, 0.f, 0.f});
 
         float x[QT][2][8];
 #pragma unroll
@@ -524,6 +529,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
                     for (int j = 0; j < 4; ++j) {
                         x[qt][c][j] = s[qt][2 * c][j];
                         x[qt][c][4 + j] = s[qt][2 * c + 1][j];
+                    }
+                    if constexpr (PLAIN) {
+                        // Keys 16t + 4g + 0..3 of the lane's query, t = 2c + u: half a piece.
+                        const int row = wave * 16 * QT + 16 * qt + r16;
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            E e[4];
+                            __builtin_memcpy(e, kvc + 2 * TILE + row * 128 + 8 * (g & 1) +
+                                                    16 * ((4 * c + 2 * u + (g >> 1)) ^ (row & 7)),
+                                             8);
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                x[qt][c][4 * u + j] =
+                                    fmaf(x[qt][c][4 * u + j], scale, TR::to_f(e[j]));
+                        }
                     }
                     continue;
                 }
@@ -561,6 +581,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             }
         }
 
+        if constexpr (PLAIN) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const uint32_t w = reinterpret_cast<const uint32_t*>(pres)[2 * kt + c];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int bit = !BM ? 8 * g + j : 4 * g + (j < 4 ? j : 12 + j);
+#pragma unroll
+                    for (int qt = 0; qt < QT; ++qt)
+                        x[qt][c][j] = (w >> bit) & 1u ? x[qt][c][j] : kMaskedLogit;
+                }
+            }
+        }
+
         float mt[QT];
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
@@ -581,12 +615,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             // Lazy rescaling: the running max moves only when the tile's max exceeds it by more
             // than kRescaleSlack (in log2 units), so P stays below 2^kRescaleSlack and most tiles
             // skip the rescale of O and l (a wave-uniform branch).
-            const bool move = fmaf(mt[qt], xs, nm[qt]) > kRescaleSlack;
+            const bool move = fmaf(mt[qt], xt, nm[qt]) > kRescaleSlack;
             if (__any(move)) {
                 // Opaque to if-conversion: without it the compiler runs the rescale on every
                 // tile (alpha = 1 when nothing moved gives the same values).
                 asm volatile("");
-                const float nm_new = move ? -mt[qt] * xs : nm[qt];
+                const float nm_new = move ? -mt[qt] * xt : nm[qt];
                 const float alpha = fast_exp2(nm_new - nm[qt]);
                 nm[qt] = nm_new;
                 lsum[qt][0] *= alpha;  // only component 0 is read
@@ -598,7 +632,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
 #pragma unroll
             for (int c = 0; c < 2; ++c)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) pf[c][j] = TR::from_f(fast_exp2(fmaf(x[qt][c][j], xs, neg)));
+                for (int j = 0; j < 8; ++j) pf[c][j] = TR::from_f(fast_exp2(fmaf(x[qt][c][j], xt, neg)));
 #pragma unroll
             for (int c = 0; c < 2; ++c) lsum[qt] = TR::mfma(ones, pf[c], lsum[qt]);
 #pragma unroll
@@ -659,8 +693,38 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
         }
     } else {
         for (int kt = 0; kt < nrun; kt += 2) {
-            tile(kt, kv0, kv1, ca, cb);
-            if (kt + 1 < nrun) tile(kt + 1, kv1, kv0, cb, ca);
+            tile(kt, kv0, kv1, ca, cb, std::false_type{});
+            if (kt + 1 < nrun) tile(kt + 1, kv1, kv0, cb, ca, std::false_type{});
+        }
+        if constexpr (PATCH) {
+            // A bias of -inf leaves NaN in the row sum of its query (the zeros of the bias MFMA's
+            // operand times it are NaN). A block with one redoes its keys in the plain form, where
+            // -inf is a weight of 0. (By its bits: this file is compiled without NaN semantics.
+            // The look at the sums and its barrier: 384 residues 269.8 -> 271.0 us, 1024 with the
+            // gate 1167 -> 1173, 1024 x 300 at D = 8 262.9 -> 266.0.)
+            bool nan = false;
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt)
+                nan = nan || (__float_as_uint(lsum[qt][0]) & 0x7fffffffu) > 0x7f800000u;
+            const bool wave_nan = __any(nan);
+            if (lane == 0) wave_last[wave] = wave_nan;
+            lds_barrier();
+            const int any_nan = (wave_last[0] | wave_last[1]) | (wave_last[2] | wave_last[3]);
+            if (__builtin_amdgcn_readfirstlane(any_nan)) {
+                async_wait();
+                __syncthreads();  // no load into a buffer is in flight, no wave reads one
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) {
+                    nm[qt] = -(0.5f * kMaskedLogit) * kLog2e;
+                    lsum[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int dt = 0; dt < G::DT; ++dt) acc[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+                stage(0, kv0);
+#pragma unroll 1
+                for (int kt = 0; kt < nrun; ++kt)
+                    tile(kt, kt & 1 ? kv1 : kv0, kt & 1 ? kv0 : kv1, ca, cb, std::true_type{});
+            }
         }
     }
     if (nrun == 0) async_wait();  // no keys: tile 0's loads end before the block (or its gate)

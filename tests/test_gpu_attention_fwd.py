@@ -7,6 +7,7 @@ from _util import TOL, assert_close, dname, np64
 from colabfold_legacy_kernels import _native, ops
 from colabfold_legacy_kernels.workloads import attention_inputs, attention_workload, gate_inputs
 from oracle import attention as ref
+from oracle import gate as ref_gate
 
 pytestmark = pytest.mark.gpu
 
@@ -430,3 +431,54 @@ def test_attention_fwd_without_keys(cuda, masked):
         after = ops.attention(g["q"], g["k"], g["v"], g["bias"], None, g["scale"])
         assert not out.any() and bool((lse == np.inf).all())
         assert torch.equal(after, want)
+
+
+# Key counts: odd, even and multiples of 8, with a ragged last tile or without.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=dname)
+@pytest.mark.parametrize("sk,d", [(67, 32), (203, 32), (130, 16), (200, 32), (192, 64), (301, 8)])
+def test_attention_fwd_infinite_bias(cuda, sk, d, dtype):
+    """-inf in the bias is a weight of exactly 0: at single present keys, at all keys but one of a
+    query, at absent keys, and (O = 0, lse = +inf) at all keys of a query. Forward in both layouts
+    and gated, and the gradients; the queries around them are untouched."""
+    n, h, sq, c = 3, 2, 131, 64
+    inp = attention_inputs(n, h, sq, sk, d, dtype, seed=sk + d, masked_tail=0.1, masked_rows=1)
+    gen = torch.Generator().manual_seed(sk)
+    hole = torch.rand((h, sq, sk), generator=gen) < 0.3
+    hole[:, :, 1] = False
+    hole[:, 3::7] = False
+    hole[0, 20] = True
+    hole[0, 20, 1] = False
+    nothing = (1, 64)  # the query without any key
+    hole[nothing] = True
+    inp["bias"] = inp["bias"].masked_fill(hole, -np.inf)
+    g = {k: (v.to(cuda) if isinstance(v, torch.Tensor) else v) for k, v in inp.items()}
+    args = (g["q"], g["k"], g["v"], g["bias"], g["kmask"])
+    out, lse = ops.attention_fwd(*args, g["scale"])
+    full = (inp["kmask"] != 0).any(1)  # rows with a present key
+    assert not out[full][:, nothing[0], nothing[1]].any()
+    assert bool((lse[full][:, nothing[0], nothing[1]] == np.inf).all())
+    # The oracle's masked logit would be that query's largest: the same value at every key there.
+    safe = inp["bias"].clone()
+    safe[nothing] = 0
+    dout = g["dout"].clone()
+    dout[:, nothing[0], nothing[1]] = 0
+    o_ref, lse_ref = _oracle({**inp, "bias": safe})
+    for t in (out, lse):
+        t[full.to(cuda), nothing[0], nothing[1]] = 0
+    o_ref[full.numpy(), nothing[0], nothing[1]] = 0
+    lse_ref[full.numpy(), nothing[0], nothing[1]] = 0
+    assert_close("O", out, o_ref, TOL[dname(dtype)]["o"])
+    assert np.abs(np64(lse) - np.where(full.numpy()[:, None, None], lse_ref, np.log(sk))).max() < 5e-2
+    t = lambda a: a.transpose(1, 2).contiguous()  # noqa: E731
+    out_s = t(ops.attention_nshd(t(g["q"]), t(g["k"]), t(g["v"]), *args[3:], g["scale"])[0])
+    assert torch.equal(out_s, out)
+    x, wg, bg = (a.to(cuda) for a in gate_inputs(n, sq, c, h * d, dtype, seed=sk))
+    gated = ops.attention_gated(*args, x, wg, bg, g["scale"])
+    assert_close("gated", gated, ref_gate.attention_gate(o_ref, np64(x), np64(wg), np64(bg)),
+                 TOL[dname(dtype)]["o"])
+    out, lse = ops.attention_fwd(*args, g["scale"])
+    grads = ops.attention_bwd(*args, out, dout, lse, g["scale"])
+    refs = ref.attention_bwd(np64(inp["q"]), np64(inp["k"]), np64(inp["v"]), np64(safe),
+                             inp["kmask"].numpy(), inp["scale"], np64(dout))
+    for name, got, want in zip(("dQ", "dK", "dV", "dBias"), grads, refs):
+        assert_close(name, got, want, TOL[dname(dtype)]["grad"])
