@@ -482,3 +482,23 @@ def test_attention_fwd_infinite_bias(cuda, sk, d, dtype):
                              inp["kmask"].numpy(), inp["scale"], np64(dout))
     for name, got, want in zip(("dQ", "dK", "dV", "dBias"), grads, refs):
         assert_close(name, got, want, TOL[dname(dtype)]["grad"])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=dname)
+@pytest.mark.parametrize("value", [np.nan, np.inf, 3e4])
+@pytest.mark.parametrize("sk", [67, 130, 200])
+def test_attention_fwd_ignores_absent_keys_k(cuda, sk, value, dtype):
+    """Whatever the K rows of absent keys hold (3e4 stands for 3e34 in bfloat16: q.k then passes
+    the masked logit) reaches nothing, in the forms with and without the bias MFMA."""
+    if value == 3e4 and dtype == torch.bfloat16:
+        value = 3e34
+    inp = attention_inputs(3, 2, 70, sk, 32, dtype, seed=sk, with_dout=False)
+    inp["kmask"][0, 5] = inp["kmask"][1, sk - 1] = 0
+    g = {k: (v.to(cuda) if isinstance(v, torch.Tensor) else v) for k, v in inp.items()}
+    g["k"][0, :, 5] = g["k"][1, 1, sk - 1] = value
+    for sign in (1, -1):
+        inp["scale"] *= sign
+        out, lse = ops.attention_fwd(g["q"], g["k"], g["v"], g["bias"], g["kmask"], inp["scale"])
+        o_ref, lse_ref = _oracle(inp)
+        assert_close("O", out, o_ref, TOL[dname(dtype)]["o"])
+        assert np.abs(np64(lse) - lse_ref).max() < 5e-2
