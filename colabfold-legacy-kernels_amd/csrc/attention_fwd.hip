@@ -189,8 +189,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     // bfloat16, float16's lowest value -65504 in float16 (the reference's own masked logit is
     // -1e4) -- and the scores need no per-key select, so the tile's MFMAs and exponentials stay
     // one straight-line block. (A row without any present key computes no scores: tile_empty.)
-    // (No larger magnitude: the exponent's FMA against the running max leaves a rounding residue of about 2^-24 of the
-    // logit, which must stay far below float32's exponent range.)
+    // (No larger magnitude: the exponent's FMA against the running max leaves a rounding residue of
+    // about 2^-24 of the logit, which must stay far below float32's exponent range.) A float16 query
+    // whose own logits lie that low is redone with -1e9 at absent keys, as below.
     constexpr bool PATCH = VEC;
     using PF = TilePrefetch<TR, QT>;
     constexpr int BQ = 4 * 16 * QT;
@@ -459,6 +460,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
         for (int dt = 0; dt < G::DT; ++dt) acc[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
+    // Float16's changed bias is no lower than a caller's may be (LOWEST): whether some tile had one.
+    constexpr bool LOWEST = PATCH && !std::is_same<TR, BF16>::value;
+    bool patched = false;
     // PLAIN (PATCH): the same tile with the bias as it is added to each score, and a select per
     // absent key, for blocks whose bias holds -inf (below).
     auto tile = [&](int kt, const char* kvc, char* kvn, PF& cur, PF& nxt, auto plain_tag) {
@@ -486,6 +490,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             asm volatile("" : "+v"(t));
             stage_rows_ld<D, kGateChannels, 256>(rw, 0, ga.HD, kvn, t);
         }
+        if (LOWEST) patched = patched || need_mask;
         // Each wave reads only its own rows of the bias tile: no barrier after the change.
         if (PATCH && !PLAIN && need_mask) {
             patch(kvc, kt);
@@ -716,18 +721,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
         if constexpr (PATCH) {
             // A bias of -inf leaves NaN in the row sum of its query (the zeros of the bias MFMA's
             // operand times it are NaN). A block with one redoes its keys in the plain form, where
-            // -inf is a weight of 0. (By its bits: this file is compiled without NaN semantics.
-            // The look at the sums and its barrier: 384 residues 269.8 -> 271.0 us, 1024 with the
+            // -inf is a weight of 0. So does a float16 block with a row maximum near -65504, where
+            // absent keys would take weight: above -65400 theirs is below float32's smallest number.
+            // (NaN by its bits: this file is compiled without NaN semantics. The look at the sums and its barrier: 384 residues 269.8 -> 271.0 us, 1024 with the
             // gate 1167 -> 1173, 1024 x 300 at D = 8 262.9 -> 266.0.)
-            bool nan = false;
+            bool bad = false;
 #pragma unroll
-            for (int qt = 0; qt < QT; ++qt)
-                nan = nan || (__float_as_uint(lsum[qt][0]) & 0x7fffffffu) > 0x7f800000u;
-            const bool wave_nan = __any(nan);
-            if (lane == 0) wave_last[wave] = wave_nan;
+            for (int qt = 0; qt < QT; ++qt) {
+                bad = bad || (__float_as_uint(lsum[qt][0]) & 0x7fffffffu) > 0x7f800000u;
+                if (LOWEST) bad = bad || (patched && nm[qt] > 65400.f * kLog2e);
+            }
+            const bool wave_bad = __any(bad);
+            if (lane == 0) wave_last[wave] = wave_bad;
             lds_barrier();
-            const int any_nan = (wave_last[0] | wave_last[1]) | (wave_last[2] | wave_last[3]);
-            if (__builtin_amdgcn_readfirstlane(any_nan)) {
+            const int any_bad = (wave_last[0] | wave_last[1]) | (wave_last[2] | wave_last[3]);
+            if (__builtin_amdgcn_readfirstlane(any_bad)) {
                 async_wait();
                 __syncthreads();  // no load into a buffer is in flight, no wave reads one
 #pragma unroll

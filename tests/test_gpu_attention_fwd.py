@@ -502,3 +502,23 @@ def test_attention_fwd_ignores_absent_keys_k(cuda, sk, value, dtype):
         o_ref, lse_ref = _oracle(inp)
         assert_close("O", out, o_ref, TOL[dname(dtype)]["o"])
         assert np.abs(np64(lse) - lse_ref).max() < 5e-2
+
+
+@pytest.mark.parametrize("scale", [32 ** -0.5, -32 ** -0.5])
+@pytest.mark.parametrize("sk", [66, 67, 200, 203])
+def test_attention_fwd_lowest_float16_bias(cuda, sk, scale):
+    """Float16 queries whose bias is the type's lowest value at every key (padded queries under an
+    additive mask): no weight goes to absent keys (-1e9) or past the last one. The logits are near
+    65504, where float32 steps by 2^-8: four roundings move a logit by 2^-7 and a weight by 0.8%."""
+    n, h, sq, d = 3, 2, 70, 32
+    inp = attention_inputs(n, h, sq, sk, d, torch.float16, seed=sk, masked_tail=0.2, masked_rows=1,
+                           with_dout=False)
+    inp["scale"] = scale
+    inp["bias"][0, 3:40] = -65504.0
+    inp["bias"][1, 60:] = -65504.0
+    g = {k: (v.to(cuda) if isinstance(v, torch.Tensor) else v) for k, v in inp.items()}
+    out, lse = ops.attention_fwd(g["q"], g["k"], g["v"], g["bias"], g["kmask"], g["scale"])
+    o_ref, lse_ref = _oracle(inp)
+    assert_close("O", out, o_ref, TOL["f16"]["o"] + 0.008)
+    full = (inp["kmask"] != 0).any(1).numpy()[:, None, None]
+    assert np.abs(np64(lse) - np.where(full, lse_ref, np.log(sk))).max() <= 2.0 ** -6
