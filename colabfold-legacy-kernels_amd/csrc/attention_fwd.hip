@@ -723,8 +723,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             // operand times it are NaN). A block with one redoes its keys in the plain form, where
             // -inf is a weight of 0. So does a float16 block with a row maximum near -65504, where
             // absent keys would take weight: above -65400 theirs is below float32's smallest number.
-            // (NaN by its bits: this file is compiled without NaN semantics. The look at the sums and its barrier: 384 residues 269.8 -> 271.0 us, 1024 with the
-            // gate 1167 -> 1173, 1024 x 300 at D = 8 262.9 -> 266.0.)
+            // (NaN by its bits: this file is compiled without NaN semantics. The look at the sums
+            // and its barrier: 384 residues 269.8 -> 271.0 us, 1024 with the gate 1167 -> 1173,
+            // 1024 x 300 at D = 8 262.9 -> 266.0.)
             bool bad = false;
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
@@ -861,26 +862,30 @@ struct FwdForm {
     bool odd, vec;
 };
 
+// Most blocks of a launch: a grid is at most 2^32 - 1 threads (more wrap around, without an error).
+constexpr int64_t kMaxBlocks = (((int64_t)1 << 32) - 1) / 256;
+
+// Query blocks of one (row, head) at 64*QT queries each.
+int fwd_qtiles(bool odd, int Sq, int QT) {
+    return odd ? 2 * ceil_div((Sq + 1) / 2, 64 * QT) : ceil_div(Sq, 64 * QT);
+}
+
 // The bias tile through LDS (vec: direct loads of 4-byte aligned pieces): at most kPresWords key
 // tiles (masked bias tiles are changed in LDS from presence words kept there). An even Sk
 // aligns every bias row. An odd one takes the parity form of the bias-MFMA kernel, when the
 // bias is a whole number of dwords (no load then reaches past its end). Other odd cases
-// (scale <= 0 or without a bias MFMA, one head or an odd number of them with an odd Sq) and longer
-// rows read bias and mask element by element, about four times slower (2395 against 550 us at 757
-// residues).
+// (scale <= 0 or without a bias MFMA, one head or an odd number of them with an odd Sq, so many
+// short rows that two parities of blocks pass the largest launch) and longer rows read bias and mask
+// element by element, about four times slower (2395 against 577 us at 757 residues).
 template <typename TR>
-FwdForm fwd_form(int H, int Sq, int Sk, float scale) {
+FwdForm fwd_form(int64_t NH, int H, int Sq, int Sk, float scale) {
     FwdForm f;
     f.terms = bias_mfma_for<TR>(scale, Sk % 8 != 0, &f.bm);
-    const bool odd = Sk % 2 && f.terms && (size_t)H * Sq * Sk % 2 == 0;
+    const bool odd = Sk % 2 && f.terms && (size_t)H * Sq * Sk % 2 == 0 &&
+                     NH * fwd_qtiles(true, Sq, Sq <= 64 ? 1 : 2) <= kMaxBlocks;
     f.vec = (Sk % 2 == 0 || odd) && Sk + (odd ? 1 : 0) <= kPresWords * 64;
     f.odd = f.vec && odd;
     return f;
-}
-
-// Query blocks of one (row, head) at 64*QT queries each.
-int fwd_qtiles(const FwdForm& f, int Sq, int QT) {
-    return f.odd ? 2 * ceil_div((Sq + 1) / 2, 64 * QT) : ceil_div(Sq, 64 * QT);
 }
 
 // Queries per block: 64 (one 16-query sub-tile a wave) or 128 (two, which share each K, V and
@@ -896,9 +901,10 @@ int fwd_qtiles(const FwdForm& f, int Sq, int QT) {
 bool fwd_small_blocks(const FwdForm& f, int D, int64_t NH, int Sq) {
     if (Sq <= 64) return true;
     if (!f.vec) return false;
-    const int m = fwd_qtiles(f, Sq, 1);
+    const int m = fwd_qtiles(f.odd, Sq, 1);
+    if (NH * m > kMaxBlocks) return false;
     if (NH * m <= (D == 64 ? 512 : 1024)) return true;
-    return m < 2 * fwd_qtiles(f, Sq, 2) && (D <= 16 || (D == 32 && m <= 7));
+    return m < 2 * fwd_qtiles(f.odd, Sq, 2) && (D <= 16 || (D == 32 && m <= 7));
 }
 
 template <typename TR, int D, int QT, bool GATE, bool NSHD>
@@ -906,7 +912,7 @@ void launch_fwd_qt(hipStream_t st, const void* q, const void* k, const void* v, 
                    const uint8_t* kmask, void* out, float* lse, int N, int H, int Sq, int Sk,
                    float scale, GateArgs<typename TR::elem> ga, const FwdForm& f) {
     using E = typename TR::elem;
-    const int qtiles = fwd_qtiles(f, Sq, QT);
+    const int qtiles = fwd_qtiles(f.odd, Sq, QT);
     const dim3 grid(qtiles * H * N);
     // The head-outer work-item order when the bias of all heads passes half of an XCD's 4 MB L2,
     // in groups of rows whose query tiles make about 48 work items, half an XCD's resident
@@ -947,7 +953,7 @@ void launch_fwd(hipStream_t st, const void* q, const void* k, const void* v, con
                 const uint8_t* kmask, void* out, float* lse, int N, int H, int Sq, int Sk,
                 float scale, GateArgs<typename TR::elem> ga, int nshd) {
     KernelTimer timer(GATE ? "attn_fwd_gated" : "attn_fwd", st);
-    const FwdForm f = fwd_form<TR>(H, Sq, Sk, scale);
+    const FwdForm f = fwd_form<TR>((int64_t)N * H, H, Sq, Sk, scale);
     const bool small = fwd_small_blocks(f, D, (int64_t)N * H, Sq);
     auto launch = [&](auto qt, auto rows_nshd) {
         launch_fwd_qt<TR, D, decltype(qt)::value, GATE, decltype(rows_nshd)::value>(

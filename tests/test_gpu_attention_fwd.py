@@ -522,3 +522,21 @@ def test_attention_fwd_lowest_float16_bias(cuda, sk, scale):
     assert_close("O", out, o_ref, TOL["f16"]["o"] + 0.008)
     full = (inp["kmask"] != 0).any(1).numpy()[:, None, None]
     assert np.abs(np64(lse) - np.where(full, lse_ref, np.log(sk))).max() <= 2.0 ** -6
+
+
+# (N, H, Sq, Sk, D): one query and one key for 8.5 million (row, head) pairs, whose two parities of
+# query blocks would pass the 2^32 - 1 threads of a launch, and 130 queries for 5.9 million, whose
+# three 64-query blocks would.
+@pytest.mark.parametrize("shape", [(65535, 130, 1, 1, 8), (65535, 90, 130, 2, 8)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_attention_fwd_most_blocks(cuda, shape):
+    n, h, sq, sk, d = shape
+    inp = attention_inputs(2, h, sq, sk, d, torch.bfloat16, seed=sq, with_dout=False)
+    g = {k: (v.to(cuda) if isinstance(v, torch.Tensor) else v) for k, v in inp.items()}
+    q, k, v = (torch.zeros((n, *g[name].shape[1:]), dtype=torch.bfloat16, device=cuda)
+               for name in "qkv")
+    for big, name in ((q, "q"), (k, "k"), (v, "v")):
+        big[0], big[-1] = g[name][0], g[name][1]
+    out = ops.attention(q, k, v, g["bias"], None, g["scale"])
+    assert_close("O", out[[0, -1]], _oracle(inp)[0], TOL["bf16"]["o"])
+    assert not out[1:-1].any()
