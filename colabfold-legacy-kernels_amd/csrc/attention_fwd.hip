@@ -11,7 +11,7 @@
 // Any even Sk, and any odd one (by query parity, the ODD form below), loads its bias through LDS.
 // Reading bias and mask element by element, as a ragged Sk once did, left the kernel waiting on
 // sixteen 2-byte loads per lane and tile: triangle attention of 757 residues (4 heads x 32)
-// 2395 -> 550 us, 1024 sequences of 300 residues (8 heads x 8) 965 -> 292 us, 203 residues
+// 2395 -> 577 us, 1024 sequences of 300 residues (8 heads x 8) 965 -> 267 us, 203 residues
 // 65 -> 29 us. That path remains for what the direct loads cannot take (fwd_form).
 //
 // A block runs only 5 to 16 key tiles, so what it does before and after them counts: of 22600
@@ -21,6 +21,10 @@
 // not exist reads zero), and the presence words wait for the mask bytes alone: D = 32, 300
 // residues 47.2 -> 45.1 us, 384 72.2 -> 69.4, 757 537 -> 515; D = 16, 300 40.5 -> 36.9;
 // D = 64, 300 91.3 -> 85.5.
+//
+// What the fast forms cannot hold -- -inf in the bias, float16 queries whose every logit lies near
+// the type's lowest value -- is found from a block's sums and maxima after its last tile, and the
+// block's keys are run again in the plain form (the end of the kernel).
 //
 // Per 64-key tile and 16-query sub-tile a wave computes S^T = K . Q^T with the keys of each
 // 32-key chunk permuted so that lane l's accumulator holds keys 8*(l/16)+0..7 of the chunk for

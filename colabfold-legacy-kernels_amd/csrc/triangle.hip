@@ -8,15 +8,16 @@
 // (A_c[i][k] = a[i,k,c]); incoming X_c = A_c^T . B_c with it first (A_c[k][i] = a[k,i,c]).
 //
 // tri_einsum_kernel: one 256 x 256 output tile of one channel per block of 8 waves (2 x 4 wave
-// tiles of 128 i x 64 j, 32 MFMA 16x16x32 accumulators each). The operands reach LDS in
-// 64-wide k slices by direct buffer->LDS loads, two stages (the next slice loads while the
-// current one is multiplied). Contraction index last: 256 rows of 128 bytes per operand (whole
+// tiles of 128 i x 64 j, 32 MFMA 16x16x32 accumulators each), or one 128 x 128 tile per block of 4
+// waves of 64 x 64 (launch_einsum chooses; the figures here are the larger form's). The operands
+// reach LDS in 64-wide k slices by direct buffer->LDS loads, two stages (the next slice loads while
+// the current one is multiplied). Contraction index last: 256 rows of 128 bytes per operand (whole
 // cache lines: 32-wide slices read half lines, 5% slower), each 16-byte piece XOR-swizzled by
 // row % 8 so the sixteen rows an operand read touches fall in distinct banks. Contraction index
 // first: 64 rows of 512 bytes, read with ds_read_b64_tr_b16 (a transposed 4 x 16 block per
 // 16-lane group), pieces swizzled by 2 * (row % 4). Per slice a block moves 64 KB from L2 for
-// 8.4 MFLOP (128 flop/B). Tiles of one channel run on one XCD, whose L2 then serves both
-// operands.
+// 8.4 MFLOP (128 flop/B; 64 in the smaller form). Tiles of one channel run on one XCD, whose L2
+// then serves both operands.
 #include "common.hpp"
 
 namespace clk {

@@ -27,7 +27,8 @@ pytestmark = [
 MFMA_KERNELS = ["attn_fwd_kernel", "attn_bwd_dq2", "attn_bwd_dkv2", "attn_bwd_dq",
                 "attn_bwd_dkv", "gdp_kernel", "gdp_stream_kernel", "ln_gdp_kernel",
                 "attn_gate_kernel", "tri_einsum_kernel", "tri_out_kernel",
-                "gdp_bwd_grad_kernel", "gdp_bwd_dx_kernel", "gdp_bwd_dw_kernel"]
+                "gdp_bwd_fused_kernel", "gdp_bwd_grad_kernel", "gdp_bwd_dx_kernel",
+                "gdp_bwd_dw_kernel", "gate_bwd_grad_kernel"]
 FUNC = re.compile(r"^[0-9a-f]+ <(?P<name>[^>]+)>:$")
 
 

@@ -263,8 +263,15 @@ def test_attention_bwd_ragged_keys(cuda, shape, dtype):
     km[4] = (torch.rand(sk, generator=g) > 0.3).to(torch.uint8)
     km[4, sk // 2] = 1
     tol = TOL[dname(dtype)]["grad"]
-    for mask in (km, torch.ones_like(km)):
+    for mask in (km, torch.ones_like(km), None):
         inp["kmask"] = mask
-        _, _, _, grads = _run(inp, cuda)
-        for name, got, r in zip(("dQ", "dK", "dV", "dBias"), grads, _oracle(inp)):
+        g, out, lse, grads = _run(inp, cuda)
+        inp["kmask"] = torch.ones_like(km) if mask is None else mask
+        refs = _oracle(inp)
+        for name, got, r in zip(("dQ", "dK", "dV", "dBias"), grads, refs):
             assert_close(name, got, r, tol)
+        t = lambda x: x.transpose(1, 2).contiguous()  # noqa: E731
+        nshd = ops.attention_bwd_nshd(t(g["q"]), t(g["k"]), t(g["v"]), g["bias"], g["kmask"],
+                                      t(out), t(g["dout"]), lse, g["scale"])
+        for a, b in zip(nshd, grads):
+            assert torch.equal(t(a) if a.dim() == 4 else a, b)

@@ -311,6 +311,18 @@ def test_attention_fwd_ragged_keys(cuda, shape, dtype):
     out_s, lse_s = ops.attention_nshd(t(g["q"]), t(g["k"]), t(g["v"]), g["bias"], g["kmask"],
                                       g["scale"], want_lse=True)
     assert torch.equal(t(out_s), out) and torch.equal(lse_s, lse)
+    # No mask and a mask of ones: the same bits, in both layouts.
+    ones = torch.ones_like(g["kmask"])
+    for scale in (g["scale"], -g["scale"]):
+        args = (g["q"], g["k"], g["v"], g["bias"])
+        out_1, lse_1 = ops.attention_fwd(*args, ones, scale)
+        out_0, lse_0 = ops.attention_fwd(*args, None, scale)
+        assert torch.equal(out_0, out_1) and torch.equal(lse_0, lse_1)
+        out_t = ops.attention_nshd(*(t(x) for x in args[:3]), g["bias"], None, scale)[0]
+        assert torch.equal(t(out_t), out_0)
+        o_1, lse_r = _oracle({**inp, "kmask": torch.ones_like(km), "scale": scale})
+        assert_close("O (no mask)", out_0, o_1, TOL[dname(dtype)]["o"])
+        assert np.abs(np64(lse_0) - lse_r).max() < 5e-2
     # A negative scale takes the form without the bias MFMA (odd: the element-wise path).
     neg = {**inp, "scale": -inp["scale"]}
     out_n = ops.attention(g["q"], g["k"], g["v"], g["bias"], g["kmask"], neg["scale"])

@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
 
 # (N, H, Sq, Sk, D, C, masked_tail, masked_rows): every head dim; one- and two-sub-tile query
 # blocks (Sq <= 64 and above) with ragged ends; gate channel counts that fill whole 64-channel
-# chunks and ones that end on a half chunk (C % 64 == 32); odd Sk (the element-wise mask path).
+# chunks and ones that end on a half chunk (C % 64 == 32); odd Sk (blocks of one query parity,
+# half of them with key tiles that start at key -1) at every head dim.
 CASES = [
     (2, 8, 70, 70, 32, 256, 0.1, 1),
     (3, 4, 64, 64, 32, 128, 0.0, 0),
@@ -26,6 +27,10 @@ CASES = [
     (2, 3, 129, 77, 32, 96, 0.05, 1),
     (1, 2, 200, 64, 16, 32, 0.0, 0),
     (2, 1, 1, 1, 32, 160, 0.0, 0),
+    (3, 4, 67, 65, 32, 64, 0.1, 1),
+    (2, 2, 131, 129, 32, 128, 0.0, 0),
+    (2, 2, 130, 63, 8, 64, 0.1, 1),
+    (2, 2, 65, 191, 64, 96, 0.1, 1),
     (2, 4, 70, 300, 32, 128, 0.5, 1),  # the last two key tiles hold no present key
     (2, 2, 40, 256, 16, 64, 0.7, 0),   # ... the last three
     # More than 256 gate channels: the epilogue's later rounds stage Wg rows into the freed K/V
@@ -102,8 +107,9 @@ def test_attention_gated_exact_cases(cuda):
     assert torch.count_nonzero(_call(g)) == 0
 
 
-def test_attention_gated_without_mask(cuda):
-    n, h, sq, sk, d, c = 2, 4, 64, 96, 32, 128
+@pytest.mark.parametrize("sk", [96, 97, 66])
+def test_attention_gated_without_mask(cuda, sk):
+    n, h, sq, d, c = 2, 4, 65, 32, 128
     g = _cuda(_inputs(n, h, sq, sk, d, c, 0.0, 0, torch.bfloat16, seed=6), cuda)
     a = ops.attention_gated(g["q"], g["k"], g["v"], g["bias"], None, g["x"], g["wg"], g["bg"])
     b = _call(g)
