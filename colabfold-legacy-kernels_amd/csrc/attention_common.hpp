@@ -349,43 +349,23 @@ struct LogitForm {
 // over the two halves of the contraction; the tile then holds logit / scale, and
 // log2(e) * logit = cexp * S. No per-score instruction touches the bias. A bias whose bias / scale
 // float32 cannot hold, -inf among them, leaves NaN, and its block is redone in the plain form.
-//
-// Ragged key counts hold scale and bias to float32: where the pair is further than 2^-24 from
-// 1/scale (bfloat16 at D = 8 and 32: 2.9e-7), a third value lo2 enters by an MFMA of its own
-// ([lo2*I | 0], three terms), and cexp = log2(e) / (hi + lo + lo2), so that the bias enters exactly
-// and q.k to the rounding of cexp (6% of the time: 757 residues, 4 heads x 32, 517 -> 550 us). At
-// multiples of 8 the pair alone is used, its error (up to 7.6e-6 of the bias in bfloat16) on the
-// bias, and cexp = scale * log2(e).
+// The pair's error (up to 7.6e-6 in bfloat16) is on the bias; cexp = scale * log2(e).
 struct BiasMfma {
-    float hi, lo, lo2, bscale, cexp;
+    float hi, lo, bscale, cexp;
 };
 
-// The terms (2 or 3) of the bias MFMA for `scale`, and its constants; 0 where the form does not
-// apply: scale <= 0, 1/scale past the input type's range, or too small to be held in it (float16:
-// scale above some hundreds, or for `exact` some tens).
+// The constants of the bias MFMA for `scale`; false where the form does not apply: scale <= 0,
+// 1/scale past the input type's range, or too small to be held in it (float16: scale above some
+// hundreds).
 template <typename TR>
-int bias_mfma_for(float scale, bool exact, BiasMfma* bm) {
+bool bias_mfma_for(float scale, BiasMfma* bm) {
     using E = typename TR::elem;
-    if (!(scale > 0.f) || !std::isfinite(scale)) return 0;
+    if (!(scale > 0.f) || !std::isfinite(scale)) return false;
     const float b = 1.f / scale;
-    if (!std::isfinite(b) || b > 6.0e4f) return 0;
-    if (!exact) {
-        const float hi = (float)(E)b, lo = (float)(E)(b - hi);
-        *bm = {hi, lo, 0.f, b, scale * kLog2e};
-        return std::fabs(b - hi - lo) <= 0x1p-16f * b ? 2 : 0;
-    }
-    const double want = 1.0 / scale;
-    double sum = 0.0;
-    float part[3];
-    for (int terms = 1; terms <= 3; ++terms) {
-        part[terms - 1] = (float)(E)(float)(want - sum);
-        sum += part[terms - 1];
-        if (terms < 2 || std::fabs(want - sum) > 0x1p-24 * want) continue;
-        *bm = {part[0], part[1], terms == 3 ? part[2] : 0.f, b, (float)(1.4426950408889634 / sum)};
-        // (float16's third value would lie below its smallest number.)
-        return terms == 2 || std::is_same<TR, BF16>::value ? terms : 0;
-    }
-    return 0;
+    if (!std::isfinite(b) || b > 6.0e4f) return false;
+    const float hi = (float)(E)b, lo = (float)(E)(b - hi);
+    *bm = {hi, lo, b, scale * kLog2e};
+    return std::fabs(b - hi - lo) <= 0x1p-16f * b;
 }
 
 // Host-side shape/dtype validation shared by the forward and backward entry points. The

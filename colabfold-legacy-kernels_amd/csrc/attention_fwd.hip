@@ -11,8 +11,8 @@
 // Any even Sk, and any odd one (by query parity, the ODD form below), loads its bias through LDS.
 // Reading bias and mask element by element, as a ragged Sk once did, left the kernel waiting on
 // sixteen 2-byte loads per lane and tile: triangle attention of 757 residues (4 heads x 32)
-// 2395 -> 577 us, 1024 sequences of 300 residues (8 heads x 8) 965 -> 267 us, 203 residues
-// 65 -> 29 us. That path remains for what the direct loads cannot take (fwd_form).
+// 2395 -> 529 us, 1024 sequences of 300 residues (8 heads x 8) 965 -> 255 us, 203 residues
+// 68 -> 23 us. That path remains for what the direct loads cannot take (fwd_form).
 //
 // A block runs only 5 to 16 key tiles, so what it does before and after them counts: of 22600
 // cycles at 384 residues, 4600 passed before the first tile was there (2500 before its loads went
@@ -165,23 +165,21 @@ struct FwdItems {
     int grp, nrows;
 };
 
-// ODD (VEC and BM): Sk is odd. The direct-to-LDS loads of the bias need 4-byte aligned addresses,
+// ODD (VEC, not BM): Sk is odd. The direct-to-LDS loads of the bias need 4-byte aligned addresses,
 // and every other bias row starts half a dword off. A block then owns queries of one parity
 // (query q0 + 2i for its i-th row), whose bias rows are all aligned or all off by one element;
 // in the second case its key tiles start one key early (tile kt: keys 64kt - 1 ...), which
 // aligns every load, and key -1 is an absent key. So the loop is the even one, with no shifting
 // of bias pieces.
-// TERMS: the terms of the bias MFMA (BM), 0 without it.
-template <typename TR, int D, int QT, bool VEC, bool GATE, int TERMS, bool NSHD, bool ODD>
+template <typename TR, int D, int QT, bool VEC, bool GATE, bool BM, bool NSHD, bool ODD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && VEC ? 3 : 1))) void attn_fwd_kernel(
     const typename TR::elem* __restrict__ q, const typename TR::elem* __restrict__ k,
     const typename TR::elem* __restrict__ v, const typename TR::elem* __restrict__ bias,
     const uint8_t* __restrict__ kmask, typename TR::elem* __restrict__ out,
     float* __restrict__ lse, int H, int Sq, int Sk, float scale,
     GateArgs<typename TR::elem> ga, BiasMfma bm, FwdItems items) {
-    constexpr bool BM = TERMS > 0;
     static_assert(!BM || VEC, "the bias MFMA reads the bias tile from LDS");
-    static_assert(!ODD || BM, "odd key counts run the bias-MFMA form");
+    static_assert(!ODD || (VEC && !BM), "odd key counts run the plain form, the bias in LDS");
     static_assert(!(NSHD && GATE), "the gated entry takes the [N, H, S, D] layout");
     using E = typename TR::elem;
     using V8 = typename TR::vec8;
@@ -405,7 +403,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
         // changed bias alone. (Rows that do not exist are zeros already. Every wave does all rows:
         // its own reads then need no barrier, and nobody writes anything else.) As asm, because the
         // compiler would have a store it can see wait for the next tile's direct-to-LDS loads
-        // (757 residues 568 -> 577 us with it, 598 with such a store).
+        // (with the bias MFMA, 757 residues 568 -> 577 us and 598).
         const unsigned long long w = pres[kt];
         const int rem = Sk + shift - kt * BK;
         unsigned long long exist = rem >= 64 ? ~0ull : (1ull << rem) - 1ull;
@@ -425,21 +423,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     const float xs = BM ? bm.cexp : kLog2e;
     // A operand [hi*I | lo*I] of the bias MFMA: lane (row r16, group g) holds columns
     // 8g .. 8g+7, so its one nonzero is element r16 % 8 when g % 2 == r16 / 8.
-    // (Three terms: a second operand [lo2*I | 0].)
-    V8 idn, idn2;
+    V8 idn;
     if constexpr (BM) {
-        auto diagonal = [&](float upper, float lower) {
-            const uint32_t v =
-                (uint32_t)__builtin_bit_cast(uint16_t, TR::from_f(g < 2 ? upper : lower))
-                << (16 * (r16 & 1));
-            const int at = (g & 1) == (r16 >> 3) ? (r16 & 7) >> 1 : -1;
-            u32x4 bits;
+        const uint32_t v = (uint32_t)__builtin_bit_cast(uint16_t, TR::from_f(g < 2 ? bm.hi : bm.lo))
+                           << (16 * (r16 & 1));
+        const int at = (g & 1) == (r16 >> 3) ? (r16 & 7) >> 1 : -1;
+        u32x4 bits;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) bits[i] = i == at ? v : 0u;
-            return bits_as<V8>(bits);
-        };
-        idn = diagonal(bm.hi, bm.lo);
-        if constexpr (TERMS == 3) idn2 = diagonal(bm.lo2, 0.f);
+        for (int i = 0; i < 4; ++i) bits[i] = i == at ? v : 0u;
+        idn = bits_as<V8>(bits);
     }
 
     // Running max, and O^T plus one extra accumulator per sub-tile: the MFMA of an all-ones
@@ -530,9 +522,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
                 for (int t = 0; t < 4; ++t) {
                     const u32x4 raw = *reinterpret_cast<const u32x4*>(
                         brow_l + 16 * ((2 * t + (g & 1)) ^ (row & 7)));
-                    f32x4 low = {0.f, 0.f, 0.f, 0.f};
-                    if constexpr (TERMS == 3) low = TR::mfma(idn2, bits_as<V8>(raw), low);
-                    s[qt][t] = TR::mfma(idn, bits_as<V8>(raw), low);
+                    s[qt][t] = TR::mfma(idn, bits_as<V8>(raw), f32x4{0.f, 0.f, 0.f, 0.f});
                 }
             }
         }
@@ -722,7 +712,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             tile(kt, kv0, kv1, ca, cb, std::false_type{});
             if (kt + 1 < nrun) tile(kt + 1, kv1, kv0, cb, ca, std::false_type{});
         }
-        if constexpr (PATCH) {
+        if constexpr (BM || LOWEST) {
             // A bias of -inf leaves NaN in the row sum of its query (the zeros of the bias MFMA's
             // operand times it are NaN). A block with one redoes its keys in the plain form, where
             // -inf is a weight of 0. So does a float16 block with a row maximum near -65504, where
@@ -859,11 +849,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     }
 }
 
-// How a call's bias reaches the kernel (terms: those of the bias MFMA, 0 without it).
+// How a call's bias reaches the kernel.
 struct FwdForm {
     BiasMfma bm{};
-    int terms;
-    bool odd, vec;
+    bool bmf, odd, vec;
 };
 
 // Most blocks of a launch: a grid is at most 2^32 - 1 threads (more wrap around, without an error).
@@ -876,16 +865,22 @@ int fwd_qtiles(bool odd, int Sq, int QT) {
 
 // The bias tile through LDS (vec: direct loads of 4-byte aligned pieces): at most kPresWords key
 // tiles (masked bias tiles are changed in LDS from presence words kept there). An even Sk
-// aligns every bias row. An odd one takes the parity form of the bias-MFMA kernel, when the
-// bias is a whole number of dwords (no load then reaches past its end). Other odd cases
-// (scale <= 0 or without a bias MFMA, one head or an odd number of them with an odd Sq, so many
-// short rows that two parities of blocks pass the largest launch) and longer rows read bias and mask
-// element by element, about four times slower (2395 against 577 us at 757 residues).
+// aligns every bias row. An odd one takes the parity form, when the bias is a whole number of
+// dwords (no load then reaches past its end). Other odd cases (one head or an odd number of them
+// with an odd Sq, so many short rows that two parities of blocks pass the largest launch) and longer
+// rows read bias and mask element by element, about four times slower (2395
+// against 529 us at 757 residues).
+//
+// Multiples of 8 take the bias MFMA (two VALU instructions a score less, 1-2% of the time). Ragged
+// counts add the bias to each score as the element-wise path does, exact in float32; a bias MFMA
+// that is (a third 16-bit term of 1/scale in bfloat16, cexp that of the pair in float16) is slower:
+// 757 residues at D = 32 566 against 529 us in bfloat16, 542 against 530 in float16, 1024 x 300 at
+// D = 8 281 against 257 and 263 against 255; D = 16, whose 1/scale is one value, 96 against 101.
 template <typename TR>
 FwdForm fwd_form(int64_t NH, int H, int Sq, int Sk, float scale) {
     FwdForm f;
-    f.terms = bias_mfma_for<TR>(scale, Sk % 8 != 0, &f.bm);
-    const bool odd = Sk % 2 && f.terms && (size_t)H * Sq * Sk % 2 == 0 &&
+    f.bmf = Sk % 8 == 0 && bias_mfma_for<TR>(scale, &f.bm);
+    const bool odd = Sk % 2 && (size_t)H * Sq * Sk % 2 == 0 &&
                      NH * fwd_qtiles(true, Sq, Sq <= 64 ? 1 : 2) <= kMaxBlocks;
     f.vec = (Sk % 2 == 0 || odd) && Sk + (odd ? 1 : 0) <= kPresWords * 64;
     f.odd = f.vec && odd;
@@ -936,20 +931,14 @@ void launch_fwd_qt(hipStream_t st, const void* q, const void* k, const void* v, 
         kernel<<<grid, 256, 0, st>>>((const E*)q, (const E*)k, (const E*)v, (const E*)bias, kmask,
                                      (E*)out, lse, H, Sq, Sk, scale, ga, f.bm, items);
     };
-    auto run_terms = [&](auto terms) {
-        if (f.odd)
-            run(attn_fwd_kernel<TR, D, QT, true, GATE, decltype(terms)::value, NSHD, true>);
-        else
-            run(attn_fwd_kernel<TR, D, QT, true, GATE, decltype(terms)::value, NSHD, false>);
-    };
-    if (!f.vec)
-        run(attn_fwd_kernel<TR, D, QT, false, GATE, 0, NSHD, false>);
-    else if (f.terms == 0)
-        run(attn_fwd_kernel<TR, D, QT, true, GATE, 0, NSHD, false>);
-    else if (f.terms == 2)
-        run_terms(std::integral_constant<int, 2>{});
-    else if constexpr (std::is_same<TR, BF16>::value)
-        run_terms(std::integral_constant<int, 3>{});
+    if (f.odd)
+        run(attn_fwd_kernel<TR, D, QT, true, GATE, false, NSHD, true>);
+    else if (f.vec && f.bmf)
+        run(attn_fwd_kernel<TR, D, QT, true, GATE, true, NSHD, false>);
+    else if (f.vec)
+        run(attn_fwd_kernel<TR, D, QT, true, GATE, false, NSHD, false>);
+    else
+        run(attn_fwd_kernel<TR, D, QT, false, GATE, false, NSHD, false>);
 }
 
 template <typename TR, int D, bool GATE>
