@@ -783,7 +783,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
             V8 xo[QT][NX];
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
-                const int row = qbase + (qt * 16 + gr16) * QS;
+                const int row = q0 + (16 * QT * (tid >> 6) + qt * 16 + gr16) * QS;
 #pragma unroll
                 for (int j = 0; j < NX; ++j) {
                     const int c = c0 + 32 * j;
@@ -825,7 +825,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 32 && 
     for (int qt = 0; qt < QT; ++qt) {
         const float l_tot = lsum[qt][0];
         const float inv = 1.0f / fmaxf(l_tot, 1e-30f);
-        const int row = qbase + (qt * 16 + er16) * QS;
+        const int row = q0 + (16 * QT * (etid >> 6) + qt * 16 + er16) * QS;
         if (row >= Sq) continue;
 #pragma unroll
         for (int dt = 0; dt < G::DT; ++dt) {
