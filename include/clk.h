@@ -68,7 +68,8 @@ int clk_profile_collect(const char** names, float* ms, int max);
  * CLK_BF16 for q, k, v, bias and out. D is 8, 16, 32 or 64. block_q and block_k are hints: any
  * value the reference dispatch accepts is accepted, and other positive values too.
  * kmask may be NULL (every key present). lse may be NULL (inference); when given, the natural-log
- * logsumexp of every query row is written for clk_attention_bwd.
+ * logsumexp of every query row is written for clk_attention_bwd. A bias of -inf gives its key the
+ * weight 0; a query left without any has O = 0 and lse = +inf.
  */
 clk_status clk_attention_fwd(hipStream_t stream, clk_dtype dtype, const void* q, const void* k,
                              const void* v, const void* bias, const uint8_t* kmask, void* out,

@@ -323,7 +323,7 @@ def test_attention_fwd_ragged_keys(cuda, shape, dtype):
         o_1, lse_r = _oracle({**inp, "kmask": torch.ones_like(km), "scale": scale})
         assert_close("O (no mask)", out_0, o_1, TOL[dname(dtype)]["o"])
         assert np.abs(np64(lse_0) - lse_r).max() < 5e-2
-    # A negative scale takes the form without the bias MFMA (odd: the element-wise path).
+    # A negative scale takes the form without the bias MFMA at any key count.
     neg = {**inp, "scale": -inp["scale"]}
     out_n = ops.attention(g["q"], g["k"], g["v"], g["bias"], g["kmask"], neg["scale"])
     assert_close("O (negative scale)", out_n, _oracle(neg)[0], TOL[dname(dtype)]["o"])
