@@ -523,8 +523,7 @@ def test_attention_fwd_lowest_float16_bias(cuda, sk, scale):
     additive mask): no weight goes to absent keys (-1e9) or past the last one. The logits are near
     65504, where float32 steps by 2^-8: four roundings move a logit by 2^-7 and a weight by 0.8%."""
     n, h, sq, d = 3, 2, 70, 32
-    inp = attention_inputs(n, h, sq, sk, d, torch.float16, seed=sk, masked_tail=0.2, masked_rows=1,
-                           with_dout=False)
+    inp = attention_inputs(n, h, sq, sk, d, torch.float16, seed=sk, masked_tail=0.2, masked_rows=1)
     inp["scale"] = scale
     inp["bias"][0, 3:40] = -65504.0
     inp["bias"][1, 60:] = -65504.0
@@ -534,6 +533,13 @@ def test_attention_fwd_lowest_float16_bias(cuda, sk, scale):
     assert_close("O", out, o_ref, TOL["f16"]["o"] + 0.008)
     full = (inp["kmask"] != 0).any(1).numpy()[:, None, None]
     assert np.abs(np64(lse) - np.where(full, lse_ref, np.log(sk))).max() <= 2.0 ** -6
+    # The gradients recompute such a weight from its logit and lse: twice that error.
+    grads = ops.attention_bwd(g["q"], g["k"], g["v"], g["bias"], g["kmask"], out, g["dout"], lse,
+                              scale)
+    refs = ref.attention_bwd(*(np64(inp[k]) for k in ("q", "k", "v", "bias")), inp["kmask"].numpy(),
+                             scale, np64(inp["dout"]))
+    for name, got, want in zip(("dQ", "dK", "dV", "dBias"), grads, refs):
+        assert_close(name, got, want, TOL["f16"]["grad"] + 0.016)
 
 
 # (N, H, Sq, Sk, D): one query and one key for 8.5 million (row, head) pairs, whose two parities of
